@@ -50,7 +50,7 @@ hipcstone_status findNeighborsSegmented(hipStream_t s, const T* x, const T* y, c
                                         const int32_t* internalToLeaf, const uint32_t* layout, const T* centers,
                                         const T* sizes, int32_t numNodesCap, uint32_t ngmax, uint32_t* neighbors,
                                         uint32_t* neighborsCount, const uint32_t* waves, uint32_t numWaves,
-                                        const int32_t* roots, const nbwalk::ChildGroup* groups);
+                                        const int32_t* roots, const nbwalk::ChildGroup<T>* groups);
 
 namespace batched
 {
@@ -702,7 +702,7 @@ private:
         for (auto* b : {&centers_, &sizes_})
             if (auto e = reserve(*b, N * 3 * sizeof(T))) return e;
         if (auto e = reserve(groups_, std::max<size_t>(nbwalk::childGroupCount(int32_t(N)), 1) *
-                                          sizeof(nbwalk::ChildGroup)))
+                                          sizeof(nbwalk::ChildGroup<float>)))
             return e;
         capL_ = cap;
         capN_ = int32_t(N);
@@ -857,9 +857,9 @@ private:
         const uint32_t numGroups = uint32_t(nbwalk::childGroupCount(capN_));
         if (numGroups > 0)
         {
-            nbwalk::childGroupsKernel<><<<ceilDiv(size_t(numGroups), 256), 256, 0, st>>>(
+            nbwalk::childGroupsKernel<float><<<ceilDiv(size_t(numGroups), 256), 256, 0, st>>>(
                 centers_.as<T>(), sizes_.as<T>(), childOffsets_.as<int32_t>(), internalToLeaf_.as<int32_t>(),
-                numGroups, groups_.as<nbwalk::ChildGroup>());
+                int32_t(capN_), numGroups, groups_.as<nbwalk::ChildGroup<float>>());
             HC_CHECK_LAUNCH("batched childGroupsKernel");
         }
         Box any = hostBoxes_[0];
@@ -870,7 +870,7 @@ private:
                                          internalToLeaf_.as<int32_t>(), layout_.as<uint32_t>(), centers_.as<T>(),
                                          sizes_.as<T>(), capN_, ngmax_, ngmax_ ? nb_.as<uint32_t>() : nullptr,
                                          nc_.as<uint32_t>(), wavesD_.as<uint32_t>(), numWaves_, roots_.as<int32_t>(),
-                                         numGroups ? groups_.as<nbwalk::ChildGroup>() : nullptr);
+                                         numGroups ? groups_.as<nbwalk::ChildGroup<float>>() : nullptr);
     }
 
     static hipcstone_status growKeep(DeviceBuf& b, size_t bytes, size_t keep, hipStream_t st)

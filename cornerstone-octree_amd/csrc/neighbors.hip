@@ -21,23 +21,30 @@ namespace hipcstone
 // Waves per workgroup: 4 by default; 2 and 8 are the other shapes the autotuner measures
 // (hipcstone_set_neighbor_waves). Every wave owns its own targets, stack and leaf list, so the shape changes only
 // how waves are grouped onto CUs (LDS per workgroup, scheduling granularity), never a result.
-// The fp32 open-box walk fits 8 waves per SIMD when its scalar registers are capped (the compiler then keeps some
-// wave-uniform values of the walk in vector-register lanes): more waves to cover the latency of its LDS, scalar-load
-// and compare-to-ballot dependencies, measured 6 % faster than the 7 waves its uncapped allocation allows. The other
-// variants keep the compiler's own allocation.
-template<class T, bool AnyPbc>
-constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> && !AnyPbc ? 8 : 1;
+// targetsPerWave: 64, or fewer where that many waves would leave the device idle (kFullWaves).
+//
+// Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a tenth busy): the walk and
+// the chunks' set-up take 2.3 of 6.3 ms, the pair tests 2.5, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
+// search of that size took 7.70 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
+// instructions a wave, now 23.4K); in fp64 at 2M, where nothing was compact either, 1.73 -> 1.05 ms.
+
+// Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.66 ms, 6 waves 6.31, 7 waves 7.1 (registers go
+// to memory; 16.8M targets). fp64 would have to spill for more than 4.
+template<class T>
+constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> ? 6 : 4;
+
+typedef uint32_t Row4 __attribute__((ext_vector_type(4), aligned(4)));
 
 template<class T, bool AnyPbc, bool SlotMajor, bool Segmented, int kNbWaves>
-__global__ __launch_bounds__(kNbWaves * kWave) __attribute__((amdgpu_waves_per_eu(kNbMinWavesPerEu<T, AnyPbc>, 8)))
+__global__ __launch_bounds__(kNbWaves * kWave) __attribute__((amdgpu_waves_per_eu(kNbMinWavesPerEu<T>, 8)))
 void findNeighborsKernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, const T* __restrict__ h,
     uint32_t firstId, uint32_t lastId, typename BoxOf<T>::type box, const int32_t* __restrict__ childOffsets,
     const int32_t* __restrict__ internalToLeaf, const uint32_t* __restrict__ layout, const T* __restrict__ centers,
     const T* __restrict__ sizes, int32_t numNodes, float ext, uint32_t ngmax, uint32_t* __restrict__ neighbors,
     uint32_t* __restrict__ neighborsCount, uint32_t numBlocksPadded, uint32_t* __restrict__ faults,
-    const uint32_t* __restrict__ waves = nullptr, uint32_t numWaves = 0, const int32_t* __restrict__ roots = nullptr,
-    const nbwalk::ChildGroup* __restrict__ groups = nullptr)
+    uint32_t targetsPerWave, const uint32_t* __restrict__ waves = nullptr, uint32_t numWaves = 0,
+    const int32_t* __restrict__ roots = nullptr, const nbwalk::ChildGroup<T>* __restrict__ groups = nullptr)
 {
     __shared__ nbwalk::Shared<T, kNbWaves> sh;
     const int lane       = laneId();
@@ -60,21 +67,47 @@ void findNeighborsKernel(
     }
     else
     {
-        first = uint64_t(firstId) + uint64_t(group) * kWave;
+        first = uint64_t(firstId) + uint64_t(group) * targetsPerWave;
         if (first >= lastId) return;
     }
-    const uint32_t i     = uint32_t(first) + uint32_t(lane);
-    const bool valid     = i < lastId;
-    const size_t rowBase = Segmented ? size_t(first) : size_t(group) * kWave; // row of lane 0 in the output
-
-    // row-major: the rows of the wave's valid targets; slot-major: all 64 rows of the wave
-    const uint32_t validRows = uint64_t(lastId) - first < uint64_t(kWave) ? uint32_t(uint64_t(lastId) - first) : kWave;
-    const uint32_t rowsBytes = ngmax ? (SlotMajor ? uint32_t(kWave) : validRows) * ngmax * uint32_t(sizeof(uint32_t))
-                                     : 0u;
+    const uint32_t i = uint32_t(first) + uint32_t(lane);
+    const bool valid = i < lastId && uint32_t(lane) < targetsPerWave;
+    // the wave's rows: row-major, or slot-major (then a wave has 64 targets)
+    const size_t rowBase   = Segmented ? size_t(first) : size_t(first) - firstId;
+    uint32_t* rows         = neighbors + (ngmax ? rowBase * ngmax : 0);
     const nbwalk::Tree<T> tree{childOffsets, internalToLeaf, layout, centers, sizes, numNodes, ext, groups};
-    const uint32_t count = nbwalk::walk<T, AnyPbc, SlotMajor, Segmented, kNbWaves>(
-        x, y, z, h, box, tree, root, first, valid, ngmax, ngmax ? neighbors + rowBase * ngmax : nullptr, rowsBytes,
-        sh, w, faults);
+    const uint32_t count = nbwalk::walk<T, AnyPbc, Segmented, kNbWaves>(
+        x, y, z, h, box, tree, root, first, valid, ngmax != 0, sh, w, faults,
+        [&](uint32_t before, uint32_t hits, auto&& next) __attribute__((always_inline)) {
+            // the row's next slots, four to a store; the last ones one by one
+            uint32_t rest = min(hits, ngmax - min(before, ngmax));
+            uint32_t slot = SlotMajor ? before * kWave + uint32_t(lane) : uint32_t(lane) * ngmax + before;
+            while (rest != 0)
+            {
+                const uint32_t j0 = next(), j1 = next(), j2 = next(), j3 = next();
+                uint32_t* row     = rows + slot;
+                if constexpr (SlotMajor)
+                {
+                    row[0] = j0;
+                    if (rest > 1) row[kWave] = j1;
+                    if (rest > 2) row[2 * kWave] = j2;
+                    if (rest > 3) row[3 * kWave] = j3;
+                    slot += 4 * kWave;
+                }
+                else
+                {
+                    if (rest > 3) *reinterpret_cast<Row4*>(row) = Row4{j0, j1, j2, j3};
+                    else
+                    {
+                        row[0] = j0;
+                        if (rest > 1) row[1] = j1;
+                        if (rest > 2) row[2] = j2;
+                    }
+                    slot += 4;
+                }
+                rest -= min(rest, 4u);
+            }
+        });
     if (valid) neighborsCount[i - firstId] = count;
 }
 
@@ -85,7 +118,7 @@ hipcstone_status findNeighborsSegmented(hipStream_t s, const T* x, const T* y, c
                                         const int32_t* internalToLeaf, const uint32_t* layout, const T* centers,
                                         const T* sizes, int32_t numNodesCap, uint32_t ngmax, uint32_t* neighbors,
                                         uint32_t* neighborsCount, const uint32_t* waves, uint32_t numWaves,
-                                        const int32_t* roots, const nbwalk::ChildGroup* groups)
+                                        const int32_t* roots, const nbwalk::ChildGroup<T>* groups)
 {
     if (numWaves == 0) return HIPCSTONE_OK;
     if (ngmax > (1u << 20)) return invalid("findNeighbors: ngmax above 2^20");
@@ -97,7 +130,7 @@ hipcstone_status findNeighborsSegmented(hipStream_t s, const T* x, const T* y, c
         blocks          = (blocks + kXcds - 1) / kXcds * kXcds;
         findNeighborsKernel<T, false, false, true, W><<<blocks, W * kWave, 0, s>>>(
             x, y, z, h, 0u, 0u, box, childOffsets, internalToLeaf, layout, centers, sizes, numNodesCap, 1.0f, ngmax,
-            neighbors, neighborsCount, blocks, faults, waves, numWaves, roots, groups);
+            neighbors, neighborsCount, blocks, faults, kWave, waves, numWaves, roots, groups);
     };
     switch (neighborWaves())
     {
@@ -113,20 +146,42 @@ template hipcstone_status findNeighborsSegmented<float>(hipStream_t, const float
                                                         const float*, const BoxOf<float>::type&, const int32_t*,
                                                         const int32_t*, const uint32_t*, const float*, const float*,
                                                         int32_t, uint32_t, uint32_t*, uint32_t*, const uint32_t*,
-                                                        uint32_t, const int32_t*, const nbwalk::ChildGroup*);
+                                                        uint32_t, const int32_t*, const nbwalk::ChildGroup<float>*);
 
-size_t neighborGroupsBytes(int32_t numNodes) { return nbwalk::childGroupCount(numNodes) * sizeof(nbwalk::ChildGroup); }
+// (a record is 128 bytes for either float type)
+size_t neighborGroupsBytes(int32_t numNodes)
+{
+    static_assert(sizeof(nbwalk::ChildGroup<float>) == 128 && sizeof(nbwalk::ChildGroup<double>) == 128);
+    return nbwalk::childGroupCount(numNodes) * sizeof(nbwalk::ChildGroup<double>);
+}
 
-hipcstone_status buildChildGroups(hipStream_t s, const float* centers, const float* sizes,
-                                  const int32_t* childOffsets, const int32_t* internalToLeaf, int32_t numNodes,
-                                  nbwalk::ChildGroup* groups)
+template<class T>
+static hipcstone_status buildChildGroups(hipStream_t s, const T* centers, const T* sizes, const int32_t* childOffsets,
+                                         const int32_t* internalToLeaf, int32_t numNodes,
+                                         nbwalk::ChildGroup<T>* groups)
 {
     const uint32_t numGroups = uint32_t(nbwalk::childGroupCount(numNodes));
     if (numGroups == 0) return HIPCSTONE_OK;
-    nbwalk::childGroupsKernel<<<(numGroups + 255) / 256, 256, 0, s>>>(centers, sizes, childOffsets, internalToLeaf,
-                                                                        numGroups, groups);
+    nbwalk::childGroupsKernel<T><<<(numGroups + 255) / 256, 256, 0, s>>>(centers, sizes, childOffsets, internalToLeaf,
+                                                                          numNodes, numGroups, groups);
     HC_CHECK_LAUNCH("childGroupsKernel");
     return HIPCSTONE_OK;
+}
+
+// Targets of a wave: 64, halved down to 4 while that gives fewer waves than kFullWaves. A wave's time is its own chain of
+// descents and chunks, so on an idle device more, smaller waves end sooner; on a full one they test more candidates.
+// Measured with 64 / 32 / 16 / 8 targets a wave (Plummer clouds, ngmax 150, fp32, us): 1000 targets 164 / 144 / 120 / 105
+// (4: 98), 16000: 588 / 528 / 460 / 432, 65000: 287 / 257 / 216 / 248, 131000: 184 / 155 / 187 / 248, 200000: 188 / 198 /
+// 227 / 323; fp64 turns at the same sizes. So each half stops paying where the double of it fills 2048 waves, two for
+// each SIMD. Below 4 targets another 1-5 %.
+constexpr uint32_t kFullWaves = 2048;
+
+static uint32_t targetsPerWave(uint32_t n)
+{
+    uint32_t t = kWave;
+    while (t > 4 && n / t < kFullWaves)
+        t /= 2;
+    return t;
 }
 
 template<class T>
@@ -145,33 +200,49 @@ static hipcstone_status findNeighbors(hipcstone_stream s, const T* x, const T* y
     if (ngmax > 0 && !neighbors) return invalid("findNeighbors: neighbors is null with ngmax > 0");
     if (ngmax > (1u << 20)) return invalid("findNeighbors: ngmax above 2^20");
     if (numNodes <= 0) return invalid("findNeighbors: numNodes must be positive");
-    size_t waveGroups = (size_t(lastId - firstId) + kWave - 1) / kWave;
+    const uint32_t perWave  = slotMajor ? uint32_t(kWave) : targetsPerWave(lastId - firstId);
+    const size_t waveGroups = (size_t(lastId - firstId) + perWave - 1) / perWave;
     uint32_t* faults = faultWord();
     if (!faults) return HIPCSTONE_HIP_ERROR;
     bool anyPbc     = box->bnd[0] == HIPCSTONE_PERIODIC || box->bnd[1] == HIPCSTONE_PERIODIC ||
                   box->bnd[2] == HIPCSTONE_PERIODIC;
-    // fp32 open boxes walk through the compact child blocks, built here into the caller's workspace (or into memory
-    // allocated on the stream for this call)
-    void* owned                       = nullptr;
-    const nbwalk::ChildGroup* groups = nullptr;
-    if constexpr (std::is_same_v<T, float>)
+    // the walk goes through the compact child blocks, built here into the caller's workspace or into memory allocated
+    // on the stream for this call; fp64 and periodic searches, which take no memory of their own elsewhere, do
+    // without them (child by child) where there is none to be had: while a stream is captured, or at the limit
+    void* owned                         = nullptr;
+    const nbwalk::ChildGroup<T>* groups = nullptr;
+    if (const size_t need = neighborGroupsBytes(numNodes))
     {
-        const size_t need = neighborGroupsBytes(numNodes);
-        if (!anyPbc && need > 0)
+        constexpr bool kOptional = !std::is_same_v<T, float>;
+        const bool optional      = kOptional || anyPbc;
+        void* dst                = groupsWs && groupsWsBytes >= need ? groupsWs : nullptr;
+        bool allocate            = !dst;
+        if (allocate && optional)
         {
-            void* dst = groupsWs;
-            if (!dst || groupsWsBytes < need)
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            HC_CHECK(hipStreamIsCapturing(stream(s), &capturing));
+            allocate = capturing == hipStreamCaptureStatusNone;
+        }
+        if (allocate)
+        {
+            const hipError_t e = hipMallocAsync(&owned, need, stream(s));
+            if (e != hipSuccess && !optional) return hipFail(e, "findNeighbors: child blocks");
+            if (e != hipSuccess)
             {
-                HC_CHECK(hipMallocAsync(&owned, need, stream(s)));
-                dst = owned;
+                (void)hipGetLastError();
+                owned = nullptr;
             }
-            if (auto e = buildChildGroups(stream(s), centers, sizes, childOffsets, internalToLeaf, numNodes,
-                                          static_cast<nbwalk::ChildGroup*>(dst)))
+            dst = owned;
+        }
+        if (dst)
+        {
+            auto* blocks = static_cast<nbwalk::ChildGroup<T>*>(dst);
+            if (auto e = buildChildGroups<T>(stream(s), centers, sizes, childOffsets, internalToLeaf, numNodes, blocks))
             {
                 if (owned) (void)hipFreeAsync(owned, stream(s));
                 return e;
             }
-            groups = static_cast<const nbwalk::ChildGroup*>(dst);
+            groups = blocks;
         }
     }
     auto shaped = [&](auto pbc, auto slots, auto wv) {
@@ -181,8 +252,7 @@ static hipcstone_status findNeighbors(hipcstone_stream s, const T* x, const T* y
         findNeighborsKernel<T, decltype(pbc)::value, decltype(slots)::value, false, W>
             <<<blocks, W * kWave, 0, stream(s)>>>(x, y, z, h, firstId, lastId, *box, childOffsets, internalToLeaf,
                                                   layout, centers, sizes, numNodes, ext, ngmax, neighbors,
-                                                  neighborsCount, blocks, faults, nullptr, 0u, nullptr,
-                                                  decltype(pbc)::value ? nullptr : groups);
+                                                  neighborsCount, blocks, faults, perWave, nullptr, 0u, nullptr, groups);
     };
     auto launch = [&](auto pbc, auto slots) {
         switch (neighborWaves())

@@ -55,8 +55,8 @@ hipcstone_status updateOctreeWarm(hipcstone_stream s, const K* keys, size_t numK
                                   uint32_t* newCounts, int32_t capacity, void* ws, size_t wsBytes, int* converged,
                                   const uint32_t* oldPos, uint32_t* posWs);
 
-// The neighbor search of hipcstone_find_neighbors_* with a workspace for the compact child blocks the fp32 open-box
-// walk reads (neighborGroupsBytes(numNodes) bytes; with less, or none, they are allocated on the stream per call).
+// The neighbor search of hipcstone_find_neighbors_* with a workspace for the compact child blocks the walk reads
+// (neighborGroupsBytes(numNodes) bytes; with less, or none, they are allocated on the stream per call).
 size_t neighborGroupsBytes(int32_t numNodes);
 template<class T>
 struct BoxOf;

@@ -1,9 +1,9 @@
 /*
  * hipcstone neighbor walk: the device side of the radius neighbor search, for HIP C++ code built for gfx950.
  *
- * One wave64 walks the octree for 64 consecutive targets and writes their neighbor rows. The library's search entry
+ * One wave64 walks the octree for up to 64 consecutive targets and hands each its neighbors. The library's search entry
  * points (hipcstone_find_neighbors_*, libhipcstone.so) launch it as is; hipcstone_ijloop.hpp instantiates it in the
- * caller's translation unit inside its fused interaction loop, which folds every wave's rows right after its walk.
+ * caller's translation unit inside its fused interaction loop, which folds the neighbors as they come.
  *
  * Reference semantics (findneighbors.hpp:77-177, traversal.hpp:26-69, boxoverlap.hpp:217-250, util/array.hpp:237-240):
  * particle i visits node n iff every node on the root->n path passes
@@ -11,25 +11,46 @@
  * and at each visited leaf records j != i with  dx*dx + dy*dy + dz*dz < 4 h_i^2  (left fold), ascending j,
  * keeping the first ngmax and counting all.
  *
- * Design — one wave64 owns 64 consecutive targets (compact in space because they are SFC-ordered):
- *  * Walk: depth-first with an explicit per-wave stack in LDS. Descending into a node evaluates its 8 children at
- *    once (their centers/sizes are contiguous, so a few wide scalar loads fetch them) and stores, per child, the
- *    ballot of lanes whose own predicate chain passed: a lane is tested at a child only if it passed the parent.
- *    A frame holds the children's lane masks and the first child's index; stepping to a child loads its child
- *    offset (and, for a leaf, its leaf index) with scalar loads.
+ * Design — one wave64 owns up to 64 consecutive targets (compact in space because they are SFC-ordered):
+ *  * Walk: depth-first with an explicit per-wave stack, one entry per lane of a few vector registers (readlane and
+ *    writelane at a uniform index), whose older half moves to LDS when it is full. Descending into a node evaluates its
+ *    8 children at once, from the compact record of the block (ChildGroup: one wide scalar load, and 12 additions for
+ *    the 8 distances), each with the ballot of lanes whose own predicate chain passed: a lane is tested at a child only
+ *    if it passed the parent. Where a block has no such record the children's own centers and sizes are loaded.
  *    The visited leaf set of every lane is therefore exactly the CPU's, not the superset a group-box walk gives.
  *    Children are taken in order 0..7, so leaves come out in the CPU's visiting order (ascending SFC order).
- *  * Leaves and their lane masks go to a per-wave list, drained in visiting order, so every target's neighbors come
- *    out in ascending j.
- *  * Leaf phase in pair slots: lanes are (target slot, leaf particle) pairs, so nearly all 64 lanes do useful pair
- *    tests even when only a few targets visit a leaf (a per-target lane layout leaves two thirds of the lanes idle
- *    on typical leaves). A ballot ranks each hit among its target's hits in ascending j, so every target's hits of a
- *    leaf are stored as one contiguous run of its row.
+ *  * Leaves and their lane masks go to a per-wave list. A full list becomes candidates: the listed leaves' particles
+ *    one after another, in chunks of 64. Each chunk is tested against all 64 targets on the matrix cores and leaves
+ *    every target one 64-bit word of hits, which then loses the candidates of leaves the target did not visit.
+ *  * Hit words are kept in LDS for several chunks, then every lane takes its own target's hits out of its words in
+ *    ascending order, four at a time, and hands them on (rows in memory, or a caller's fold over the neighbors).
  *  * Every loop is bounded: the walk by 2 * numNodes + 8 steps and the stack depth by the key's level count. A guard
  *    that fires ends the walk and ORs its HIPCSTONE_FAULT_* bit into the fault word.
  *
- * Everything is evaluated in the reference's floating-point order; compile with -ffp-contract=off and without
- * packed fp32 ops (-Xclang -target-feature -Xclang -packed-fp32-ops).
+ * The pair test on the matrix cores. With coordinates relative to a center c near the wave's targets,
+ *     D = |x_j - x_i|^2 - 4 h_i^2 = (|x_i|^2 - 4 h_i^2) + |x_j|^2 - 2 x_i . x_j
+ * is one 16x16x4 fp32 product (x_j, y_j, z_j, |x_j|^2) . (-2 x_i, -2 y_i, -2 z_i, 1) accumulated onto the target's
+ * constant: the sign of D is the test. D is not the reference's rounded distance, so the sign is taken only where
+ * |D| >= E, with E an upper bound of the error of D and of the reference's own distance for every pair that matters:
+ * with u = 2^-24, a = |x_i|, r = 2 h_i and S = 2 a + r, a pair with D near 0 has |x_j| <= a + r, so the roundings of
+ * the relative coordinates (2 u r S), of |x_j|^2 and |x_i|^2 (7 u S^2), of the four accumulations (each of at most
+ * (a + |x_j|)^2 + r^2 <= S^2 + r^2, counted with a whole ulp) and of the reference's distance (5 u r^2) stay below
+ * 16 u (S^2 + r^2); pairs farther away have D > |x_j|^2 / 4, far above their error. E is that bound at the wave's
+ * largest target. A chunk with a |D| < E (about one wave in five has one at 100 neighbors) tests the 16-candidate
+ * groups it occurs in again, in the reference's own operations; if E is not a normal number (coordinates or h out of
+ * fp32's range) every chunk is. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
+ * A wave with a target whose 2h box leaves a periodic domain folds its candidates to their images nearest to c. While
+ * S < L / 2 these are the reference's images for every pair that can be a hit, and the folded differences are off by at
+ * most 2 u L per dimension, the reference's included, so E grows by 8 u r L; with a larger S every chunk is tested in
+ * the reference's operations, and so is a chunk with a particle outside the domain (the reference folds only for
+ * targets near its faces).
+ *
+ * What bounds it is instruction issue: a wave of 64 targets with 100 neighbors takes 12.5K vector, 7.4K scalar and
+ * 2.6K branch instructions, and 322 matrix products, which replace some 90K multiply-adds and compares by lane. Pair
+ * tests one candidate at a time took 16.2K vector and 12.8K scalar instructions (16.8M targets: 7.70 ms, now 6.31).
+ *
+ * Everything that decides is evaluated in the reference's floating-point order; compile with -ffp-contract=off and
+ * without packed fp32 ops (-Xclang -target-feature -Xclang -packed-fp32-ops).
  */
 #pragma once
 
@@ -107,197 +128,258 @@ struct BoxOf<double>
 namespace nbwalk
 {
 
-constexpr int kMaxDepth = 22; // 21 levels below the root for 64-bit keys
-constexpr int kLeafList = 64;
+constexpr int kLeafList = kWave;
+// the walk's stack: 64 entries in registers, of which 32 at a time move to memory when they run out. A descent leaves
+// at most 7 siblings per level behind and adds 8: 21 levels below the root need at most 155 entries.
+constexpr int kSpillEntries = 32;
+constexpr int kSpills       = 3;
+// Chunks of 64 candidates whose hits are kept before they are taken out, and kept hit entries per target: as many as six
+// waves per SIMD leave LDS for. With more kept hits the lanes' counts differ less and fewer turns are spent on the fullest
+// lane, with more waves the latencies hide better: 16 chunks at 2 waves per SIMD took 13.0 ms, 10 at 3 9.9, 8 at 4 8.4.
+constexpr int kChunks  = 5;
+constexpr int kEntries = 13;
 
-// per leaf-chunk size nj in [1, 32]: slots = 64 / nj, the multiplier with floor(l / nj) == (l * magic) >> 16 for
-// every lane l < 64 (checked exhaustively), so the per-chunk slot layout needs no division, the lane mask of the
-// slots' last lanes {nj - 1, 2 nj - 1, ..., slots * nj - 1} and that of all slot lanes [0, slots * nj); one 32-byte
-// scalar load per chunk
-struct SlotInfo
-{
-    uint32_t magic;
-    uint32_t slots;
-    uint64_t last;
-    uint64_t inSlots;
-    uint64_t pad;
-};
-constexpr int kMaxChunk = 32;
-struct SlotTable
-{
-    SlotInfo e[kMaxChunk + 1];
-};
+typedef float Float4 __attribute__((ext_vector_type(4)));
 
-constexpr SlotTable makeSlotTable()
+// wave-wide inclusive scans (row shifts, then the rows' last lanes broadcast into the rows above)
+template<int Ctrl, int RowMask>
+__device__ inline uint32_t dppOrZero(uint32_t v)
 {
-    SlotTable t{};
-    for (int nj = 1; nj <= kMaxChunk; ++nj)
-    {
-        const int slots = kWave / nj;
-        t.e[nj].magic   = (65536u + uint32_t(nj) - 1) / uint32_t(nj);
-        t.e[nj].slots   = uint32_t(slots);
-        t.e[nj].last    = 0;
-        for (int k = 1; k <= slots; ++k)
-            t.e[nj].last |= uint64_t(1) << (k * nj - 1);
-        t.e[nj].inSlots = slots * nj >= kWave ? ~uint64_t(0) : (uint64_t(1) << (slots * nj)) - 1;
-    }
-    return t;
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), Ctrl, RowMask, 0xF, false));
+}
+template<class Op>
+__device__ inline uint32_t waveScan(uint32_t v, Op op)
+{
+    v = op(v, dppOrZero<0x111, 0xF>(v)); // row_shr:1
+    v = op(v, dppOrZero<0x112, 0xF>(v));
+    v = op(v, dppOrZero<0x114, 0xF>(v));
+    v = op(v, dppOrZero<0x118, 0xF>(v));
+    v = op(v, dppOrZero<0x142, 0xA>(v)); // row_bcast:15 into rows 1 and 3
+    return op(v, dppOrZero<0x143, 0xC>(v)); // row_bcast:31 into rows 2 and 3
+}
+__device__ inline uint32_t waveScanAdd(uint32_t v) { return waveScan(v, [](uint32_t a, uint32_t b) { return a + b; }); }
+__device__ inline uint32_t waveScanMax(uint32_t v)
+{
+    return waveScan(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 
-// one copy per translation unit, internal to it, so that device code addresses it relative to the program counter
-// (no global offset table entry to load first)
-namespace
+__device__ inline uint32_t readLane(uint32_t v, int l) { return uint32_t(__builtin_amdgcn_readlane(int(v), l)); }
+__device__ inline float readLane(float v, int l)
 {
-constexpr SlotTable kSlotTable = makeSlotTable();
+    return __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(__float_as_uint(v)), l)));
+}
+__device__ inline double readLane(double v, int l)
+{
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    return __longlong_as_double((long long)((uint64_t(readLane(uint32_t(b >> 32), l)) << 32) | readLane(uint32_t(b), l)));
 }
 
-// v + (this lane's bit of the wave-uniform mask) as one add with the mask as carry-in
-__device__ inline uint32_t addLaneBit(uint32_t v, uint64_t mask)
+// (a's rows 0, 1 and b's rows 0, 1), (a's rows 2, 3 and b's rows 2, 3), a row being 16 lanes
+__device__ inline void swapHalves(uint32_t& a, uint32_t& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a            = r[0];
+    b            = r[1];
+}
+// a's odd rows exchanged with b's even rows
+__device__ inline void swapRows(uint32_t& a, uint32_t& b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a            = r[0];
+    b            = r[1];
+}
+// 4 x 4 transpose of registers and rows: row k of register q becomes row q of register k
+__device__ inline void transposeRows(float (&f)[4])
+{
+    uint32_t v[4];
+    for (int k = 0; k < 4; ++k)
+        v[k] = __float_as_uint(f[k]);
+    swapHalves(v[0], v[2]);
+    swapHalves(v[1], v[3]);
+    swapRows(v[0], v[1]);
+    swapRows(v[2], v[3]);
+    for (int k = 0; k < 4; ++k)
+        f[k] = __uint_as_float(v[k]);
+}
+
+// index of the lowest set bit, 2^32 - 1 for zero (one instruction; the language's forms leave zero undefined or
+// select a value for it)
+__device__ inline uint32_t lowestBit(uint32_t v)
 {
     uint32_t r;
-    uint64_t carryOut;
-    asm("v_addc_co_u32_e64 %0, %1, %2, 0, %3" : "=v"(r), "=s"(carryOut) : "v"(v), "s"(mask));
+    asm("v_ffbl_b32 %0, %1" : "=v"(r) : "v"(v));
     return r;
 }
 
-// all ones if bit b of the wave-uniform v is set, else zero (one scalar sign-extending bit-field extract)
-__device__ inline uint32_t sbfeBit(uint32_t v, int b) { return uint32_t(__builtin_amdgcn_sbfe(int(v), b, 1)); }
-
-// a1 where the wave-uniform m is set, a0 elsewhere, as one v_bfi_b32 (the compiler would otherwise turn the bit
-// select of an all-ones-or-zero mask into a scalar compare, a scalar select of a lane mask and a v_cndmask)
-__device__ inline float pickBits(uint32_t m, uint32_t a1, uint32_t a0)
+// lo |= low half, hi |= high half of v in the lanes of the mask. Call where all lanes are active.
+__device__ inline void orLanes(uint64_t mask, uint64_t v, uint32_t& lo, uint32_t& hi)
 {
-    uint32_t r;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(m), "v"(a1), "v"(a0));
-    return __uint_as_float(r);
+    asm volatile("s_mov_b64 exec, %2\n\tv_or_b32_e32 %0, %3, %0\n\tv_or_b32_e32 %1, %4, %1\n\ts_mov_b64 exec, -1"
+        : "+v"(lo), "+v"(hi)
+        : "s"(mask), "s"(uint32_t(v)), "s"(uint32_t(v >> 32)));
 }
 
-// bit k set iff m[k] != 0, two scalar instructions per mask (compare, then shift the compare bit in)
-__device__ inline uint32_t nonzeroBits8(const uint64_t* m)
+// v with lane l's value replaced by the wave-uniform x (l < 64), which has no clang builtin
+__device__ int writeLaneI32(int x, int l, int v) __asm("llvm.amdgcn.writelane.i32");
+__device__ inline uint32_t writeLane(uint32_t v, int l, uint32_t x) { return uint32_t(writeLaneI32(int(x), l, int(v))); }
+
+// m[k] = lanes of `in` with v[k] < r: the compares run under `in`, which masks them for nothing. Call where all lanes
+// are active.
+__device__ inline void lessIn(uint64_t in, const float (&v)[8], float r, uint64_t (&m)[8])
 {
-    uint32_t acc = 0;
-    asm("s_cmp_lg_u64 %1, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %2, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %3, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %4, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %5, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %6, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %7, 0\n\ts_addc_u32 %0, %0, %0\n\t"
-        "s_cmp_lg_u64 %8, 0\n\ts_addc_u32 %0, %0, %0"
-        : "+s"(acc)
-        : "s"(m[7]), "s"(m[6]), "s"(m[5]), "s"(m[4]), "s"(m[3]), "s"(m[2]), "s"(m[1]), "s"(m[0])
-        : "scc");
-    return acc;
+    asm volatile("s_mov_b64 exec, %8\n\t"
+        "v_cmp_lt_f32_e64 %0, %9, %17\n\tv_cmp_lt_f32_e64 %1, %10, %17\n\t"
+        "v_cmp_lt_f32_e64 %2, %11, %17\n\tv_cmp_lt_f32_e64 %3, %12, %17\n\t"
+        "v_cmp_lt_f32_e64 %4, %13, %17\n\tv_cmp_lt_f32_e64 %5, %14, %17\n\t"
+        "v_cmp_lt_f32_e64 %6, %15, %17\n\tv_cmp_lt_f32_e64 %7, %16, %17\n\t"
+        "s_mov_b64 exec, -1"
+        : "=&s"(m[0]), "=&s"(m[1]), "=&s"(m[2]), "=&s"(m[3]), "=&s"(m[4]), "=&s"(m[5]), "=&s"(m[6]), "=&s"(m[7])
+        : "s"(in), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(r));
+}
+__device__ inline void lessIn(uint64_t in, const double (&v)[8], double r, uint64_t (&m)[8])
+{
+    asm volatile("s_mov_b64 exec, %8\n\t"
+        "v_cmp_lt_f64_e64 %0, %9, %17\n\tv_cmp_lt_f64_e64 %1, %10, %17\n\t"
+        "v_cmp_lt_f64_e64 %2, %11, %17\n\tv_cmp_lt_f64_e64 %3, %12, %17\n\t"
+        "v_cmp_lt_f64_e64 %4, %13, %17\n\tv_cmp_lt_f64_e64 %5, %14, %17\n\t"
+        "v_cmp_lt_f64_e64 %6, %15, %17\n\tv_cmp_lt_f64_e64 %7, %16, %17\n\t"
+        "s_mov_b64 exec, -1"
+        : "=&s"(m[0]), "=&s"(m[1]), "=&s"(m[2]), "=&s"(m[3]), "=&s"(m[4]), "=&s"(m[5]), "=&s"(m[6]), "=&s"(m[7])
+        : "s"(in), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(r));
 }
 
-// the structured buffer store of the LLVM AMDGPU back end (address = base + vindex * stride; with stride != 0 a
-// vindex at or past the record count is out of range and the store is dropped), which has no clang builtin
-__device__ void structBufferStoreB32(uint32_t data, __amdgpu_buffer_rsrc_t rsrc, int vindex, int voffset, int soffset,
-                                     int aux) __asm("llvm.amdgcn.struct.ptr.buffer.store.i32");
-
-// the matching structured buffer load of one 32-bit value (an index at or past the record count reads zero)
+// the structured buffer load of the LLVM AMDGPU back end (address = base + vindex * stride), which has no clang builtin:
+// fp32 coordinates as buffers of 4-byte records take the particle index itself, with no 64-bit address arithmetic
 __device__ float structBufferLoadF32(__amdgpu_buffer_rsrc_t rsrc, int vindex, int voffset, int soffset,
                                      int aux) __asm("llvm.amdgcn.struct.ptr.buffer.load.f32");
 
 // dword 3 of an untyped, unswizzled buffer resource on gfx9-family targets (32-bit data format); with a stride in
-// dword 1, accesses are range checked against the record count in dword 2
+// dword 1, accesses are range checked against the record count in dword 2 (none here)
 constexpr int kBufferFlags = 0x00020000;
 
-template<class T>
-struct alignas(4 * sizeof(T)) Particle4
+// the LDS of one walking wave
+struct WaveShared
 {
-    T x, y, z, w;
+    uint32_t spilled[kSpills][3][kSpillEntries]; // stack entries that did not fit the registers
+    uint32_t marks[kWave];                       // scratch of one chunk
+    uint32_t cand[(kChunks + 1) * kWave];        // the kept chunks' candidates (particle indices), and the next one's
+    uint32_t entries[kEntries + 1][kWave];       // column l: target l's kept hits (see HitReader), then a zero
 };
 
-template<class T>
-struct alignas(4 * sizeof(T)) TargetRec
-{
-    Particle4<T> p; // x, y, z, 4h^2
-    uint32_t wpos;  // element offset (from the wave's first row) of the target's next neighbor slot
-    uint32_t limit; // element offset of the end of the target's row
-    uint32_t meta;  // periodic-image flags (bits 0-2) | lane of the target (bits 8-13)
-    uint32_t pad;
-};
+// LDS by its address
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+__device__ inline uint32_t ldsAddress(const void* p) { return uint32_t((__UINTPTR_TYPE__)(const LdsWord*)p); }
+__device__ inline uint32_t ldsRead(uint32_t address) { return *(const LdsWord*)(__UINTPTR_TYPE__)address; }
+__device__ inline void ldsWrite(uint32_t address, uint32_t v) { *(LdsWord*)(__UINTPTR_TYPE__)address = v; }
 
-// the LDS of kNbWaves walking waves
 template<class T, int kNbWaves>
 struct Shared
 {
-    uint64_t mask[kNbWaves][kMaxDepth][8];
-    int32_t co[kNbWaves][kMaxDepth];
-    uint32_t rem[kNbWaves][kMaxDepth]; // bit k: child k of the frame has lanes and is not taken yet
-    int32_t listLeaf[kNbWaves][kLeafList];
-    uint64_t listMask[kNbWaves][kLeafList];
-    // the current leaf's active targets, compacted in lane order: wave w's records are [w * 64, w * 64 + 64); the
-    // 64 records past the last wave's are padding, so slot indexes up to 127 read inside the array (such reads
-    // belong to slots without a target and are masked out) and need no clamp
-    TargetRec<T> ctgt[kNbWaves * kWave + kWave];
+    WaveShared wave[kNbWaves];
 };
 
-// The 8 children of one internal node in a compact form (fp32 trees): in each dimension the children's centers take
-// two values and their sizes one (true of geometric centers, which depend only on a node's integer box), so a
-// child's distance terms are one of two values per dimension, computed once per lane for all 8 children. Record g
-// describes the children [8 g + 1, 8 g + 9), the child block of some internal node in the level-major layout.
-//   v0, v1, s: the two center values and the size per dimension (v1 == v0 where only one value occurs)
-//   perm:      bit 4 k + 2 - d is set if child k's center in dimension d is v1
-//   flags:     bit k set if child k is internal; kGroupValid if every child matched v0/v1 and s bit for bit (the
-//              walk falls back to the children's own centers and sizes otherwise)
-//   leaf:      the children's leaf indices (internalToLeaf)
+// The 8 children of one internal node in a compact form. In each dimension geometric centers depend only on the node's
+// integer box, so the children's centers take two values and their sizes one, and along the Hilbert curve (which all
+// node boxes are decoded from) the children's octants follow one pattern up to the order of the axes: one axis changes
+// with every second child (kFast), one with every fourth (kMiddle), one half way (kSlow). With the first child's
+// center as each axis' first value, child k therefore lies at the second one where bit k of the axis' pattern is set.
+// Record g describes the children [8 g + 1, 8 g + 9), the child block of some internal node.
+//   v0, v1, s: the center of child 0, the other center and the size, for x, for the faster of y and z, and for the other
+//   flags:     bit k set if child k is internal; kXFast, kXMiddle: x's pattern (neither: it is the slow axis); kZFaster:
+//              z is faster than y; kGroupValid if every child matched bit for bit (else the walk takes the children's
+//              own centers and sizes); kGroupOutside if an internal child's block lies outside the tree,
+//              kGroupBackward if one does not come after its parent
+//   link:      a leaf child's leaf index (internalToLeaf), an internal child's own child block (childOffsets)
+template<class T>
 struct alignas(128) ChildGroup
 {
-    float v0[3], v1[3], s[3];
-    uint32_t perm;
+    T v0[3], v1[3], s[3];
     uint32_t flags;
-    uint32_t pad[5];
-    int32_t leaf[8];
+    alignas(32) int32_t link[8];
 };
-typedef uint32_t ChildGroupHead __attribute__((ext_vector_type(16))); // dwords 0-15 of a ChildGroup, one load
-constexpr uint32_t kGroupValid = 0x80000000u;
+typedef uint32_t Words16 __attribute__((ext_vector_type(16)));
+typedef uint32_t Words8 __attribute__((ext_vector_type(8)));
+typedef int32_t Links8 __attribute__((ext_vector_type(8)));
+constexpr uint32_t kGroupValid = 0x80000000u, kGroupOutside = 0x40000000u, kGroupBackward = 0x20000000u;
+constexpr uint32_t kXFast = 0x100u, kXMiddle = 0x200u, kZFaster = 0x400u;
+constexpr uint32_t kFast = 0x66u, kMiddle = 0x3Cu, kSlow = 0xF0u;
 
-// the ChildGroup records of an fp32 tree with numNodes nodes: (numNodes - 1) / 8 of them (none for a root-only tree)
+// the ChildGroup records of a tree with numNodes nodes: (numNodes - 1) / 8 of them (none for a root-only tree)
 inline size_t childGroupCount(int32_t numNodes) { return numNodes > 8 ? size_t((numNodes - 1) / 8) : 0; }
 
 // builds the ChildGroup records, one thread per block of 8 children [8 g + 1, 8 g + 9); a template so that every
 // translation unit that launches it has its own copy
-template<int = 0>
-__global__ void childGroupsKernel(const float* __restrict__ centers, const float* __restrict__ sizes,
+template<class T>
+__global__ void childGroupsKernel(const T* __restrict__ centers, const T* __restrict__ sizes,
                                   const int32_t* __restrict__ childOffsets, const int32_t* __restrict__ internalToLeaf,
-                                  uint32_t numGroups, ChildGroup* __restrict__ groups)
+                                  int32_t numNodes, uint32_t numGroups, ChildGroup<T>* __restrict__ groups)
 {
+    using Bits = std::conditional_t<std::is_same_v<T, float>, uint32_t, uint64_t>;
+    auto bits  = [](T v) { return __builtin_bit_cast(Bits, v); };
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= numGroups) return;
     const size_t co = size_t(g) * 8 + 1;
-    ChildGroup r{};
-    bool same      = true;
-    uint32_t perm  = 0;
-    uint32_t inner = 0;
+    bool same = true;
+    T v0[3], v1[3], size[3];
+    uint32_t pattern[3];
     for (int d = 0; d < 3; ++d)
     {
-        const uint32_t a = __float_as_uint(centers[co * 3 + d]);
-        const uint32_t s = __float_as_uint(sizes[co * 3 + d]);
-        uint32_t b       = a;
+        const T a  = centers[co * 3 + d];
+        const T s  = sizes[co * 3 + d];
+        T b        = a;
+        pattern[d] = 0;
         for (int k = 1; k < 8; ++k)
         {
-            const uint32_t c = __float_as_uint(centers[(co + k) * 3 + d]);
-            if (c != a)
+            const T c = centers[(co + k) * 3 + d];
+            if (bits(c) != bits(a))
             {
-                if (b == a) b = c;
-                same = same && c == b;
-                perm |= 1u << (4 * k + 2 - d);
+                if (pattern[d] == 0) b = c;
+                same = same && bits(c) == bits(b);
+                pattern[d] |= 1u << k;
             }
-            same = same && __float_as_uint(sizes[(co + k) * 3 + d]) == s;
+            same = same && bits(sizes[(co + k) * 3 + d]) == bits(s);
         }
-        r.v0[d] = __uint_as_float(a);
-        r.v1[d] = __uint_as_float(b);
-        r.s[d]  = __uint_as_float(s);
+        v0[d]   = a;
+        v1[d]   = b;
+        size[d] = s;
+    }
+    // the axes' order; an axis whose two centers round to one value goes with any pattern
+    constexpr uint32_t kOrders[6][4] = {{kFast, kMiddle, kSlow, kXFast},   {kFast, kSlow, kMiddle, kXFast | kZFaster},
+                                        {kMiddle, kFast, kSlow, kXMiddle}, {kMiddle, kSlow, kFast, kXMiddle | kZFaster},
+                                        {kSlow, kFast, kMiddle, 0u},       {kSlow, kMiddle, kFast, kZFaster}};
+    bool found     = false;
+    uint32_t flags = 0;
+    for (int o = 0; o < 6; ++o)
+    {
+        bool ok = true;
+        for (int d = 0; d < 3; ++d)
+            ok = ok && (pattern[d] == kOrders[o][d] || pattern[d] == 0);
+        if (ok && !found)
+        {
+            found = true;
+            flags = kOrders[o][3];
+        }
+    }
+    ChildGroup<T> r{};
+    const bool swapped = (flags & kZFaster) != 0;
+    for (int d = 0; d < 3; ++d)
+    {
+        const int to = d == 0 || !swapped ? d : 3 - d;
+        r.v0[to]     = v0[d];
+        r.v1[to]     = v1[d];
+        r.s[to]      = size[d];
     }
     for (int k = 0; k < 8; ++k)
     {
-        inner |= uint32_t(childOffsets[co + k] != 0) << k;
-        r.leaf[k] = internalToLeaf[co + k];
+        const int32_t child = childOffsets[co + k];
+        r.link[k]           = child != 0 ? child : internalToLeaf[co + k];
+        if (child == 0) continue;
+        flags |= 1u << k;
+        if (child < 0 || child > numNodes - 8) flags |= kGroupOutside;
+        if (child <= int32_t(co) + k) flags |= kGroupBackward;
     }
-    r.perm    = perm;
-    r.flags   = inner | (same ? kGroupValid : 0u);
+    if (same && found) flags |= kGroupValid;
+    r.flags   = flags;
     groups[g] = r;
 }
 
@@ -315,27 +397,61 @@ struct Tree
     const T* sizes;
     int32_t numNodes;
     float ext;
-    // optional (fp32, open boxes): the child blocks in compact form, numbered by (first child - 1) / 8
-    const ChildGroup* groups = nullptr;
+    // optional: the child blocks in compact form, numbered by (first child - 1) / 8
+    const ChildGroup<T>* groups = nullptr;
 };
 
 /*
- * Walks the tree from `root` for the wave's targets first + lane (lanes with `valid` false take no part) and writes
- * their neighbor rows; returns this lane's neighbor count (all neighbors, of which the first ngmax are stored).
+ * A target's kept hits, in ascending order. They lie in its lane's column of WaveShared::entries, one entry per group of
+ * 16 consecutive candidates that has any: bits 0-15 the hits, bits 16-31 the address of the group's first candidate
+ * (in words of LDS). next() may be called past the last hit (by lanes that have fewer than others): the zero entry at
+ * the end then stays the current one and some word of LDS is returned.
+ */
+struct HitReader
+{
+    uint32_t at, end;    // addresses of the entry read ahead and of the last, zero one
+    uint32_t cur, ahead; // the entry being emptied, the one after it
+
+    static constexpr uint32_t kEntryStep = kWave * sizeof(uint32_t);
+
+    __device__ inline HitReader(uint32_t from, uint32_t last)
+        : at(min(from + kEntryStep, last))
+        , end(last)
+        , cur(ldsRead(from))
+        , ahead(ldsRead(at))
+    {
+    }
+
+    __device__ inline uint32_t next()
+    {
+        const uint32_t j = ldsRead(((cur >> 16) + lowestBit(cur)) * 4u);
+        cur &= cur - 1;
+        if (uint16_t(cur) == 0)
+        {
+            cur   = ahead;
+            at    = min(at + kEntryStep, end);
+            ahead = ldsRead(at);
+        }
+        return j;
+    }
+};
+
+/*
+ * Walks the tree from `root` for the wave's targets first + lane (lanes with `valid` false take no part); returns this
+ * lane's neighbor count (all neighbors). Whenever hits have been collected, consume(before, hits, next) is called from all
+ * lanes: `before` and `hits` are the numbers of this target's neighbors handed on before and now, and next() returns the
+ * latter one by one, in ascending order. consume is not called if `handOn` is false (only the counts are wanted).
  *
- * Rows: lane l's row starts at rows + l * ngmax (row-major) or, with SlotMajor, neighbor k of lane l is at
- * rows[k * 64 + l]. rowsBytes is the byte size of the row buffer: stores past it are dropped by the hardware's
- * range check (row-major: the rows of the wave's targets only, SlotMajor: all 64 rows).
  * Segmented: the tree is one of many in the same arrays, children may lie before their parents (only the bounds
  * and depth guards and the step budget apply).
- * w is the wave's index in its workgroup (its part of `sh`). Call from all 64 lanes, with wave-uniform arguments
+ * w is the wave's index in its workgroup (its part of `shared`). Call from all 64 lanes, with wave-uniform arguments
  * except `valid`.
  */
-template<class T, bool AnyPbc, bool SlotMajor, bool Segmented, int kNbWaves>
+template<class T, bool AnyPbc, bool Segmented, int kNbWaves, class Consume>
 __device__ __attribute__((always_inline)) inline uint32_t
 walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, const T* __restrict__ h,
-     const typename BoxOf<T>::type& box, const Tree<T>& tree, int32_t root, uint64_t first, bool valid,
-     uint32_t ngmax, uint32_t* rowsPtr, uint32_t rowsBytes, Shared<T, kNbWaves>& sh, int w, uint32_t* faults)
+     const typename BoxOf<T>::type& box, const Tree<T>& tree, int32_t root, uint64_t first, bool valid, bool handOn,
+     Shared<T, kNbWaves>& shared, int w, uint32_t* faults, Consume&& consume)
 {
     const int32_t* __restrict__ childOffsets   = tree.childOffsets;
     const int32_t* __restrict__ internalToLeaf = tree.internalToLeaf;
@@ -343,8 +459,8 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
     const T* __restrict__ centers              = tree.centers;
     const T* __restrict__ sizes                = tree.sizes;
     const int32_t numNodes                     = tree.numNodes;
-    constexpr bool kGroups = std::is_same_v<T, float> && !AnyPbc;
-    const ChildGroup* __restrict__ groups = kGroups ? tree.groups : nullptr;
+    const ChildGroup<T>* __restrict__ groups   = tree.groups;
+    WaveShared& sh = shared.wave[w];
 
     const int lane   = laneId();
     const uint32_t i = uint32_t(first) + uint32_t(lane);
@@ -357,8 +473,8 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
         zi = z[i];
         hi = h[i];
     }
-    const T radiusSq = T(4.0) * hi * hi;
-    const T cellR2   = radiusSq * T(tree.ext) * T(tree.ext);
+    const T radiusSq0 = T(4.0) * hi * hi;
+    const T cellR2    = radiusSq0 * T(tree.ext) * T(tree.ext);
 
     // periodic images only for particles whose 2h box leaves the domain (findneighbors.hpp:102-104)
     bool px = false, py = false, pz = false;
@@ -386,17 +502,111 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
         return d0 * d0 + (d1 * d1 + d2 * d2);
     };
 
-    // per-target state: the lane of target t keeps its next row slot in a register (the count is wpos - rowOff, all
-    // neighbors counted, only the first ngmax stored); while a leaf is drained the leaf's active targets are copied,
-    // compacted, into LDS for the lanes that test them
-    constexpr uint32_t kSlotStep = SlotMajor ? uint32_t(kWave) : 1u; // element distance of consecutive slots
-    const uint32_t rowOff        = SlotMajor ? uint32_t(lane) : uint32_t(lane) * ngmax;
-    const TargetRec<T> myRec{Particle4<T>{xi, yi, zi, radiusSq}, rowOff, rowOff + ngmax * kSlotStep,
-                             uint32_t((px ? 1 : 0) | (py ? 2 : 0) | (pz ? 4 : 0)) | (uint32_t(lane) << 8), 0u};
-    uint32_t myWpos = rowOff;
+    // the pair test in the reference's operations (with radiusSq0, which the rare callers compute anew)
+    auto close = [&](T xj, T yj, T zj, T radiusSq) -> bool {
+        T xx = fold(xj - xi, px, 0);
+        T yy = fold(yj - yi, py, 1);
+        T zz = fold(zj - zi, pz, 2);
+        return xx * xx + yy * yy + zz * zz < radiusSq;
+    };
 
-    // fp32 particle coordinates as structured buffers of 4-byte records (no range limit): the leaf phase's loads
-    // then take the particle index itself, with no 64-bit address arithmetic
+    const T* rc             = centers + size_t(root) * 3;
+    const T* rsz            = sizes + size_t(root) * 3;
+    const uint64_t rootMask = ballot(valid & (nodeDist2(rc[0], rc[1], rc[2], rsz[0], rsz[1], rsz[2]) < cellR2));
+    if (rootMask == 0) return 0;
+    const bool inRoot = laneIn(rootMask);
+
+    // ---- operands of the matrix-core pair test (see the top of this file). The center is the mean of four targets
+    //      spread over the wave's; lanes without a target stand at the first one's place and get a constant that
+    //      keeps D far above zero.
+    const int laneF = __builtin_ctzll(rootMask);
+    const int laneL = 63 - __builtin_clzll(rootMask);
+    auto middle     = [&](T p) -> T {
+        const T q = inRoot ? p : readLane(p, laneF);
+        T s       = 0;
+#pragma unroll
+        for (int k = 1; k < 8; k += 2)
+            s += readLane(q, laneF + (laneL - laneF) * k / 8);
+        return readLane(s * T(0.25), 0); // (held in scalar registers)
+    };
+    const T cx = middle(xi), cy = middle(yi), cz = middle(zi);
+    float tgt[4];
+    Float4 tgtConst[4]; // per 16 targets: the constant of target lane % 16, in every register of the accumulator
+    float errBound;
+    bool allExact;
+    [[maybe_unused]] bool images = false; // some target's neighbors are looked for across a periodic face
+    {
+        const float xr  = inRoot ? float(xi - cx) : 0.0f;
+        const float yr  = inRoot ? float(yi - cy) : 0.0f;
+        const float zr  = inRoot ? float(zi - cz) : 0.0f;
+        const float a2  = xr * xr + yr * yr + zr * zr;
+        const float r2  = inRoot ? float(radiusSq0) : 0.0f;
+        const float s   = 2.0f * __builtin_amdgcn_sqrtf(a2) + __builtin_amdgcn_sqrtf(r2);
+        const float s2r = inRoot ? s * s + r2 : 0.0f;
+        // (non-negative floats order as their bit patterns; a NaN's is above infinity's)
+        const float most = __uint_as_float(readLane(waveScanMax(__float_as_uint(s2r) & 0x7FFFFFFFu), kWave - 1));
+        errBound         = readLane(1.0e-6f * most, 0); // 16 u (S^2 + r^2), rounded up
+        allExact         = !(errBound >= 1.0e-30f && errBound <= 1.0e20f);
+        if constexpr (AnyPbc)
+        {
+            images = ballot(px | py | pz) != 0;
+            if (images)
+            {
+                const float mostR2 = __uint_as_float(readLane(waveScanMax(__float_as_uint(r2) & 0x7FFFFFFFu), kWave - 1));
+                float longest      = 0.0f;
+                for (int d = 0; d < 3; ++d)
+                {
+                    if (box.bnd[d] != HIPCSTONE_PERIODIC) continue;
+                    longest  = fmaxf(longest, float(box.len[d]));
+                    allExact = allExact || !(sqrtf(most) < 0.4999f * float(box.len[d]));
+                }
+                // (u of the coordinates' own type: fp64 ones are folded in fp64)
+                constexpr float kFold = std::is_same_v<T, float> ? 5.0e-7f : 1.0e-15f;
+                errBound = readLane(errBound + kFold * sqrtf(mostR2) * longest, 0);
+                allExact = allExact || !(errBound <= 1.0e20f);
+            }
+        }
+        float c0[4];
+        c0[0] = c0[1] = c0[2] = c0[3] = inRoot ? a2 - r2 : 1.0e30f;
+        transposeRows(c0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            tgtConst[t] = Float4{c0[t], c0[t], c0[t], c0[t]};
+        tgt[0] = -2.0f * xr;
+        tgt[1] = -2.0f * yr;
+        tgt[2] = -2.0f * zr;
+        tgt[3] = 1.0f;
+        transposeRows(tgt);
+    }
+    // the candidate (of a chunk of 64) whose position this lane loads: with rows 4 g + r of the q-th product being
+    // candidates 16 g + 4 q + r, the 16 results a lane gets for one target are 16 consecutive candidates
+    const int loadPos = 16 * ((lane & 15) >> 2) + 4 * (lane >> 4) + (lane & 3);
+    // byte selector that joins the even rows' low or the odd rows' high halves of two words
+    const uint32_t halfSel = (lane & 16) ? 0x07060302u : 0x05040100u;
+
+    uint32_t total   = 0; // neighbors of this lane's target so far
+    uint32_t handed  = 0; // those of them handed on
+    int numChunks    = 0; // kept chunks
+    uint32_t slot    = 0; // the next chunk's place in sh.cand, a ring
+    // the place of this lane's next entry
+    const uint32_t entriesAt = ldsAddress(&sh.entries[0][0]);
+    uint32_t entryEnd        = entriesAt + uint32_t(lane) * 4u;
+    const uint32_t candAt = ldsAddress(sh.cand) / 4u;
+
+    auto handOver = [&]() __attribute__((always_inline)) {
+        ldsWrite(entryEnd, 0);
+        waveSync();
+        if (handOn)
+        {
+            HitReader hits(entriesAt + uint32_t(lane) * 4u, entryEnd);
+            consume(handed, total - handed, [&]() __attribute__((always_inline)) { return hits.next(); });
+        }
+        waveSync();
+        handed    = total;
+        numChunks = 0;
+        entryEnd  = entriesAt + uint32_t(lane) * 4u;
+    };
+
     [[maybe_unused]] __amdgpu_buffer_rsrc_t xRes, yRes, zRes;
     if constexpr (std::is_same_v<T, float>)
     {
@@ -405,410 +615,405 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
         zRes = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(z), 4, -1, kBufferFlags);
     }
 
-    // the wave's output rows as a structured buffer of 4-byte records: a store takes the row slot itself as its
-    // index, and a lane without a hit stores at index 2^32 - 1, past the record count, where the hardware's range
-    // check drops it (no branch around the store, no byte-offset arithmetic)
-    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-        rowsBytes ? static_cast<void*>(rowsPtr) : nullptr, 4, int(rowsBytes / 4u), kBufferFlags);
+    // ---- leaves to be tested, in visiting order: entry e in lane e (the leaf and the lanes that visit it)
+    uint32_t listLeaf = 0, listLo = 0, listHi = 0;
+    int listCount   = 0;
+    auto appendLeaf = [&](int32_t leafIdx, uint64_t m) __attribute__((always_inline)) {
+        listLeaf = writeLane(listLeaf, listCount, uint32_t(leafIdx));
+        listLo   = writeLane(listLo, listCount, uint32_t(m));
+        listHi   = writeLane(listHi, listCount, uint32_t(m >> 32));
+        ++listCount;
+        // (keeps the compiler from merging this tail with the stack's, which would put both counts into memory)
+        asm volatile("; listed");
+    };
 
-    // ---- leaf phase. A leaf chunk of nj <= 32 particles is tested against its active targets in pair slots:
-    //      lane = (slot, jj) with slot = lane / nj, jj = lane % nj, S = 64 / nj slots; slot s of an iteration tests
-    //      active targets k = k0 + s and k0 + S + s (two independent targets per lane, for instruction-level
-    //      parallelism) against particle jj. Within a slot, lanes are ascending jj, so the ballot of hits ranks each
-    //      hit among its target's hits in ascending j and all of a target's hits of the chunk land contiguously in
-    //      its row (coalesced runs). The slot's last lane advances the target's count. Chunks are taken in order,
-    //      at most 32 particles each: a leaf of 33-64 particles as one chunk would have one slot per iteration,
-    //      as 32 + the rest it has at least two. ----
-    int listCount = 0;
-    // drain and its pair-loop body are forced inline: as out-of-line calls their captured state (the row
-    // buffer resource among it) would live in scratch memory
-    auto drain = [&]() __attribute__((always_inline)) {
-        waveSync();
-        for (int e = 0; e < listCount; ++e)
+    // ---- the listed leaves' particles become candidates, 64 at a time, and are tested; `last`: nothing follows
+    auto drain = [&](bool last) __attribute__((always_inline)) {
+        uint32_t jb = 0, cnt = 0;
+        if (lane < listCount)
         {
-            int32_t leafIdx = uniform(sh.listLeaf[w][e]);
-            uint64_t m      = uniform64(sh.listMask[w][e]);
-            uint32_t jb     = uniform(layout[leafIdx]);
-            uint32_t je     = uniform(layout[leafIdx + 1]);
-            const uint32_t pc     = uint32_t(__builtin_popcountll(m));
-            const bool mine       = laneIn(m);
-            const unsigned myRank = laneRank(m);
-            TargetRec<T>* recs    = &sh.ctgt[w * kWave];
-            if (mine)
-            {
-                TargetRec<T> r = myRec;
-                r.wpos         = myWpos;
-                recs[myRank]   = r;
-            }
-            // no active target can reach the end of its row in this leaf (at most je - jb hits each): the
-            // per-hit row-end compare is skipped. wpos keeps counting past the row end, so compare in 64 bits.
-            const bool fits = uint64_t(myWpos) + uint64_t(je - jb) * kSlotStep <= uint64_t(myRec.limit);
-            const bool noOverflow = (ballot(!fits) & m) == 0;
-            waveSync();
-            for (uint32_t cs = jb, nj = 0; cs < je; cs += nj)
-            {
-                nj                = je - cs < uint32_t(kMaxChunk) ? je - cs : uint32_t(kMaxChunk);
-                const SlotInfo si = kSlotTable.e[nj];
-                const uint32_t S  = si.slots;
-                uint32_t slot     = __umul24(uint32_t(lane), si.magic) >> 16; // lane < 64, magic <= 2^16
-                uint32_t jj       = uint32_t(lane) - slot * nj;
-                uint32_t j        = cs + jj;
-                // lanes of this and later slots (slot * nj < 64): a hit's rank among its slot's hits
-                const uint64_t notBelow = ~uint64_t(0) << (slot * nj);
-                const uint32_t nbLo     = uint32_t(notBelow);
-                const uint32_t nbHi     = uint32_t(notBelow >> 32);
-                // the slots' last lanes: each advances the count of its slot's target
-                const uint64_t lastLanes = si.last;
-                // lanes of the first b slots, [0, b * nj), as a wave-uniform mask (scalar arithmetic)
-                auto slotsBelow = [&](uint32_t b) -> uint64_t {
-                    const uint32_t bits = b * nj;
-                    return bits >= uint32_t(kWave) ? ~uint64_t(0) : (uint64_t(1) << bits) - 1;
-                };
-                // lanes past the last slot test a NaN particle, which fails every distance compare
-                T xj = std::numeric_limits<T>::quiet_NaN(), yj = xj, zj = xj;
-                if constexpr (std::is_same_v<T, float>)
-                {
-                    // every lane loads (spare lanes a particle of the chunk), only x is replaced by the NaN: no
-                    // lane mask around the loads
-                    const uint32_t jc = j < je ? j : je - 1;
-                    xj                = structBufferLoadF32(xRes, int(jc), 0, 0, 0);
-                    yj                = structBufferLoadF32(yRes, int(jc), 0, 0, 0);
-                    zj                = structBufferLoadF32(zRes, int(jc), 0, 0, 0);
-                    xj                = laneIn(si.inSlots) ? xj : std::numeric_limits<T>::quiet_NaN();
-                }
-                else
-                {
-                    if (slot < S)
-                    {
-                        xj = x[j];
-                        yj = y[j];
-                        zj = z[j];
-                    }
-                }
-                // j == i is possible only if the chunk overlaps this wave's own targets
-                // (one unsigned compare: cs + nj - 1 - first wraps to a large value when the chunk ends before first)
-                const bool selfChunk = cs + nj - 1u - uint32_t(first) <= uint32_t(kWave) - 2u + nj;
-                const uint32_t jRel  = j - uint32_t(first);
+            jb  = layout[int32_t(listLeaf)];
+            cnt = layout[int32_t(listLeaf) + 1] - jb;
+        }
+        // leaves without particles leave the list
+        const uint64_t filled = ballot(cnt != 0);
+        if (filled != (listCount == kWave ? ~uint64_t(0) : (uint64_t(1) << listCount) - 1))
+        {
+            const uint32_t numFilled = uint32_t(__builtin_popcountll(filled));
+            const int to = int((cnt != 0 ? laneRank(filled) : numFilled + laneRank(~filled)) << 2);
+            jb           = uint32_t(__builtin_amdgcn_ds_permute(to, int(jb)));
+            cnt          = uint32_t(__builtin_amdgcn_ds_permute(to, int(cnt)));
+            listLo       = uint32_t(__builtin_amdgcn_ds_permute(to, int(listLo)));
+            listHi       = uint32_t(__builtin_amdgcn_ds_permute(to, int(listHi)));
+        }
+        const uint32_t upTo = waveScanAdd(cnt);
+        const uint32_t off  = upTo - cnt; // the leaf's first position among the candidates
+        const uint32_t num  = readLane(upTo, kWave - 1);
 
-                // the pair test of particle j against a target record: distance (and, in chunks that overlap the
-                // wave's own targets, j != target); each condition is a single compare, so its ballot is the
-                // compare's own lane mask
-                auto close = [&](const TargetRec<T>& rec) -> bool {
-                    bool fx = false, fy = false, fz = false;
-                    if constexpr (AnyPbc)
-                    {
-                        fx = rec.meta & 1;
-                        fy = rec.meta & 2;
-                        fz = rec.meta & 4;
-                    }
-                    T xx = fold(xj - rec.p.x, fx, 0);
-                    T yy = fold(yj - rec.p.y, fy, 1);
-                    T zz = fold(zj - rec.p.z, fz, 2);
-                    return xx * xx + yy * yy + zz * zz < rec.p.w;
-                };
-                // slot position of a hit in its target's row: wpos + rank among the slot's hits
-                auto position = [&](uint64_t H, uint32_t wpos) -> uint32_t {
-                    if constexpr (SlotMajor)
-                    {
-                        uint32_t r = __builtin_amdgcn_mbcnt_hi(uint32_t(H >> 32) & nbHi,
-                                                               __builtin_amdgcn_mbcnt_lo(uint32_t(H) & nbLo, 0u));
-                        return wpos + (r << 6);
-                    }
-                    else
-                    {
-                        return __builtin_amdgcn_mbcnt_hi(uint32_t(H >> 32) & nbHi,
-                                                         __builtin_amdgcn_mbcnt_lo(uint32_t(H) & nbLo, wpos));
-                    }
-                };
-                // the slot position after a lane's own pair: pos, plus one slot if the lane's bit of H is set
-                auto advance = [&](uint32_t pos, uint64_t H) -> uint32_t {
-                    if constexpr (SlotMajor) { return pos + (laneIn(H) ? kSlotStep : 0u); }
-                    else { return addLaneBit(pos, H); }
-                };
-                auto iterate = [&](auto checkSelf, auto checkLimit) {
-                    // hits of particle j against a target record, among the lanes of `in`
-                    auto hits = [&](const TargetRec<T>& rec, uint64_t in) -> uint64_t {
-                        uint64_t H = ballot(close(rec)) & in;
-                        if constexpr (decltype(checkSelf)::value) { H &= ballot(jRel != (rec.meta >> 8)); }
-                        return H;
-                    };
-                    // store index of a lane's pair: its row slot for a hit (inside the row), else 2^32 - 1, past the
-                    // record count, where the store is dropped (an inline constant: no register holds it)
-                    auto storeOffset = [&](const TargetRec<T>& rec, uint64_t H, uint32_t pos) -> uint32_t {
-                        if constexpr (decltype(checkLimit)::value)
-                        {
-                            return (laneIn(H) & (pos < rec.limit)) ? pos : ~0u;
-                        }
-                        else { return laneIn(H) ? pos : ~0u; }
-                    };
-                    // the hits' stores: with the row-end check, every lane stores (a miss or a slot past the row end
-                    // at an index past the record count); without it, only the hit lanes store, under their lane
-                    // mask (no per-lane index select)
-                    auto storeHits = [&](const TargetRec<T>& rec, uint64_t H, uint32_t pos)
-                                         __attribute__((always_inline)) {
-                        if constexpr (decltype(checkLimit)::value)
-                        {
-                            structBufferStoreB32(j, rows, int(storeOffset(rec, H, pos)), 0, 0, 0);
-                        }
-                        else
-                        {
-                            if (laneIn(H)) structBufferStoreB32(j, rows, int(pos), 0, 0, 0);
-                        }
-                    };
-                    // slot s of an iteration holds targets k0 + s (A) and k0 + S + s (B). In the iterations with
-                    // k0 + 2S <= pc every slot holds a target (lanes past the last slot test a NaN particle, which
-                    // fails every compare), so no lane mask applies; the last, partial iteration masks the slots
-                    // past pc with wave-uniform masks, and has no B half if pc - k0 <= S. Both records are read
-                    // before either count is written back.
-                    // sameWriteBack: wA == wB (full iterations), both counts are written back under one lane mask
-                    auto body2 = [&](TargetRec<T>* rA, uint64_t inA, uint64_t inB, uint64_t wA, uint64_t wB,
-                                     auto sameWriteBack) __attribute__((always_inline)) {
-                        TargetRec<T>* rB        = rA + S;
-                        const TargetRec<T> recA = *rA;
-                        const TargetRec<T> recB = *rB;
-                        const uint64_t HA       = hits(recA, inA);
-                        const uint64_t HB       = hits(recB, inB);
-                        const uint32_t posA     = position(HA, recA.wpos);
-                        const uint32_t posB     = position(HB, recB.wpos);
-                        storeHits(recA, HA, posA);
-                        storeHits(recB, HB, posB);
-                        if constexpr (decltype(sameWriteBack)::value)
-                        {
-                            if (laneIn(wA))
-                            {
-                                rA->wpos = advance(posA, HA);
-                                rB->wpos = advance(posB, HB);
-                            }
-                        }
-                        else
-                        {
-                            if (laneIn(wA)) rA->wpos = advance(posA, HA);
-                            if (laneIn(wB)) rB->wpos = advance(posB, HB);
-                        }
-                    };
-                    auto body1 = [&](TargetRec<T>* rA, uint64_t inA, uint64_t wA) __attribute__((always_inline)) {
-                        const TargetRec<T> recA = *rA;
-                        const uint64_t HA       = hits(recA, inA);
-                        const uint32_t posA     = position(HA, recA.wpos);
-                        storeHits(recA, HA, posA);
-                        if (laneIn(wA)) rA->wpos = advance(posA, HA);
-                    };
-                    TargetRec<T>* rA = recs + slot; // index < 128: pc <= 64 and slot <= S <= 64
-                    uint32_t left    = pc;
-                    for (; left >= 2 * S; left -= 2 * S, rA += 2 * S)
-                    {
-                        body2(rA, ~uint64_t(0), ~uint64_t(0), lastLanes, lastLanes, std::true_type{});
-                    }
-                    if (left > S)
-                    {
-                        const uint64_t inB = slotsBelow(left - S);
-                        body2(rA, ~uint64_t(0), inB, lastLanes, lastLanes & inB, std::false_type{});
-                    }
-                    else if (left > 0)
-                    {
-                        const uint64_t inA = slotsBelow(left);
-                        body1(rA, inA, lastLanes & inA);
-                    }
-                };
-                if (selfChunk)
-                {
-                    if (noOverflow) iterate(std::true_type{}, std::false_type{});
-                    else iterate(std::true_type{}, std::true_type{});
-                }
-                else
-                {
-                    if (noOverflow) iterate(std::false_type{}, std::false_type{});
-                    else iterate(std::false_type{}, std::true_type{});
-                }
-                waveSync();
-            }
-            if (mine) myWpos = recs[myRank].wpos;
+        // a chunk's candidates and, in the order of the matrix operand's rows, their positions; read one chunk ahead
+        uint32_t nextEntry = 0, nextJ = 0;
+        uint32_t started   = 0; // list entries that start before the chunk's end
+        T nextX = 0, nextY = 0, nextZ = 0;
+        auto fetch = [&](uint32_t at) __attribute__((always_inline)) {
+            // list entry of each position: the entries that start in this chunk mark their first position; a position
+            // belongs to the last entry that starts at or before it
+            const uint32_t start = off - at;
+            sh.marks[lane]       = 0;
             waveSync();
+            if (cnt != 0 && start < uint32_t(kWave)) sh.marks[start] = 1;
+            waveSync();
+            const uint64_t starts = ballot(sh.marks[lane] != 0);
+            nextEntry = __builtin_amdgcn_mbcnt_hi(
+                uint32_t(starts >> 33), __builtin_amdgcn_mbcnt_lo(uint32_t(starts >> 1),
+                                                                  started + (uint32_t(starts) & 1u) - 1u));
+            started += uint32_t(__builtin_popcountll(starts));
+            // positions past the last repeat the last candidate (their hits are masked out)
+            const uint32_t p = min(at + uint32_t(lane), num - 1u);
+            nextJ            = p + uint32_t(__builtin_amdgcn_ds_bpermute(int(nextEntry << 2), int(jb - off)));
+            uint32_t* cand   = sh.cand + slot * kWave;
+            cand[lane]       = nextJ;
+            waveSync();
+            const uint32_t jl = cand[loadPos];
+            if constexpr (std::is_same_v<T, float>)
+            {
+                nextX = structBufferLoadF32(xRes, int(jl), 0, 0, 0);
+                nextY = structBufferLoadF32(yRes, int(jl), 0, 0, 0);
+                nextZ = structBufferLoadF32(zRes, int(jl), 0, 0, 0);
+            }
+            else
+            {
+                nextX = x[jl];
+                nextY = y[jl];
+                nextZ = z[jl];
+            }
+        };
+        if (num != 0) fetch(0);
+        for (uint32_t at = 0;; at += kWave)
+        {
+            const bool more = at < num;
+            if (more)
+            {
+                const uint32_t entry    = nextEntry;
+                const uint32_t j        = nextJ;
+                const T xj = nextX, yj = nextY, zj = nextZ;
+                const uint32_t lastLeaf = started - 1u;
+                const uint32_t group    = candAt + slot * kWave; // of the chunk's first 16 candidates
+                slot                    = slot == uint32_t(kChunks) ? 0u : slot + 1u;
+                if (at + kWave < num) fetch(at + kWave);
+
+                const uint32_t inChunk = num - at < uint32_t(kWave) ? num - at : uint32_t(kWave);
+                const uint64_t present = ~uint64_t(0) >> (kWave - inChunk);
+                // the candidates this lane's target visited, leaf by leaf
+                uint32_t seenLo = 0, seenHi = 0;
+                for (uint32_t e = readLane(entry, 0); e <= lastLeaf; ++e)
+                {
+                    const uint64_t range = ballot(entry == e) & present;
+                    const uint64_t lanes = (uint64_t(readLane(listHi, e)) << 32) | readLane(listLo, e);
+                    orLanes(lanes, range, seenLo, seenHi);
+                }
+                // a target is not its own neighbor
+                const uint64_t own = ballot(j - uint32_t(first) < uint32_t(kWave)) & present;
+                if (own != 0)
+                {
+                    sh.marks[lane] = kWave;
+                    waveSync();
+                    if (laneIn(own)) sh.marks[j - uint32_t(first)] = uint32_t(lane);
+                    waveSync();
+                    const uint32_t self = sh.marks[lane];
+                    if (self < 32u) seenLo &= ~(1u << self);
+                    else if (self < 64u) seenHi &= ~(1u << (self - 32u));
+                }
+                const uint64_t active = ballot((seenLo | seenHi) != 0);
+
+                // D of 4 x 16 candidates and 4 x 16 targets: per 16 targets four products, whose signs are shifted
+                // into one word (bit s of its half: candidate 16 (lane / 16) + s)
+                float cnd[4];
+                T dx = xj - cx, dy = yj - cy, dz = zj - cz;
+                bool outside = false;
+                if constexpr (AnyPbc)
+                {
+                    if (images)
+                    {
+                        const bool bx = box.bnd[0] == HIPCSTONE_PERIODIC, by = box.bnd[1] == HIPCSTONE_PERIODIC,
+                                   bz = box.bnd[2] == HIPCSTONE_PERIODIC;
+                        dx      = fold(dx, bx, 0);
+                        dy      = fold(dy, by, 1);
+                        dz      = fold(dz, bz, 2);
+                        outside = (bx && !(xj >= box.lim[0] && xj <= box.lim[1])) ||
+                                  (by && !(yj >= box.lim[2] && yj <= box.lim[3])) ||
+                                  (bz && !(zj >= box.lim[4] && zj <= box.lim[5]));
+                    }
+                }
+                cnd[0]          = float(dx);
+                cnd[1]          = float(dy);
+                cnd[2]          = float(dz);
+                cnd[3]          = __builtin_fmaf(cnd[2], cnd[2], __builtin_fmaf(cnd[1], cnd[1], cnd[0] * cnd[0]));
+                const bool far  = !(cnd[3] < 1.0e30f); // or not a number
+                transposeRows(cnd);
+                float least = std::numeric_limits<float>::max();
+                auto tile   = [&](uint32_t bits, int t) __attribute__((always_inline)) -> uint32_t {
+                    if ((uint32_t(active >> (16 * t)) & 0xFFFFu) == 0) return bits << 16;
+                    Float4 d[4];
+#pragma unroll
+                    for (int q = 3; q >= 0; --q)
+                        d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(cnd[q], tgt[t], tgtConst[t], 0, 0, 0);
+#pragma unroll
+                    for (int q = 3; q >= 0; --q)
+                    {
+#pragma unroll
+                        for (int r = 3; r >= 0; --r)
+                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[q][r]), 31);
+                        least = fminf(fminf(least, fabsf(d[q][0])), fabsf(d[q][1]));
+                        least = fminf(fminf(least, fabsf(d[q][2])), fabsf(d[q][3]));
+                    }
+                    return bits;
+                };
+                uint32_t b01 = 0, b23 = 0;
+                b01 = tile(b01, 1);
+                b01 = tile(b01, 0);
+                b23 = tile(b23, 3);
+                b23 = tile(b23, 2);
+                // row k of a lane's targets gets its 16 bits from all four rows: candidates [0, 32) and [32, 64)
+                swapHalves(b01, b23);
+                uint32_t o01 = b01, o23 = b23;
+                swapRows(b01, o01);
+                swapRows(b23, o23);
+                uint32_t lo = __builtin_amdgcn_perm(o01, b01, halfSel);
+                uint32_t hw = __builtin_amdgcn_perm(o23, b23, halfSel);
+
+                uint64_t unsure = ballot(least < errBound);
+                if (allExact || ballot(far || outside) != 0) unsure = ~uint64_t(0);
+                if (unsure != 0)
+                {
+                    // the 16-candidate groups with a pair too close to call, in the reference's operations
+                    const T hAgain   = valid ? h[i] : T(0);
+                    const T radiusSq = T(4.0) * hAgain * hAgain;
+#pragma unroll 1
+                    for (int g = 0; g < 4; ++g)
+                    {
+                        if ((uint32_t(unsure >> (16 * g)) & 0xFFFFu) == 0) continue;
+                        uint32_t bits = 0;
+#pragma unroll 1
+                        for (int s = 0; s < 16; ++s)
+                        {
+                            const int from = 16 * (s >> 2) + 4 * g + (s & 3);
+                            bits |= uint32_t(close(readLane(xj, from), readLane(yj, from), readLane(zj, from), radiusSq))
+                                    << s;
+                        }
+                        const uint32_t shift = 16u * (g & 1);
+                        uint32_t& word       = g < 2 ? lo : hw;
+                        word                 = (word & ~(0xFFFFu << shift)) | (bits << shift);
+                    }
+                }
+                lo &= seenLo;
+                hw &= seenHi;
+                total += uint32_t(__builtin_popcount(lo)) + uint32_t(__builtin_popcount(hw));
+                // an entry for each group of 16 with hits: every group's is written, only those with hits stay
+                auto append = [&](uint32_t entry) {
+                    ldsWrite(entryEnd, entry);
+                    entryEnd += uint16_t(entry) != 0 ? HitReader::kEntryStep : 0u;
+                };
+                append((group << 16) | (lo & 0xFFFFu));
+                append(((group + 16u) << 16) | (lo >> 16));
+                append(((group + 32u) << 16) | (hw & 0xFFFFu));
+                append(((group + 48u) << 16) | (hw >> 16));
+                ++numChunks;
+            }
+            // a full set of chunks, or a column without room for another chunk's entries, goes out; at the end the rest
+            const bool full = numChunks == kChunks ||
+                              ballot(entryEnd >= entriesAt + (kEntries - 3) * HitReader::kEntryStep) != 0;
+            if (more ? full : last && numChunks != 0) handOver();
+            if (!more) break;
         }
         listCount = 0;
-    };
-
-    // leaves go to the wave's list (drained before it can overflow: the walk drains it whenever fewer than 9 free
-    // entries are left, and one descent appends at most 8 leaves); the drain reads the list after a wave sync
-    auto appendLeaf = [&](int32_t leafIdx, uint64_t m) {
-        if (lane == 0)
-        {
-            sh.listLeaf[w][listCount] = leafIdx;
-            sh.listMask[w][listCount] = m;
-        }
-        listCount++;
-    };
-
-    // evaluate the 8 children of node range [co, co + 8) for the lanes in `pm`. If every child that some lane
-    // passes is a leaf, those leaves are appended in child order and no frame is pushed (true of most nodes at
-    // the bottom of the tree); otherwise the children's lane masks are pushed as the frame at `depth`. The 48 node
-    // values and the 16 child offsets / leaf indices are loaded up front (contiguous, wave-uniform) and the tests
-    // are branch-free. Returns whether a frame was pushed.
-    auto pushFrame = [&](int depth, int32_t co, const uint64_t* mk, uint32_t passed) {
-        if (lane == 0)
-        {
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-            {
-                sh.mask[w][depth][k] = mk[k];
-            }
-            sh.co[w][depth]  = co;
-            sh.rem[w][depth] = passed;
-        }
         waveSync();
     };
-    auto descend = [&](int depth, int32_t co, uint64_t pm) -> bool {
-        if constexpr (kGroups)
+
+    // ---- the walk's stack, entry e in lane e: a leaf (its complement) or an internal node's child block, and the lanes
+    //      that passed it
+    uint32_t stackLink = 0, stackLo = 0, stackHi = 0;
+    int stackCount = 0, spills = 0;
+    uint32_t fault = 0; // a guard that fires ends the walk: the counts and what was handed on are then incomplete
+    auto push = [&](int32_t link, uint64_t m) __attribute__((always_inline)) {
+        stackLink = writeLane(stackLink, stackCount, uint32_t(link));
+        stackLo   = writeLane(stackLo, stackCount, uint32_t(m));
+        stackHi   = writeLane(stackHi, stackCount, uint32_t(m >> 32));
+        ++stackCount;
+    };
+    auto inTree = [&](int32_t block) { return block > 0 && block <= numNodes - 8; };
+
+    // the 8 children [co, co + 8) of a node that the lanes `pm` passed: leaves that come before every internal child go
+    // to the list, the rest that some lane passes onto the stack, first child on top
+    auto descend = [&](int32_t co, uint64_t pm) __attribute__((always_inline)) {
+        uint64_t mk[8]; // the lanes that pass child k
+        Links8 link;
+        uint32_t flags = 0;
+        if (groups != nullptr && ((co - 1) & 7) == 0)
         {
-            // compact child block: per lane two distance terms per dimension, each child's terms picked with a
-            // bit-field select (v_bfi with a wave-uniform mask); the sums are the per-child nodeDist2 bit for bit
-            if (groups != nullptr && ((co - 1) & 7) == 0)
+            // the whole record with a few wide scalar loads, issued together
+            const ChildGroup<T>* __restrict__ g = groups + (uint32_t(co - 1) >> 3);
+            const Words16 head                  = *reinterpret_cast<const Words16*>(g);
+            link                                = *reinterpret_cast<const Links8*>(g->link);
+            T geo[9];
+            if constexpr (std::is_same_v<T, float>)
             {
-                const ChildGroup* __restrict__ g = groups + ((co - 1) >> 3);
-                // geometry, perm and flags arrive with one 64-byte scalar load
-                const ChildGroupHead hd = *reinterpret_cast<const ChildGroupHead*>(g);
-                const uint32_t flags    = hd[10];
-                if (flags & kGroupValid)
-                {
-                    const uint32_t perm = hd[9];
-                    auto term = [&](uint32_t c, uint32_t s, float p) -> uint32_t {
-                        float d = fmaxf(fabsf(__uint_as_float(c) - p) - __uint_as_float(s), 0.0f);
-                        return __float_as_uint(d * d);
-                    };
-                    const uint32_t ax0 = term(hd[0], hd[6], xi);
-                    const uint32_t ax1 = term(hd[3], hd[6], xi);
-                    const uint32_t ay0 = term(hd[1], hd[7], yi);
-                    const uint32_t ay1 = term(hd[4], hd[7], yi);
-                    const uint32_t az0 = term(hd[2], hd[8], zi);
-                    const uint32_t az1 = term(hd[5], hd[8], zi);
-                    uint64_t mk[8];
+                asm volatile("" ::"s"(link)); // (waits for both loads here, not for one after the other)
 #pragma unroll
-                    for (int k = 0; k < 8; ++k)
-                    {
-                        const float dx = pickBits(sbfeBit(perm, 4 * k + 2), ax1, ax0);
-                        const float dy = pickBits(sbfeBit(perm, 4 * k + 1), ay1, ay0);
-                        const float dz = pickBits(sbfeBit(perm, 4 * k), az1, az0);
-                        mk[k]          = ballot(dx + (dy + dz) < cellR2) & pm;
-                    }
-                    const uint32_t passed = nonzeroBits8(mk);
-                    if ((passed & flags & 0xFFu) == 0)
-                    {
-#pragma unroll
-                        for (int k = 0; k < 8; ++k)
-                        {
-                            if (passed & (1u << k)) appendLeaf(g->leaf[k], mk[k]);
-                        }
-                        return false;
-                    }
-                    pushFrame(depth, co, mk, passed);
-                    return true;
-                }
+                for (int k = 0; k < 9; ++k)
+                    geo[k] = __uint_as_float(head[k]);
+                flags = head[9];
             }
-        }
-        const T* c = centers + size_t(co) * 3;
-        const T* s = sizes + size_t(co) * 3;
-        T cv[24], sv[24];
-        int32_t cc[8], lf[8];
+            else
+            {
+                const Words8 more = *reinterpret_cast<const Words8*>(reinterpret_cast<const char*>(g) + sizeof(head));
+                asm volatile("" ::"s"(link), "s"(more));
 #pragma unroll
-        for (int k = 0; k < 24; ++k)
-        {
-            cv[k] = c[k];
-            sv[k] = s[k];
-        }
+                for (int k = 0; k < 9; ++k)
+                {
+                    const uint32_t lo = k < 8 ? head[2 * k % 16] : more[0];
+                    const uint32_t hw = k < 8 ? head[(2 * k + 1) % 16] : more[1];
+                    geo[k]            = __longlong_as_double((long long)((uint64_t(hw) << 32) | lo));
+                }
+                flags = more[2];
+            }
+            // two distance terms per lane and axis, 8 sums of them: nodeDist2 of the 8 children bit for bit
+            auto term = [&](T c, T half, T p, bool pbc, T len, T ilen) {
+                T d = c - p;
+                if constexpr (AnyPbc) { d = pbc ? d - len * rint(d * ilen) : d; }
+                d = fmax(fabs(d) - half, T(0));
+                return d * d;
+            };
+            const bool zy = flags & kZFaster;
+            const T pa = zy ? zi : yi, pb = zy ? yi : zi;
+            const bool wa = AnyPbc && (zy ? pz : py), wb = AnyPbc && (zy ? py : pz);
+            const T la = zy ? box.len[2] : box.len[1], lb = zy ? box.len[1] : box.len[2];
+            const T ia = zy ? box.ilen[2] : box.ilen[1], ib = zy ? box.ilen[1] : box.ilen[2];
+            const T tx[2] = {term(geo[0], geo[6], xi, px, box.len[0], box.ilen[0]),
+                             term(geo[3], geo[6], xi, px, box.len[0], box.ilen[0])};
+            const T ta[2] = {term(geo[1], geo[7], pa, wa, la, ia), term(geo[4], geo[7], pa, wa, la, ia)};
+            const T tb[2] = {term(geo[2], geo[8], pb, wb, lb, ib), term(geo[5], geo[8], pb, wb, lb, ib)};
+            const T tab[2][2] = {{ta[0] + tb[0], ta[0] + tb[1]}, {ta[1] + tb[0], ta[1] + tb[1]}};
+            auto compare = [&](uint32_t patX, uint32_t patA, uint32_t patB) __attribute__((always_inline)) {
+                T d2[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-        {
-            cc[k] = childOffsets[co + k];
-            lf[k] = internalToLeaf[co + k];
+                for (int k = 0; k < 8; ++k)
+                    d2[k] = tx[(patX >> k) & 1] + tab[(patA >> k) & 1][(patB >> k) & 1];
+                lessIn(pm, d2, cellR2, mk);
+            };
+            if (flags & kXFast) compare(kFast, kMiddle, kSlow);
+            else if (flags & kXMiddle) compare(kMiddle, kFast, kSlow);
+            else compare(kSlow, kFast, kMiddle);
         }
-        uint64_t mk[8];
-        // the ballot of the bare compare is the compare's own lane mask; the parent's lanes are applied as a
-        // scalar AND
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
+        if (!(flags & kGroupValid))
         {
-            T d2  = nodeDist2(cv[3 * k], cv[3 * k + 1], cv[3 * k + 2], sv[3 * k], sv[3 * k + 1], sv[3 * k + 2]);
-            mk[k] = ballot(d2 < cellR2) & pm;
-        }
-        bool allLeaves = true;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-        {
-            allLeaves = allLeaves && (mk[k] == 0 || cc[k] == 0);
-        }
-        if (allLeaves)
-        {
+            // children in no such form: from their own centers and sizes
+            flags = 0;
 #pragma unroll
             for (int k = 0; k < 8; ++k)
             {
-                if (mk[k] != 0) appendLeaf(lf[k], mk[k]);
+                const T* c        = centers + (size_t(co) + k) * 3;
+                const T* sz       = sizes + (size_t(co) + k) * 3;
+                mk[k]             = ballot(nodeDist2(c[0], c[1], c[2], sz[0], sz[1], sz[2]) < cellR2) & pm;
+                const int32_t block = childOffsets[co + k];
+                link[k]           = block != 0 ? block : internalToLeaf[co + k];
+                if (block == 0) continue;
+                flags |= 1u << k;
+                if (!inTree(block)) flags |= kGroupOutside;
+                if (block <= co + k) flags |= kGroupBackward;
             }
-            return false;
         }
-        pushFrame(depth, co, mk, nonzeroBits8(mk));
-        return true;
+        if (flags & (Segmented ? kGroupOutside : kGroupOutside | kGroupBackward))
+        {
+            fault = HIPCSTONE_FAULT_MALFORMED_TREE;
+            return;
+        }
+        bool inner = false; // met an internal child
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            if (inner || mk[k] == 0) continue;
+            if (flags & (1u << k)) { inner = true; }
+            else
+            {
+                appendLeaf(link[k], mk[k]);
+                mk[k] = 0;
+            }
+        }
+        if (!inner) return;
+#pragma unroll
+        for (int k = 7; k >= 0; --k)
+        {
+            if (mk[k] != 0) push(flags & (1u << k) ? link[k] : ~link[k], mk[k]);
+        }
     };
 
     // root (traversal.hpp:35-45)
-    const T* rc       = centers + size_t(root) * 3;
-    const T* rsz      = sizes + size_t(root) * 3;
-    uint64_t rootMask = ballot(valid & (nodeDist2(rc[0], rc[1], rc[2], rsz[0], rsz[1], rsz[2]) < cellR2));
-    if (rootMask != 0)
+    const int32_t rootChild = uniform(childOffsets[root]);
+    if (rootChild == 0) { appendLeaf(uniform(internalToLeaf[root]), rootMask); }
+    else if (!inTree(rootChild)) { fault = HIPCSTONE_FAULT_MALFORMED_TREE; }
+    else { push(rootChild, rootMask); }
+    // a 32-bit budget (saturated) of nodes taken from the stack, so that the test is a scalar compare
+    const uint64_t budget = 2 * uint64_t(uint32_t(numNodes)) + 8;
+    uint32_t stepsLeft    = budget > 0xFFFFFFFFu ? 0xFFFFFFFFu : uint32_t(budget);
+    while (true)
     {
-        int32_t rootChild = uniform(childOffsets[root]);
-        // a guard that fires (out-of-range node, stack overflow, step budget) ends the walk and sets its bit in
-        // the fault word: the wave's rows and counts are then incomplete
-        uint32_t fault = 0;
-        if (rootChild == 0) { appendLeaf(uniform(internalToLeaf[root]), rootMask); }
-        else if (rootChild < 0 || rootChild + 8 > numNodes) { fault = HIPCSTONE_FAULT_MALFORMED_TREE; }
-        else
+        bool done = fault != 0;
+        if (stackCount == 0)
         {
-            int depth         = descend(0, rootChild, rootMask) ? 0 : -1;
-            // a 32-bit budget (saturated), so that the per-step test is a scalar compare
-            const uint64_t budget = 2 * uint64_t(uint32_t(numNodes)) + 8;
-            uint32_t stepsLeft    = budget > 0xFFFFFFFFu ? 0xFFFFFFFFu : uint32_t(budget);
-            while (depth >= 0)
+            if (spills == 0) { done = true; }
+            else
             {
-                if (stepsLeft-- == 0)
+                // (lanes from kSpillEntries on keep what they have: the count says which entries are live)
+                --spills;
+                if (lane < kSpillEntries)
                 {
-                    fault = HIPCSTONE_FAULT_WALK_BUDGET;
-                    break;
+                    stackLink = sh.spilled[spills][0][lane];
+                    stackLo   = sh.spilled[spills][1][lane];
+                    stackHi   = sh.spilled[spills][2][lane];
                 }
-                if (listCount > kLeafList - 9) drain();
-                // the frame's next child with lanes: the lowest bit of its remaining-children word
-                const uint32_t rem = uniform(sh.rem[w][depth]);
-                if (rem == 0)
-                {
-                    --depth;
-                    continue;
-                }
-                const int k        = __builtin_ctz(rem);
-                const uint64_t m   = uniform64(sh.mask[w][depth][k]);
-                int32_t node       = uniform(sh.co[w][depth]) + k;
-                if (lane == 0) sh.rem[w][depth] = rem & (rem - 1);
-                waveSync();
-                if (node <= 0 || node >= numNodes)
-                {
-                    fault = HIPCSTONE_FAULT_MALFORMED_TREE;
-                    break;
-                }
-                int32_t cco = uniform(childOffsets[node]);
-                if (cco == 0) { appendLeaf(uniform(internalToLeaf[node]), m); }
-                else
-                {
-                    if (depth + 1 >= kMaxDepth || (!Segmented && cco <= node) || cco <= 0 || cco + 8 > numNodes)
-                    {
-                        fault = HIPCSTONE_FAULT_MALFORMED_TREE;
-                        break;
-                    }
-                    if (descend(depth + 1, cco, m)) ++depth;
-                }
+                stackCount = kSpillEntries;
             }
         }
-        if (fault != 0 && lane == 0) atomicOr(faults, fault);
-        drain();
+        if (done || listCount > kLeafList - 9)
+        {
+            drain(done);
+            if (done) break;
+        }
+        --stackCount;
+        const int32_t link = int32_t(readLane(stackLink, stackCount));
+        const uint64_t m   = (uint64_t(readLane(stackHi, stackCount)) << 32) | readLane(stackLo, stackCount);
+        if (link < 0)
+        {
+            appendLeaf(~link, m);
+            continue;
+        }
+        if (stepsLeft == 0) fault = HIPCSTONE_FAULT_WALK_BUDGET;
+        --stepsLeft;
+        if (stackCount > kWave - 8)
+        {
+            if (spills == kSpills) { fault = HIPCSTONE_FAULT_MALFORMED_TREE; }
+            else
+            {
+                if (lane < kSpillEntries)
+                {
+                    sh.spilled[spills][0][lane] = stackLink;
+                    sh.spilled[spills][1][lane] = stackLo;
+                    sh.spilled[spills][2][lane] = stackHi;
+                }
+                waveSync();
+                ++spills;
+                const int from = ((lane + kSpillEntries) & (kWave - 1)) << 2;
+                stackLink      = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(stackLink)));
+                stackLo        = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(stackLo)));
+                stackHi        = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(stackHi)));
+                stackCount -= kSpillEntries;
+            }
+        }
+        if (link == 0) fault = HIPCSTONE_FAULT_MALFORMED_TREE;
+        if (fault == 0) descend(link, m);
     }
-    return SlotMajor ? (myWpos - rowOff) >> 6 : myWpos - rowOff;
+    if (fault != 0 && lane == 0) atomicOr(faults, fault);
+    return total;
 }
 
 } // namespace nbwalk

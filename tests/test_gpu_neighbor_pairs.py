@@ -1,0 +1,168 @@
+"""The pair test of the neighbor search where it can go wrong, bit for bit against the oracle (no tolerance): pairs on
+and next to the search radius, where the matrix-core distance cannot decide and the reference's own operations must;
+magnitudes outside fp32's normal range and values that are not numbers; chunks and waves that are not full; leaves
+larger than a chunk and leaves without particles; more leaves in flight than the walk's registers hold; and periodic
+images, including search radii near half the box."""
+
+import numpy as np
+import pytest
+
+from helpers import cpu_pipeline, neighbor_rows_equal
+from oracle_py import HILBERT
+from oracle_py import make_box as orc_box
+
+pytestmark = pytest.mark.gpu
+
+TS = [np.float32, np.float64]
+
+
+def _search(hip, p, gbox, first, last, ngmax, ext=1.0):
+    dev = lambda a: hip.DeviceArray.from_numpy(np.ascontiguousarray(a))
+    d = {k: dev(p[k]) for k in ("x", "y", "z", "h", "childOffsets", "parents", "internalToLeaf", "layout")}
+    c, s = dev(p["centers"].reshape(-1)), dev(p["sizes"].reshape(-1))
+    n = last - first
+    nb, nc = hip.DeviceArray(max(1, n * ngmax), np.uint32), hip.DeviceArray(n, np.uint32)
+    hip.find_neighbors(d["x"], d["y"], d["z"], d["h"], first, last, gbox, d["childOffsets"], d["parents"],
+                       d["internalToLeaf"], d["layout"], c, s, p["prefixes"].size, ngmax, nb if ngmax else None, nc,
+                       ext)
+    return nb.download(n * ngmax).reshape(n, ngmax), nc.download()
+
+
+def _check(hip, oracle, p, lo, hi, ngmax, first=0, last=None, boundary=(0, 0, 0), ext=1.0):
+    T = p["x"].dtype.type
+    last = p["x"].size if last is None else last
+    gbox, obox = hip.make_box(lo, hi, T, boundary), orc_box(lo, hi, T, boundary)
+    tree = {k: p[k] for k in ("childOffsets", "parents", "internalToLeaf")}
+    rnb, rnc = oracle.find_neighbors(p["x"], p["y"], p["z"], p["h"], first, last, obox, tree, p["layout"],
+                                     p["centers"], p["sizes"], ngmax, ext)
+    nb, nc = _search(hip, p, gbox, first, last, ngmax, ext)
+    assert np.array_equal(nc, rnc)
+    assert neighbor_rows_equal(nb, nc, rnb, rnc, ngmax)
+    return rnc
+
+
+def _tree(oracle, x, y, z, h, lo, hi, bucket, kd=np.uint64, boundary=(0, 0, 0)):
+    return cpu_pipeline(oracle, x, y, z, h, orc_box(lo, hi, x.dtype.type, boundary), kd, bucket, HILBERT)
+
+
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("boundary", [(0, 0, 0), (1, 1, 1)])
+def test_pairs_on_the_search_radius(hip, oracle, T, boundary):
+    """A lattice of spacing 1/16 whose radius 2h is exactly 2 or sqrt(5) spacings, one ulp to either side included:
+    every particle has many pairs whose squared distance is the squared radius or its neighbor in floating point."""
+    k = np.arange(4096)
+    x, y, z = ((v.astype(T) + T(0.5)) / T(16) for v in (k % 16, k // 16 % 16, k // 256))
+    rng = np.random.default_rng(11)
+    r = np.where(rng.random(k.size) < 0.5, T(2) / T(16), np.sqrt(T(5)) / T(16)).astype(T)
+    r = np.where(rng.random(k.size) < 0.3, np.nextafter(r, T(1)), r)
+    r = np.where(rng.random(k.size) < 0.3, np.nextafter(r, T(0)), r)
+    p = _tree(oracle, x, y, z, (r / T(2)).astype(T), 0.0, 1.0, 16, boundary=boundary)
+    counts = _check(hip, oracle, p, 0.0, 1.0, 64, boundary=boundary)
+    assert len(np.unique(counts)) > 2
+
+
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129, 1000, 32767, 32769, 65599])
+def test_partial_waves(hip, oracle, T, n):
+    """Sizes around the waves' 16, 32 and 64 targets and around the counts where the targets per wave change."""
+    rng = np.random.default_rng(n)
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    h = np.full(n, 0.5 * (30 / (4.19 * max(n, 8))) ** (1 / 3), T) * (T(0.5) + rng.random(n).astype(T))
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 32)
+    _check(hip, oracle, p, 0.0, 1.0, 24)
+    if n > 64:
+        _check(hip, oracle, p, 0.0, 1.0, 40, first=n // 3, last=n - 5)
+
+
+@pytest.mark.parametrize("T", TS)
+def test_large_and_empty_leaves(hip, oracle, T):
+    """1500 particles in one deepest leaf of 32-bit keys (more than 20 chunks of 64), 70 exactly coincident ones, and a
+    sparse rest with many empty leaves; rows longer and shorter than the counts."""
+    rng = np.random.default_rng(3)
+    n = 4000
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    x[:1500], y[:1500], z[:1500] = (T(0.300001) + rng.random((3, 1500)).astype(T) * T(2e-4))
+    x[1500:1570], y[1500:1570], z[1500:1570] = T(0.7), T(0.7), T(0.7)
+    h = np.full(n, 0.03, T)
+    h[:700] = T(3e-5)
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 8, kd=np.uint32)
+    assert p["counts"].max() > 600 and (p["counts"] == 0).sum() > 20
+    for ngmax in (7, 2000):
+        _check(hip, oracle, p, 0.0, 1.0, ngmax)
+
+
+@pytest.mark.parametrize("T", TS)
+def test_deep_tree_with_everything_in_reach(hip, oracle, T):
+    """Particles around the origin corner at every scale down to the deepest level: each node on the way down leaves its
+    seven other children behind, more entries than the walk's stack registers hold, and every target reaches all of
+    them."""
+    rng = np.random.default_rng(5)
+    pts = []
+    for level in range(1, 20):
+        s = 2.0**-level
+        for o in range(1, 8):
+            corner = np.array([o >> 2, (o >> 1) & 1, o & 1]) * s
+            pts.append(corner + rng.random((3, 3)) * s)
+    pts.append(rng.random((12, 3)) * 2.0**-19)
+    pts = np.concatenate(pts)
+    x, y, z = (np.ascontiguousarray(pts[:, d]).astype(T) for d in range(3))
+    h = np.where(rng.random(x.size) < 0.5, 1.0, 0.01).astype(T)
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 8)
+    assert p["levelRange"].size > 20 and _check(hip, oracle, p, 0.0, 1.0, 450).max() == x.size - 1
+
+
+@pytest.mark.parametrize("T,scale", [(np.float32, 1e-17), (np.float32, 1e-12), (np.float32, 1e12), (np.float32, 3e18),
+                                     (np.float64, 1e-40), (np.float64, 1e-12), (np.float64, 1e12), (np.float64, 1e40)])
+def test_magnitudes(hip, oracle, T, scale):
+    """Coordinates and radii whose squares leave fp32's range, or come near its ends, and a box far from the origin."""
+    rng = np.random.default_rng(9)
+    n = 3000
+    x, y, z = ((rng.random(n) * scale).astype(T) for _ in range(3))
+    h = ((0.4 + 0.4 * rng.random(n)) * 0.1 * scale).astype(T)
+    p = _tree(oracle, x, y, z, h, 0.0, scale, 16)
+    assert _check(hip, oracle, p, 0.0, scale, 200).mean() > 10
+    x, y, z = ((v + T(64 * scale)).astype(T) for v in (x, y, z))
+    p = _tree(oracle, x, y, z, h, 64 * scale, 65 * scale, 16)
+    _check(hip, oracle, p, 64 * scale, 65 * scale, 200)
+
+
+@pytest.mark.parametrize("T", TS)
+def test_values_that_are_not_ordinary_numbers(hip, oracle, T):
+    """Zero, infinite and not-a-number radii, and particles whose coordinates are not numbers, infinite or far away (in
+    the search's own arrays; the tree is that of the ordinary particles)."""
+    rng = np.random.default_rng(13)
+    n = 5000
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    h = np.full(n, 0.05, T)
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 32)
+    pick = rng.choice(n, 40, replace=False)
+    p["h"][pick[:4]] = 0
+    p["h"][pick[4:8]] = np.nan
+    p["h"][pick[8:10]] = np.inf
+    p["h"][pick[10:12]] = -0.04
+    p["x"][pick[12:16]] = np.nan
+    p["y"][pick[16:20]] = np.inf
+    p["z"][pick[20:24]] = -np.inf
+    p["x"][pick[24:28]] = T(1e16)
+    p["y"][pick[28:32]] = T(3e38)
+    with np.errstate(all="ignore"):
+        _check(hip, oracle, p, 0.0, 1.0, 128)
+
+
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("radius", [0.04, 0.12, 0.24, 0.3, 0.6])
+@pytest.mark.parametrize("boundary", [(1, 1, 1), (0, 1, 0)])
+def test_periodic_radii(hip, oracle, T, radius, boundary):
+    """Search radii from a small part of the box to more than half of it, particles on the faces, and some outside the
+    domain; a leaf extension as well."""
+    rng = np.random.default_rng(int(radius * 100))
+    n = 3000
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    x[:50], y[50:100], z[100:150] = T(0), T(0), np.nextafter(T(1), T(0))
+    h = ((0.8 + 0.4 * rng.random(n)) * radius / 2).astype(T)
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 32, boundary=boundary)
+    _check(hip, oracle, p, 0.0, 1.0, 150, boundary=boundary)
+    out = rng.choice(n, 20, replace=False)
+    p["x"][out[:10]] -= T(0.02)
+    p["y"][out[10:]] += T(1.03)
+    _check(hip, oracle, p, 0.0, 1.0, 150, boundary=boundary, ext=1.1)
