@@ -35,26 +35,42 @@ namespace hipcstone
 namespace serve
 {
 
-// order-independent digest: the wrapping sum over particles of a hash of (i, key, count, stored neighbors)
-__global__ __launch_bounds__(256) void digestKernel(const uint64_t* __restrict__ keys,
+// order-independent digest: the wrapping sum over particles of a hash of (i, key, count, stored neighbors). 16 lanes share
+// a particle's row and read consecutive slots (with a thread per row every load touched 64 rows), and a workgroup adds
+// its sum once: the additions to one word, a chain of about 10 ns each, bound what is left.
+// Mean over clouds of 10k to 150k particles, four on the device at once, ngmax 128: 183 -> 86 us.
+constexpr int kDigestLanes   = 16;
+constexpr int kDigestThreads = 512;
+constexpr int kDigestBlocks  = 512;
+
+__global__ __launch_bounds__(kDigestThreads) void digestKernel(const uint64_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ counts,
                                                      const uint32_t* __restrict__ nb, size_t n, uint32_t ngmax,
                                                      unsigned long long* __restrict__ out)
 {
     unsigned long long acc = 0;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
+    const uint32_t sub     = threadIdx.x % kDigestLanes;
+    const size_t rows      = size_t(gridDim.x) * (blockDim.x / kDigestLanes);
+    for (size_t i = (size_t(blockIdx.x) * blockDim.x + threadIdx.x) / kDigestLanes; i < n; i += rows)
     {
-        uint32_t c = counts[i];
-        uint64_t d = mix64(uint64_t(i) * 0x9E3779B97F4A7C15ull ^ keys[i]) + mix64((uint64_t(i) << 32) | c);
-        uint32_t m = c < ngmax ? c : ngmax;
-        for (uint32_t k = 0; k < m; ++k)
-            d += mix64((uint64_t(nb[i * size_t(ngmax) + k]) << 20) ^ (uint64_t(k) << 52) ^ uint64_t(i));
-        acc += d;
+        const uint32_t c = counts[i];
+        if (sub == 0) acc += mix64(uint64_t(i) * 0x9E3779B97F4A7C15ull ^ keys[i]) + mix64((uint64_t(i) << 32) | c);
+        const uint32_t m    = c < ngmax ? c : ngmax;
+        const uint32_t* row = nb + i * size_t(ngmax);
+        for (uint32_t k = sub; k < m; k += kDigestLanes)
+            acc += mix64((uint64_t(row[k]) << 20) ^ (uint64_t(k) << 52) ^ uint64_t(i));
     }
-    // wave sum, then one atomic per wave
     for (int off = 32; off > 0; off >>= 1)
         acc += __shfl_down(acc, off, kWave);
-    if (laneId() == 0) atomicAdd(out, acc);
+    __shared__ unsigned long long sums[kDigestThreads / kWave];
+    if (laneId() == 0) sums[threadIdx.x / kWave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        for (int w = 1; w < kDigestThreads / kWave; ++w)
+            acc += sums[w];
+        atomicAdd(out, acc);
+    }
 }
 
 __global__ void zeroU64Kernel(unsigned long long* p) { *p = 0; }
@@ -394,7 +410,8 @@ private:
         {
             auto* d = digest.as<unsigned long long>();
             zeroU64Kernel<<<1, 1, 0, s>>>(d);
-            digestKernel<<<std::max<unsigned>(1, std::min<unsigned>(1024, ceilDiv(n, 256))), 256, 0, s>>>(
+            digestKernel<<<std::max<unsigned>(1, std::min<unsigned>(kDigestBlocks, ceilDiv(n * kDigestLanes, kDigestThreads))),
+                           kDigestThreads, 0, s>>>(
                 static_cast<const uint64_t*>(v.keys), c.nc.as<uint32_t>(), c.nb.as<uint32_t>(), n, cfg_.ngmax, d);
             HC_CHECK_LAUNCH("digestKernel");
             unsigned long long h = 0;
