@@ -760,11 +760,9 @@ private:
                 if (auto e = nb.reserve(nOutMax * sizeof(SplitNode))) return e;
                 swap(nb, frontier_[1 - cur]);
             }
-            if (leaves + nOutMax > splitKeys_.bytes / sizeof(K))
-            {
-                if (auto e = growKeep(splitKeys_, (leaves + nOutMax) * sizeof(K), leaves * sizeof(K), st)) return e;
-                if (auto e = growKeep(splitCounts_, (leaves + nOutMax) * sizeof(uint32_t), leaves * 4, st)) return e;
-            }
+            // (each by its own size: the two grow by different amounts)
+            if (auto e = growKeep(splitKeys_, (leaves + nOutMax) * sizeof(K), leaves * sizeof(K), st)) return e;
+            if (auto e = growKeep(splitCounts_, (leaves + nOutMax) * sizeof(uint32_t), leaves * 4, st)) return e;
             setPairKernel<<<1, 1, 0, st>>>(splitCounters_.as<uint32_t>(), 0u, leaves);
             HC_CHECK_LAUNCH("setPairKernel");
             splitLevelKernel<<<ceilDiv(nOutMax, 256), 256, 0, st>>>(
