@@ -15,26 +15,27 @@ struct DeviceBuf
 {
     void* ptr    = nullptr;
     size_t bytes = 0;
+    bool pooled  = false; // from the pool (PoolScope)
     DeviceBuf()  = default;
     DeviceBuf(const DeviceBuf&)            = delete;
     DeviceBuf& operator=(const DeviceBuf&) = delete;
     ~DeviceBuf()
     {
-        if (ptr) (void)hipFree(ptr);
+        (void)release();
     }
     friend void swap(DeviceBuf& a, DeviceBuf& b) noexcept
     {
         std::swap(a.ptr, b.ptr);
         std::swap(a.bytes, b.bytes);
+        std::swap(a.pooled, b.pooled);
     }
     hipcstone_status reserve(size_t b)
     {
         if (b <= bytes) return HIPCSTONE_OK;
-        if (ptr) HC_CHECK(hipFree(ptr));
-        ptr   = nullptr;
-        bytes = 0;
+        HC_CHECK(release());
         size_t grown = b + b / 8 + 256;
-        hipError_t e = hipMalloc(&ptr, grown);
+        pooled       = poolScope() != nullptr;
+        hipError_t e = pooled ? poolTake(&ptr, grown) : deviceMalloc(&ptr, grown);
         if (e != hipSuccess)
         {
             ptr = nullptr;
@@ -48,6 +49,19 @@ struct DeviceBuf
     V* as() const
     {
         return static_cast<V*>(ptr);
+    }
+
+private:
+    hipError_t release()
+    {
+        hipError_t e = hipSuccess;
+        if (!ptr) return e;
+        if (!pooled) e = hipFree(ptr);
+        else if (poolScope()) poolScope()->freed.push_back(ptr);
+        else poolGive(ptr, false);
+        ptr   = nullptr;
+        bytes = 0;
+        return e;
     }
 };
 

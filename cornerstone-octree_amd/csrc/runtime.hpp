@@ -5,6 +5,7 @@
 
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "hipcstone.h"
 
@@ -41,6 +42,36 @@ hipcstone_status checkFaults(uint32_t faults);
 // orchestration objects' fault-word copy.
 constexpr int kPinnedWords = 64;
 uint32_t* pinnedStaging();
+// Device memory that is kept for the next taker instead of given back to the driver: an allocation of 64 MB and more takes
+// 0.3 ms, several where other processes use the device, and hipFree waits for everything that runs on it. Blocks are
+// returned only when no work on any stream uses them any more, so any stream may use them next. At most kPoolBytes per
+// device are kept (the oldest go first); an allocation of this library that fails gives them all back and tries again,
+// and so does poolTrim(). Safe from several threads.
+constexpr size_t kPoolBytes = size_t(1) << 30;
+hipError_t poolTake(void** ptr, size_t bytes); // of the current device
+void poolGive(void* ptr, bool idle = true);    // a block of poolTake; not idle: freed
+void poolTrim();
+// hipMalloc, and once more after poolTrim() if it fails
+hipError_t deviceMalloc(void** ptr, size_t bytes);
+// streams likewise (default priority, idle when returned, at most kPoolStreams kept per device)
+constexpr size_t kPoolStreams = 16;
+hipError_t poolTakeStream(hipStream_t* s);
+void poolGiveStream(hipStream_t s);
+
+// While a thread has one, its DeviceBuf take their memory from the pool and leave it in `freed` instead of freeing it;
+// flush() hands those blocks back. Call it when the device is done with all that the thread enqueued before.
+struct PoolScope
+{
+    PoolScope();
+    ~PoolScope();
+    PoolScope(const PoolScope&)            = delete;
+    PoolScope& operator=(const PoolScope&) = delete;
+    void flush(bool idle = true);
+    std::vector<void*> freed;
+    PoolScope* outer;
+};
+PoolScope* poolScope(); // of this thread, or nullptr
+
 // the radix sort's look-back poll limit (hipcstone_set_sort_lookback_limit)
 uint32_t sortLookbackLimit();
 // waves per workgroup of the neighbor search (hipcstone_set_neighbor_waves): 2, 4 or 8

@@ -134,7 +134,9 @@ public:
         }
         int dev = 0;
         HC_CHECK(hipGetDevice(&dev));
-        HC_CHECK(hipStreamCreate(&dispatchStream_));
+        HC_CHECK(poolTakeStream(&dispatchStream_));
+        // (this thread frees clouds only when nothing of theirs is in flight)
+        PoolScope scope;
         start_ = Clock::now();
         std::vector<std::thread> workers;
         for (int w = 0; w < cfg_.slots; ++w)
@@ -151,7 +153,8 @@ public:
         for (auto& kv : clouds_)
             if (kv.second.pipe) hipcstone_pipeline_destroy(kv.second.pipe);
         clouds_.clear();
-        (void)hipStreamDestroy(dispatchStream_);
+        scope.flush();
+        poolGiveStream(dispatchStream_);
         if (firstError_ != HIPCSTONE_OK) setError(firstErrorText_);
         return firstError_;
     }
@@ -209,6 +212,7 @@ private:
                 swap(a, victim->nb);
                 swap(b, victim->nc);
             }
+            poolScope()->flush();
             used_ -= victim->bytes;
             victim->bytes    = 0;
             victim->resident = false;
@@ -301,11 +305,12 @@ private:
     {
         (void)hipSetDevice(dev);
         hipStream_t s = nullptr;
-        if (hipStreamCreate(&s) != hipSuccess)
+        if (poolTakeStream(&s) != hipSuccess)
         {
             fail(HIPCSTONE_HIP_ERROR, "serve: hipStreamCreate failed");
             return;
         }
+        PoolScope scope;
         DeviceBuf digest;
         (void)digest.reserve(64);
         while (true)
@@ -328,6 +333,8 @@ private:
                 c = &clouds_[q.cloud];
             }
             hipcstone_status st = execute(job, q, *c, s, digest, out);
+            // a request that succeeded has synchronized the stream
+            scope.flush(st == HIPCSTONE_OK || hipStreamSynchronize(s) == hipSuccess);
             double end          = now();
             size_t actual       = c->pipe ? hipcstone_pipeline_device_bytes(c->pipe) + c->nb.bytes + c->nc.bytes : 0;
             {
@@ -348,7 +355,12 @@ private:
             }
             cvDone_.notify_all();
         }
-        (void)hipStreamDestroy(s);
+        {
+            DeviceBuf d;
+            swap(d, digest);
+        }
+        scope.flush();
+        poolGiveStream(s);
     }
 
     hipcstone_status execute(const Job& job, const hipcstone_serve_request& q, Cloud& c, hipStream_t s,
@@ -366,6 +378,7 @@ private:
                 return invalid("serve: a build needs its particles");
             if (c.pipe) hipcstone_pipeline_destroy(c.pipe);
             c.pipe = nullptr;
+            poolScope()->flush(); // (the stream and the cloud are idle when a request begins)
             if (auto e = hipcstone_pipeline_create(&c.pipe, cfg_.curve, 64, 32, cfg_.bucket_size, cfg_.ngmax)) return e;
             DeviceBuf in[4];
             const float* src[4] = {q.x, q.y, q.z, q.h};

@@ -105,6 +105,12 @@ const char* hipcstone_build_info(void);
 
 hipcstone_status hipcstone_device_alloc(void** ptr, size_t bytes);
 hipcstone_status hipcstone_device_free(void* ptr);
+/* Scratch memory of one call: like device_alloc / device_free, but a block is kept for the next taker (at most 1 GiB per
+ * device; given back when an allocation of this library fails, or by scratch_trim). Return a block only when the device
+ * has finished all work that uses it. */
+hipcstone_status hipcstone_scratch_alloc(void** ptr, size_t bytes);
+hipcstone_status hipcstone_scratch_free(void* ptr);
+hipcstone_status hipcstone_scratch_trim(void);
 hipcstone_status hipcstone_memcpy_h2d(void* dst, const void* src, size_t bytes, hipcstone_stream s);
 hipcstone_status hipcstone_memcpy_d2h(void* dst, const void* src, size_t bytes, hipcstone_stream s);
 hipcstone_status hipcstone_memcpy_d2d(void* dst, const void* src, size_t bytes, hipcstone_stream s);
