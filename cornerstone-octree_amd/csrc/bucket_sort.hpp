@@ -136,12 +136,17 @@ constexpr uint32_t kHintLeaves = 16;
 // hint[g] = the leaf of the previous layout that holds position 64 g (the previous step's leaf of the particle that
 // now sits first in wave g): one thread per leaf writes the waves whose first position falls in it. layout[0..L] is
 // the previous leaf layout of exactly n particles.
+// Also clears the buckets' counts and the largest one (layout may be null: then only that).
 template<int Unused = 0>
 __global__ __launch_bounds__(256) void waveLeafHintKernel(const uint32_t* __restrict__ layout, int32_t L, uint32_t n,
-                                                          uint32_t* __restrict__ hint)
+                                                          uint32_t* __restrict__ hint, uint32_t* __restrict__ segCount,
+                                                          uint32_t* __restrict__ maxBucket)
 {
     const uint32_t l = blockIdx.x * 256u + threadIdx.x;
     if (l >= uint32_t(L)) return;
+    segCount[l] = 0u;
+    if (l == 0) *maxBucket = 0u;
+    if (!layout) return;
     const uint32_t a = layout[l], b = layout[l + 1];
     for (uint32_t g = (a + 63u) / 64u; 64u * g < b && 64u * g < n; ++g)
         hint[g] = l;
@@ -277,13 +282,6 @@ __global__ __launch_bounds__(256) void maxBucketKernel(const uint32_t* __restric
         const uint32_t b = std::max(std::max(sh[0], sh[1]), std::max(sh[2], sh[3]));
         if (b > *out) atomicMax(out, b); // the pre-check skips most atomics
     }
-}
-
-template<int Unused = 0>
-__global__ void zeroU32Kernel(uint32_t* p, uint32_t n)
-{
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i < n) p[i] = 0u;
 }
 
 template<class K>
@@ -537,10 +535,6 @@ hipcstone_status sortByLeafBuckets(hipcstone_stream s, K* keys, size_t n, const 
 
     uint32_t* maxBucket = idx + n;
 
-    zeroU32Kernel<<<ceilDiv(size_t(L), 256), 256, 0, st>>>(segCount, uint32_t(L));
-    HC_CHECK_LAUNCH("zeroU32Kernel");
-    zeroU32Kernel<<<1, 256, 0, st>>>(maxBucket, 1u);
-    HC_CHECK_LAUNCH("zeroU32Kernel");
     // the previous layout (of the same particle count, in the order the keys come in) gives each wave a leaf to
     // start from
     uint32_t* hint = nullptr;
@@ -548,14 +542,18 @@ hipcstone_status sortByLeafBuckets(hipcstone_stream s, K* keys, size_t n, const 
     {
         if (auto e = hintWs->reserve(size_t(ceilDiv(n, 64)) * sizeof(uint32_t))) return e;
         hint = hintWs->as<uint32_t>();
-        waveLeafHintKernel<<<ceilDiv(size_t(L), 256), 256, 0, st>>>(prevLayout, L, n32, hint);
-        HC_CHECK_LAUNCH("waveLeafHintKernel");
     }
+    waveLeafHintKernel<<<ceilDiv(size_t(L), 256), 256, 0, st>>>(hint ? prevLayout : nullptr, L, n32, hint, segCount,
+                                                                maxBucket);
+    HC_CHECK_LAUNCH("waveLeafHintKernel");
     bucketByLeafKernel<K><<<ceilDiv(n, 256), 256, 0, st>>>(keys, n32, leaves, L, segCount, bucketBuf, slot, hint);
     HC_CHECK_LAUNCH("bucketByLeafKernel");
     maxBucketKernel<<<ceilDiv(size_t(L), kMaxPerBlock), 256, 0, st>>>(segCount, uint32_t(L), maxBucket);
     HC_CHECK_LAUNCH("maxBucketKernel");
-    if (maxOut && deferMax) { HC_CHECK(hipMemcpyAsync(maxOut, maxBucket, sizeof(uint32_t), hipMemcpyDeviceToHost, st)); }
+    if (maxOut && deferMax)
+    {
+        if (auto e = enqueueWordRead(st, maxBucket, maxOut)) return e;
+    }
     else
     {
         uint32_t largest = 0;

@@ -125,9 +125,14 @@ __global__ __launch_bounds__(256) void rebalanceKernel(const K* __restrict__ tre
 }
 
 __global__ void setIntKernel(int* p, int v) { *p = v; }
-__global__ void copyI32Kernel(const int32_t* src, int32_t* dst) { *dst = *src; }
+// the flag and the new node count, side by side in pinned host memory
+__global__ void readNodeOpsKernel(const int* flag, const int32_t* newNumNodes, uint32_t* host)
+{
+    host[0] = uint32_t(*flag);
+    host[1] = uint32_t(*newNumNodes);
+}
 
-// workspace: [flag int, new node count int (256 B)][scan partials]
+// workspace: [flag int (256 B)][scan partials]
 static size_t nodeOpsWorkspace(int32_t numNodes) { return 256 + scan::workspaceBytes(size_t(numNodes) + 1); }
 
 template<class K>
@@ -162,12 +167,10 @@ static hipcstone_status computeNodeOps(hipcstone_stream s, const K* tree, int32_
     if (auto e = scan::exclusiveScan<int32_t>(st, nodeOps, nodeOps, size_t(numNodes) + 1, 0, nullptr, scanWs,
                                               wsBytes - 256))
         return e;
-    // the flag and the new node count side by side, read back with one copy into pinned memory
-    copyI32Kernel<<<1, 1, 0, st>>>(nodeOps + numNodes, reinterpret_cast<int32_t*>(flag) + 1);
-    HC_CHECK_LAUNCH("copyI32Kernel");
     uint32_t* pin = pinnedStaging();
     if (!pin) return HIPCSTONE_HIP_ERROR;
-    HC_CHECK(hipMemcpyAsync(pin, flag, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    readNodeOpsKernel<<<1, 1, 0, st>>>(flag, nodeOps + numNodes, pin);
+    HC_CHECK_LAUNCH("readNodeOpsKernel");
     HC_CHECK(hipStreamSynchronize(st));
     if (newNumNodes) *newNumNodes = int32_t(pin[1]);
     if (converged) *converged = int(pin[0]);
@@ -185,43 +188,50 @@ static hipcstone_status rebalanceTree(hipcstone_stream s, const K* tree, int32_t
     return HIPCSTONE_OK;
 }
 
-// Warm-step node counts from the particle positions of the old leaf boundaries: oldPos[i] = lower_bound(keys,
-// tree[i]) for the old leaf array (the bucket offsets of a sort through those leaves, i in [0, numNodes]). Every
-// boundary of the rebalanced array is an old boundary (kept or merged nodes, the first child of a split), whose
-// position is oldPos, or a split child's start inside old node i, whose lower bound lies in [oldPos[i], oldPos[i+1])
-// and is searched there only. One thread per old node writes the positions of the boundaries it produced (the same
-// mapping as rebalanceKernel); counts are then differences of consecutive positions, exactly computeNodeCounts'.
+// The rebalanced array of a warm step with its node counts, from the particle positions of the old leaf boundaries:
+// oldPos[i] = lower_bound(keys, tree[i]) for the old leaf array (the bucket offsets of a sort through those leaves, i in
+// [0, numNodes]). Every boundary of the new array is an old boundary (kept or merged nodes, the first child of a split),
+// whose position is oldPos, or a split child's start inside old node i, whose lower bound lies in
+// [oldPos[i], oldPos[i+1]) and is searched there only. One thread per old node writes the nodes it leaves behind
+// (rebalanceKernel's mapping) and their counts, exactly computeNodeCounts': a kept node ends where the next one begins
+// that is not merged away (at most 7 further on).
 template<class K>
-__global__ __launch_bounds__(256) void warmBoundaryPosKernel(const K* __restrict__ tree, int32_t numNodes,
-                                                             const int32_t* __restrict__ nodeOps,
-                                                             const K* __restrict__ newTree,
-                                                             const K* __restrict__ keys,
-                                                             const uint32_t* __restrict__ oldPos,
-                                                             uint32_t* __restrict__ pos)
+__global__ __launch_bounds__(256) void rebalanceWarmKernel(const K* __restrict__ tree, int32_t numNodes,
+                                                           const int32_t* __restrict__ nodeOps,
+                                                           const K* __restrict__ keys,
+                                                           const uint32_t* __restrict__ oldPos, uint32_t maxCount,
+                                                           K* __restrict__ newTree, uint32_t* __restrict__ counts)
 {
     int32_t i = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i == numNodes) pos[nodeOps[numNodes]] = oldPos[numNodes];
+    if (i == numNodes) newTree[nodeOps[numNodes]] = tree[numNodes];
     if (i >= numNodes) return;
-    const int32_t op  = nodeOps[i + 1] - nodeOps[i];
     const int32_t dst = nodeOps[i];
+    const int32_t op  = nodeOps[i + 1] - dst;
     if (op == 0) return;
-    const uint32_t a = oldPos[i];
-    pos[dst]         = a;
-    if (op >= 8)
+    const K thisNode = tree[i];
+    int32_t next     = i + 1;
+    while (next < numNodes && nodeOps[next + 1] == dst + op)
+        ++next;
+    uint32_t from      = oldPos[i];
+    const uint32_t end = oldPos[next];
+    if (op == 1)
     {
-        const uint32_t b = oldPos[i + 1];
-        for (int32_t c = 1; c < op; ++c)
-            pos[dst + c] = a + uint32_t(lowerBound(keys + a, size_t(b - a), newTree[dst + c]));
+        newTree[dst] = thisNode;
+        counts[dst]  = min(end - from, maxCount);
+        return;
     }
-}
-
-__global__ __launch_bounds__(256) void countsFromPosKernel(const uint32_t* __restrict__ pos, int32_t numNodes,
-                                                           uint32_t maxCount, uint32_t* __restrict__ counts)
-{
-    int32_t i = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= numNodes) return;
-    const uint32_t c = pos[i + 1] - pos[i];
-    counts[i]        = c < maxCount ? c : maxCount;
+    const unsigned level     = treeLevel(K(tree[i + 1] - thisNode));
+    const unsigned levelDiff = op == 8 ? 1u : log8ceil(K(uint32_t(op)));
+    const K step             = nodeRange<K>(level + levelDiff);
+    const uint32_t a = from, b = oldPos[i + 1];
+    for (int32_t c = 0; c < op; ++c)
+    {
+        const uint32_t to =
+            c + 1 < op ? a + uint32_t(lowerBound(keys + a, size_t(b - a), K(thisNode + K(c + 1) * step))) : end;
+        newTree[dst + c] = thisNode + K(c) * step;
+        counts[dst + c]  = min(to - from, maxCount);
+        from             = to;
+    }
 }
 
 // workspace: [nodeOps (numNodes+1) int32][node-ops workspace]
@@ -234,8 +244,7 @@ template<class K>
 static hipcstone_status updateOctree(hipcstone_stream s, const K* keys, size_t numKeys, uint32_t bucketSize,
                                      const K* tree, const uint32_t* counts, int32_t* numNodes, K* newTree,
                                      uint32_t* newCounts, int32_t capacity, uint32_t maxCount, void* ws,
-                                     size_t wsBytes, int* converged, const uint32_t* oldPos = nullptr,
-                                     uint32_t* posWs = nullptr)
+                                     size_t wsBytes, int* converged, const uint32_t* oldPos = nullptr)
 {
     if (!numNodes || *numNodes <= 0) return invalid("updateOctree: numNodes must be positive");
     if (bucketSize == 0) return invalid("updateOctree: bucketSize must be positive");
@@ -255,16 +264,19 @@ static hipcstone_status updateOctree(hipcstone_stream s, const K* keys, size_t n
         hipcstone::setError("updateOctree: capacity too small for the rebalanced tree");
         return HIPCSTONE_CAPACITY;
     }
-    if (auto e = rebalanceTree<K>(s, tree, n, newN, nodeOps, newTree)) return e;
-    if (oldPos && posWs)
+    if (oldPos)
     {
-        warmBoundaryPosKernel<K><<<ceilDiv(size_t(n) + 1, 256), 256, 0, stream(s)>>>(tree, n, nodeOps, newTree, keys,
-                                                                                      oldPos, posWs);
-        HC_CHECK_LAUNCH("warmBoundaryPosKernel");
-        countsFromPosKernel<<<ceilDiv(size_t(newN), 256), 256, 0, stream(s)>>>(posWs, newN, maxCount, newCounts);
-        HC_CHECK_LAUNCH("countsFromPosKernel");
+        if (newN <= 0) return invalid("rebalanceTree: sizes must be positive");
+        if (!newTree || !newCounts || (numKeys && !keys)) return invalid("updateOctree: null pointer");
+        rebalanceWarmKernel<K><<<ceilDiv(size_t(n) + 1, 256), 256, 0, stream(s)>>>(tree, n, nodeOps, keys, oldPos,
+                                                                                    maxCount, newTree, newCounts);
+        HC_CHECK_LAUNCH("rebalanceWarmKernel");
     }
-    else if (auto e = computeNodeCounts<K>(s, newTree, newCounts, newN, keys, numKeys, maxCount)) return e;
+    else
+    {
+        if (auto e = rebalanceTree<K>(s, tree, n, newN, nodeOps, newTree)) return e;
+        if (auto e = computeNodeCounts<K>(s, newTree, newCounts, newN, keys, numKeys, maxCount)) return e;
+    }
     *numNodes = newN;
     return HIPCSTONE_OK;
 }
@@ -273,18 +285,18 @@ template<class K>
 hipcstone_status updateOctreeWarm(hipcstone_stream s, const K* keys, size_t numKeys, uint32_t bucketSize,
                                   const K* tree, const uint32_t* counts, int32_t* numNodes, K* newTree,
                                   uint32_t* newCounts, int32_t capacity, void* ws, size_t wsBytes, int* converged,
-                                  const uint32_t* oldPos, uint32_t* posWs)
+                                  const uint32_t* oldPos)
 {
     return updateOctree<K>(s, keys, numKeys, bucketSize, tree, counts, numNodes, newTree, newCounts, capacity,
-                           0xFFFFFFFFu, ws, wsBytes, converged, oldPos, posWs);
+                           0xFFFFFFFFu, ws, wsBytes, converged, oldPos);
 }
 
 template hipcstone_status updateOctreeWarm<uint32_t>(hipcstone_stream, const uint32_t*, size_t, uint32_t,
                                                      const uint32_t*, const uint32_t*, int32_t*, uint32_t*, uint32_t*,
-                                                     int32_t, void*, size_t, int*, const uint32_t*, uint32_t*);
+                                                     int32_t, void*, size_t, int*, const uint32_t*);
 template hipcstone_status updateOctreeWarm<uint64_t>(hipcstone_stream, const uint64_t*, size_t, uint32_t,
                                                      const uint64_t*, const uint32_t*, int32_t*, uint64_t*, uint32_t*,
-                                                     int32_t, void*, size_t, int*, const uint32_t*, uint32_t*);
+                                                     int32_t, void*, size_t, int*, const uint32_t*);
 
 } // namespace hipcstone
 

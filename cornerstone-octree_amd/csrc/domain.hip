@@ -97,7 +97,9 @@ __global__ __launch_bounds__(6 * kWave) void minMaxFinalKernel(const T* __restri
 
 // ---------------------------------------------------------------- global tree: largest leaf count
 
-__global__ void maxCountKernel(const uint32_t* __restrict__ counts, int32_t n, uint32_t* __restrict__ out)
+constexpr int kMaxCountThreads = 512;
+
+__global__ __launch_bounds__(kMaxCountThreads) void maxCountKernel(const uint32_t* __restrict__ counts, int32_t n, uint32_t* __restrict__ out)
 {
     uint32_t m = 0;
     for (int32_t i = int32_t(blockIdx.x * blockDim.x + threadIdx.x); i < n; i += int32_t(gridDim.x * blockDim.x))
@@ -107,8 +109,26 @@ __global__ void maxCountKernel(const uint32_t* __restrict__ counts, int32_t n, u
         uint32_t o = __shfl_xor(m, off, kWave);
         m          = o > m ? o : m;
     }
-    // the maximum only grows: skip the atomic when it already holds at least m (thousands of waves share *out)
-    if (laneId() == 0 && m > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, m);
+    // one atomic per workgroup: the atomics on one word, one after the other, are what this kernel waits for (one per
+    // wave, 4096 of them, made it 51 us for 440k counts, now 4.6)
+    __shared__ uint32_t most[kMaxCountThreads / kWave];
+    if (laneId() == 0) most[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        for (uint32_t o : most)
+            m = o > m ? o : m;
+        atomicMax(out, m);
+    }
+}
+
+// the three flags of a focus update, its new leaf count and the fault word, into pinned host memory
+__global__ void readFocusKernel(const int32_t* flags, const int32_t* newNumLeaves, const uint32_t* faults, uint32_t* host)
+{
+    const int t = threadIdx.x;
+    if (t < 3) host[t] = uint32_t(flags[t]);
+    if (t == 3) host[t] = uint32_t(*newNumLeaves);
+    if (t == 4) host[t] = *faults;
 }
 
 // ---------------------------------------------------------------- focus tree decisions
@@ -664,10 +684,11 @@ private:
             int blocks = int(std::min<size_t>(kMmBlocks, ceilDiv(n_, kMmThreads)));
             minMaxPartialKernel<T><<<blocks, kMmThreads, 0, stream(s)>>>(x, y, z, n_, mmPartials_.as<T>());
             HC_CHECK_LAUNCH("minMaxPartialKernel");
-            minMaxFinalKernel<T><<<1, 6 * kWave, 0, stream(s)>>>(mmPartials_.as<T>(), blocks, mmOut_.as<T>());
+            uint32_t* pin = pinnedStaging();
+            if (!pin) return HIPCSTONE_HIP_ERROR;
+            T* mm = reinterpret_cast<T*>(pin + kMinMaxWords);
+            minMaxFinalKernel<T><<<1, 6 * kWave, 0, stream(s)>>>(mmPartials_.as<T>(), blocks, mm);
             HC_CHECK_LAUNCH("minMaxFinalKernel");
-            T mm[6];
-            HC_CHECK(hipMemcpyAsync(mm, mmOut_.ptr, sizeof(mm), hipMemcpyDeviceToHost, stream(s)));
             HC_CHECK(hipStreamSynchronize(stream(s)));
             for (int d = 0; d < 3; ++d)
                 if (!keep[d])
@@ -763,7 +784,6 @@ private:
             if (auto e = xyzh_[a].reserve(n * sizeof(T))) return e;
         if (auto e = sortWs_.reserve(A::sortWs(n))) return e;
         if (auto e = mmPartials_.reserve(size_t(kMmBlocks) * 6 * sizeof(T))) return e;
-        if (auto e = mmOut_.reserve(6 * sizeof(T))) return e;
         if (auto e = small_.reserve(64)) return e;
         capN_ = n;
         return HIPCSTONE_OK;
@@ -816,12 +836,10 @@ private:
             hipcstone_status e;
             if (warm)
             {
-                if (auto g = posWs_.reserve((size_t(capGlobal_) + 1) * sizeof(uint32_t))) return g;
                 e = updateOctreeWarm<K>(s, keys_.as<K>(), n_, bucket_, gTree_[gCur_].template as<K>(),
                                         gCounts_[gCur_].template as<uint32_t>(), &nn, gTree_[other].template as<K>(),
                                         gCounts_[other].template as<uint32_t>(), capGlobal_, updWs_.ptr,
-                                        updWs_.bytes, &conv, bsWs_.as<uint32_t>() + numGlobal_,
-                                        posWs_.as<uint32_t>());
+                                        updWs_.bytes, &conv, bsWs_.as<uint32_t>() + numGlobal_);
             }
             else
             {
@@ -845,11 +863,14 @@ private:
             uint32_t* dmax = small_.as<uint32_t>();
             setU32Kernel<<<1, 1, 0, stream(s)>>>(dmax, 0u);
             HC_CHECK_LAUNCH("setU32Kernel");
-            unsigned blocks = std::min<unsigned>(1024, ceilDiv(size_t(nn), 256));
-            maxCountKernel<<<blocks, 256, 0, stream(s)>>>(gCounts_[gCur_].template as<uint32_t>(), nn, dmax);
+            unsigned blocks = std::min<unsigned>(256, ceilDiv(size_t(nn), kMaxCountThreads));
+            maxCountKernel<<<blocks, kMaxCountThreads, 0, stream(s)>>>(gCounts_[gCur_].template as<uint32_t>(), nn, dmax);
             HC_CHECK_LAUNCH("maxCountKernel");
-            HC_CHECK(hipMemcpyAsync(result, dmax, sizeof(uint32_t), hipMemcpyDeviceToHost, stream(s)));
+            uint32_t* pin = pinnedStaging();
+            if (!pin) return HIPCSTONE_HIP_ERROR;
+            if (auto g = enqueueWordRead(stream(s), dmax, pin + kCountWord)) return g;
             HC_CHECK(hipStreamSynchronize(stream(s)));
+            *result = pin[kCountWord];
             return HIPCSTONE_OK;
         }
         return invalid("domain: global leaf capacity growth did not converge");
@@ -955,15 +976,16 @@ private:
         if (auto e = scan::exclusiveScan<int32_t>(stream(s), leafOps_.as<int32_t>(), leafOps_.as<int32_t>(),
                                                   size_t(L) + 1, 0, nullptr, scanWs_.ptr, scanWs_.bytes))
             return e;
-        int32_t hostFlags[4];
-        HC_CHECK(hipMemcpyAsync(hostFlags, flags, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, stream(s)));
-        HC_CHECK(hipMemcpyAsync(hostFlags + 3, leafOps_.as<int32_t>() + L, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                stream(s)));
-        // the device's fault word rides along with this synchronization (guards of the sort and earlier kernels)
-        uint32_t faults = 0;
-        if (auto e = enqueueFaultRead(stream(s), &faults)) return e;
+        // the flags, the new leaf count and the device's fault word (guards of the sort and earlier kernels)
+        uint32_t* pin         = pinnedStaging();
+        const uint32_t* fault = faultWord();
+        if (!pin || !fault) return HIPCSTONE_HIP_ERROR;
+        const uint32_t* words = pin + kFocusWords;
+        readFocusKernel<<<1, kWave, 0, stream(s)>>>(flags, leafOps_.as<int32_t>() + L, fault, pin + kFocusWords);
+        HC_CHECK_LAUNCH("readFocusKernel");
         HC_CHECK(hipStreamSynchronize(stream(s)));
-        if (auto e = checkFaults(faults)) return e;
+        const int32_t hostFlags[4] = {int32_t(words[0]), int32_t(words[1]), int32_t(words[2]), int32_t(words[3])};
+        if (auto e = checkFaults(words[4])) return e;
         const int status = hostFlags[0];
         const int32_t newL = hostFlags[3];
         int conv = hostFlags[1] == 0;
@@ -994,11 +1016,9 @@ private:
             uniqueScatterKernel<K><<<ceilDiv(size_t(total), 256), 256, 0, stream(s)>>>(
                 fLeavesNew_.as<K>(), injFlags_.as<uint32_t>(), total, injKeyBuf_.as<K>());
             HC_CHECK_LAUNCH("uniqueScatterKernel");
-            uint32_t unique = 0;
-            HC_CHECK(hipMemcpyAsync(&unique, injFlags_.as<uint32_t>() + total, sizeof(uint32_t),
-                                    hipMemcpyDeviceToHost, stream(s)));
+            if (auto e = enqueueWordRead(stream(s), injFlags_.as<uint32_t>() + total, pin + kCountWord)) return e;
             HC_CHECK(hipStreamSynchronize(stream(s)));
-            numKeys = int32_t(unique);
+            numKeys = int32_t(pin[kCountWord]);
             HC_CHECK(hipMemcpyAsync(fLeavesNew_.ptr, injKeyBuf_.ptr, size_t(numKeys) * sizeof(K),
                                     hipMemcpyDeviceToDevice, stream(s)));
         }
@@ -1061,14 +1081,17 @@ private:
     int32_t fL_ = 0, fN_ = 0;
     int globalSteps_ = 0, focusSteps_ = 0, focusConverged_ = 0;
 
-    DeviceBuf keys_, keyBuf_, perm_, valBuf_, sortWs_, mmPartials_, mmOut_, small_, bsWs_, bsScanWs_, gLayout_,
+    DeviceBuf keys_, keyBuf_, perm_, valBuf_, sortWs_, mmPartials_, small_, bsWs_, bsScanWs_, gLayout_,
         hintWs_;
     // pinned word of the calling thread that receives a deferred largest bucket (the pipeline's is word 9)
     static constexpr int kMaxWord = 10;
+    // and others for what kernels store on the way to a synchronization
+    static constexpr int kCountWord = 11, kFocusWords = 16 /* 5 of them */, kMinMaxWords = 32 /* 6 T */;
+    static_assert(kMinMaxWords + 6 * sizeof(T) / 4 <= kPinnedWords);
     uint32_t lastMaxBucket_ = ~0u;  // largest bucket of the last bucket sort, ~0 when unknown
     bool maxPending_        = false; // the last sort's largest bucket is on its way to pinned word kMaxWord
     DeviceBuf xyzh_[4];
-    DeviceBuf gTree_[2], gCounts_[2], updWs_, posWs_;
+    DeviceBuf gTree_[2], gCounts_[2], updWs_;
     bool warmPos_ = false; // this call's bucket sort left the old global boundaries' positions in bsWs_
     DeviceBuf fLeaves_, fLeavesNew_, fLeafCounts_, fNodeCounts_, leafOps_, ops_, prot_;
     DeviceBuf prefixes_, childOffsets_, parents_, levelRange_, internalToLeaf_, leafToInternal_, buildWs_;

@@ -7,6 +7,7 @@
 #include "common.hpp"
 #include "runtime.hpp"
 #include "scan.hpp"
+#include "sort.hpp"
 
 extern "C" size_t hipcstone_sort_by_key_workspace_size_u32(size_t n);
 
@@ -48,12 +49,16 @@ __global__ __launch_bounds__(256) void nodeLevelsKernel(const K* __restrict__ le
     }
 }
 
-// order = the first numNodes sorted entries: prefixes[i] = unsorted prefix of node order[i];
-// leafToInternal[order[i]] = i; internalToLeaf[i] = order[i] - numInternal (octree.hpp:176-185)
+// order and level = the first numNodes sorted entries: prefixes[i] = unsorted prefix of node order[i];
+// leafToInternal[order[i]] = i; internalToLeaf[i] = order[i] - numInternal (octree.hpp:176-185); childOffsets[i] = 0 for
+// linkKernel; levelRange (getLevelRangeCpu, octree.hpp:151-160): the first node index of every level from the places
+// where the level changes, levelRange[L + 1] = numNodes
 template<class K>
-__global__ void invertOrderKernel(const uint32_t* __restrict__ order, int32_t numNodes, int32_t numInternal,
-                                  const K* __restrict__ unsortedPrefixes, K* __restrict__ prefixes,
-                                  int32_t* __restrict__ internalToLeaf, int32_t* __restrict__ leafToInternal)
+__global__ void invertOrderKernel(const uint32_t* __restrict__ order, const uint32_t* __restrict__ level,
+                                  int32_t numNodes, int32_t numInternal, const K* __restrict__ unsortedPrefixes,
+                                  K* __restrict__ prefixes, int32_t* __restrict__ internalToLeaf,
+                                  int32_t* __restrict__ leafToInternal, int32_t* __restrict__ childOffsets,
+                                  int32_t* __restrict__ levelRange)
 {
     int32_t i = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= numNodes) return;
@@ -61,6 +66,17 @@ __global__ void invertOrderKernel(const uint32_t* __restrict__ order, int32_t nu
     prefixes[i]        = unsortedPrefixes[o];
     leafToInternal[o]  = i;
     internalToLeaf[i]  = o - numInternal;
+    childOffsets[i]    = 0;
+    constexpr int L    = int(maxLevel<K>());
+    const int here     = min(int(level[i]), L);
+    const int before   = i > 0 ? int(level[i - 1]) : -1;
+    for (int l = before + 1; l <= here; ++l)
+        levelRange[l] = i;
+    if (i == numNodes - 1)
+    {
+        for (int l = here + 1; l <= L + 1; ++l)
+            levelRange[l] = numNodes;
+    }
 }
 
 template<class K>
@@ -82,17 +98,7 @@ __device__ inline int32_t lowerBoundIdx(const K* a, int32_t lo, int32_t hi, K v)
     return lo;
 }
 
-// getLevelRangeCpu (octree.hpp:151-160): first node index of every level, levelRange[L+1] = numNodes
-template<class K>
-__global__ void levelRangeKernel(const K* __restrict__ prefixes, int32_t numNodes, int32_t* __restrict__ levelRange)
-{
-    int level = int(threadIdx.x);
-    constexpr int L = int(maxLevel<K>());
-    if (level <= L) levelRange[level] = lowerBoundIdx(prefixes, 0, numNodes, encodePlaceholderBit(K(0), 3 * level));
-    if (level == L + 1) levelRange[level] = numNodes;
-}
-
-// linkTreeCpu (octree.hpp:114-148), childOffsets pre-zeroed
+// linkTreeCpu (octree.hpp:114-148), childOffsets pre-zeroed (invertOrderKernel)
 template<class K>
 __global__ __launch_bounds__(256) void linkKernel(const K* __restrict__ prefixes, int32_t numInternal,
                                                   const int32_t* __restrict__ leafToInternal,
@@ -115,12 +121,6 @@ __global__ __launch_bounds__(256) void linkKernel(const K* __restrict__ prefixes
         childOffsets[idxA]          = childIdx;
         parents[(childIdx - 1) / 8] = idxA;
     }
-}
-
-__global__ void fillI32Kernel(int32_t* p, size_t n, int32_t v)
-{
-    size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
 }
 
 // nodeFpCenters + centerAndSize; node keys decoded as Hilbert keys like the reference (sfcKey -> SfcKind)
@@ -148,9 +148,6 @@ __global__ __launch_bounds__(256) void geoCentersKernel(const K* __restrict__ pr
     sizes[o + 1]   = T(ib[3] - ib[2]) * hy;
     sizes[o + 2]   = T(ib[5] - ib[4]) * hz;
 }
-
-extern "C" hipcstone_status hipcstone_sort_by_key_u32(hipcstone_stream, uint32_t*, uint32_t*, size_t, uint32_t*,
-                                                      uint32_t*, void*, size_t, int);
 
 static inline size_t a256(size_t v) { return (v + 255) & ~size_t(255); }
 
@@ -182,28 +179,25 @@ static hipcstone_status buildOctree(hipcstone_stream s, const K* leaves, int32_t
     char* w             = static_cast<char*>(ws);
     K* unsortedPrefixes = reinterpret_cast<K*>(w);
     w += a256(N * sizeof(K));
-    uint32_t* level = reinterpret_cast<uint32_t*>(w);
+    uint32_t* level = reinterpret_cast<uint32_t*>(w); // the sorted entries' levels
     w += a256(E * 4);
-    uint32_t* order = reinterpret_cast<uint32_t*>(w); // the node of each entry, then (sorted) the node order
+    uint32_t* order = reinterpret_cast<uint32_t*>(w); // and nodes
     w += a256(E * 4);
-    uint32_t* keyBuf = reinterpret_cast<uint32_t*>(w);
+    uint32_t* keyBuf = reinterpret_cast<uint32_t*>(w); // the entries in creation order
     w += a256(E * 4);
     uint32_t* valueBuf = reinterpret_cast<uint32_t*>(w);
     w += a256(E * 4);
     const size_t sortWsBytes = wsBytes - size_t(w - static_cast<char*>(ws));
 
     nodeLevelsKernel<K><<<ceilDiv(size_t(numLeaves), 256), 256, 0, st>>>(leaves, numInternal, numLeaves,
-                                                                          unsortedPrefixes, level, order);
+                                                                          unsortedPrefixes, keyBuf, valueBuf);
     HC_CHECK_LAUNCH("nodeLevelsKernel");
     // one 8-bit pass: levels are at most 21, 255 marks the entries without a node (they sort last)
-    if (auto e = hipcstone_sort_by_key_u32(st, level, order, E, keyBuf, valueBuf, w, sortWsBytes, 8)) return e;
-    invertOrderKernel<K><<<ceilDiv(N, 256), 256, 0, st>>>(order, numNodes, numInternal, unsortedPrefixes, prefixes,
-                                                          internalToLeaf, leafToInternal);
+    if (auto e = sortPairsFromBuf(st, keyBuf, valueBuf, E, level, order, w, sortWsBytes, 8)) return e;
+    invertOrderKernel<K><<<ceilDiv(N, 256), 256, 0, st>>>(order, level, numNodes, numInternal, unsortedPrefixes,
+                                                          prefixes, internalToLeaf, leafToInternal, childOffsets,
+                                                          levelRange);
     HC_CHECK_LAUNCH("invertOrderKernel");
-    levelRangeKernel<K><<<1, 64, 0, st>>>(prefixes, numNodes, levelRange);
-    HC_CHECK_LAUNCH("levelRangeKernel");
-    fillI32Kernel<<<ceilDiv(N, 256), 256, 0, st>>>(childOffsets, N, 0);
-    HC_CHECK_LAUNCH("fillI32Kernel");
     if (numInternal > 0)
     {
         linkKernel<K><<<ceilDiv(size_t(numInternal), 256), 256, 0, st>>>(prefixes, numInternal, leafToInternal,

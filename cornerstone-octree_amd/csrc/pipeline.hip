@@ -153,11 +153,12 @@ __device__ inline uint32_t lowerBoundIn(const K* __restrict__ keys, uint32_t lo,
 // the root's key range: keys at or past nodeRange(0) (removed particles) belong to no leaf
 template<class K>
 __global__ void splitRootKernel(const K* __restrict__ keys, uint32_t n, SplitNode<K>* __restrict__ frontier,
-                                uint32_t* __restrict__ rootCount)
+                                uint32_t* __restrict__ counters, uint32_t* __restrict__ host)
 {
     uint32_t hi = lowerBoundIn(keys, 0u, n, nodeRange<K>(0));
     frontier[0] = SplitNode<K>{K(0), 0u, hi};
-    *rootCount  = hi;
+    counters[0] = counters[1] = 0;
+    *host       = hi;
 }
 
 // 8 lanes per frontier node, lane k for child k; counters[0] counts the next frontier, counters[1] all leaves
@@ -198,10 +199,12 @@ __global__ __launch_bounds__(256) void splitLevelKernel(const K* __restrict__ ke
     }
 }
 
-__global__ void setU32PairKernel(uint32_t* p, uint32_t a, uint32_t b)
+// a level's counts into pinned host memory; the next level's frontier starts at zero, the leaves add up
+__global__ void takeSplitCountersKernel(uint32_t* counters, uint32_t* host)
 {
-    p[0] = a;
-    p[1] = b;
+    host[0]     = counters[0];
+    host[1]     = counters[1];
+    counters[0] = 0;
 }
 
 template<class K, class T>
@@ -414,7 +417,7 @@ public:
     size_t deviceBytes() const override
     {
         size_t b = 0;
-        for (const DeviceBuf* d : {&keys_, &keyBuf_, &perm_, &valBuf_, &sortWs_, &segWs_, &hintWs_, &updWs_, &posWs_,
+        for (const DeviceBuf* d : {&keys_, &keyBuf_, &perm_, &valBuf_, &sortWs_, &segWs_, &hintWs_, &updWs_,
                                    &splitKeys_, &splitCounts_, &splitCounters_, &splitSortWs_, &prefixes_, &childOffsets_,
                                    &parents_, &levelRange_, &internalToLeaf_, &leafToInternal_, &buildWs_, &centers_,
                                    &sizes_, &layout_, &scanWs_, &assignOff_, &assignBnd_, &assignCnt_, &assignWs_,
@@ -523,11 +526,10 @@ private:
             hipcstone_status e;
             if (warm)
             {
-                if (auto g = posWs_.reserve((size_t(capLeaves_) + 1) * sizeof(uint32_t))) return g;
                 e = updateOctreeWarm<K>(s, keys_.as<K>(), n_, bucket_, tree_[treeCur_].template as<K>(),
                                         counts_[treeCur_].template as<uint32_t>(), &nn, tree_[other].template as<K>(),
                                         counts_[other].template as<uint32_t>(), capLeaves_, updWs_.ptr, updWs_.bytes,
-                                        converged, segWs_.as<uint32_t>() + numLeaves_, posWs_.as<uint32_t>());
+                                        converged, segWs_.as<uint32_t>() + numLeaves_);
             }
             else
             {
@@ -557,18 +559,20 @@ private:
         if (auto e = reserveLeaves(std::max<int32_t>(capLeaves_, 4096))) return e;
         if (auto e = splitCounters_.reserve(2 * sizeof(uint32_t))) return e;
         if (auto e = frontier_[0].reserve(sizeof(SplitNode<K>))) return e;
+        uint32_t* pin = pinnedStaging();
+        if (!pin) return HIPCSTONE_HIP_ERROR;
+        uint32_t* host = pin + 16; // (words of the level counts)
         splitRootKernel<K><<<1, 1, 0, stream(s)>>>(keys_.as<K>(), uint32_t(n_), frontier_[0].as<SplitNode<K>>(),
-                                                   splitCounters_.as<uint32_t>());
+                                                   splitCounters_.as<uint32_t>(), host);
         HC_CHECK_LAUNCH("splitRootKernel");
-        uint32_t host[2];
-        HC_CHECK(hipMemcpyAsync(host, splitCounters_.ptr, sizeof(uint32_t), hipMemcpyDeviceToHost, stream(s)));
         HC_CHECK(hipStreamSynchronize(stream(s)));
         const K rootKeys[2] = {K(0), nodeRange<K>(0)};
-        if (host[0] <= bucket_)
+        const uint32_t rootCount = host[0];
+        if (rootCount <= bucket_)
         {
             HC_CHECK(hipMemcpyAsync(tree_[treeCur_].ptr, rootKeys, sizeof(rootKeys), hipMemcpyHostToDevice,
                                     stream(s)));
-            HC_CHECK(hipMemcpyAsync(counts_[treeCur_].ptr, &host[0], sizeof(uint32_t), hipMemcpyHostToDevice,
+            HC_CHECK(hipMemcpyAsync(counts_[treeCur_].ptr, &rootCount, sizeof(uint32_t), hipMemcpyHostToDevice,
                                     stream(s)));
             numLeaves_      = 1;
             convergedCalls_ = 0;
@@ -584,14 +588,13 @@ private:
             if (auto e = growKeep(splitKeys_, (leaves + nOutMax) * sizeof(K), leaves * sizeof(K), s)) return e;
             if (auto e = growKeep(splitCounts_, (leaves + nOutMax) * sizeof(uint32_t), leaves * sizeof(uint32_t), s))
                 return e;
-            setU32PairKernel<<<1, 1, 0, stream(s)>>>(splitCounters_.as<uint32_t>(), 0u, leaves);
-            HC_CHECK_LAUNCH("setU32PairKernel");
             splitLevelKernel<K><<<ceilDiv(nOutMax, 256), 256, 0, stream(s)>>>(
                 keys_.as<K>(), frontier_[cur].as<SplitNode<K>>(), nIn, childLevel, bucket_,
                 frontier_[1 - cur].as<SplitNode<K>>(), splitKeys_.as<K>(), splitCounts_.as<uint32_t>(),
                 splitCounters_.as<uint32_t>());
             HC_CHECK_LAUNCH("splitLevelKernel");
-            HC_CHECK(hipMemcpyAsync(host, splitCounters_.ptr, sizeof(host), hipMemcpyDeviceToHost, stream(s)));
+            takeSplitCountersKernel<<<1, 1, 0, stream(s)>>>(splitCounters_.as<uint32_t>(), host);
+            HC_CHECK_LAUNCH("takeSplitCountersKernel");
             HC_CHECK(hipStreamSynchronize(stream(s)));
             nIn    = host[0];
             leaves = host[1];
@@ -693,7 +696,7 @@ private:
 
     DeviceBuf keys_, keyBuf_, perm_, valBuf_, sortWs_, segWs_, hintWs_;
     DeviceBuf xyzh_[2][4];
-    DeviceBuf tree_[2], counts_[2], updWs_, posWs_;
+    DeviceBuf tree_[2], counts_[2], updWs_;
     DeviceBuf frontier_[2], splitKeys_, splitCounts_, splitCounters_, splitSortWs_;
     DeviceBuf prefixes_, childOffsets_, parents_, levelRange_, internalToLeaf_, leafToInternal_, buildWs_;
     DeviceBuf centers_, sizes_, layout_, scanWs_, groupsWs_;

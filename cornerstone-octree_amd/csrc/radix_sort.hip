@@ -480,11 +480,12 @@ static int numPassesFor(int endBit)
     return (endBit + kRadixBits - 1) / kRadixBits;
 }
 
-// Generic driver. valueMode 0/1/2 as in onesweepPassKernel. When gather is set, the last pass gathers.
+// Generic driver. valueMode 0/1/2 as in onesweepPassKernel. When gather is set, the last pass gathers. fromBuf: the
+// input is in keyBuf and valueBuf (an odd number of passes, which then needs no copy to start with).
 template<class K, class GT>
 static hipcstone_status radixSort(hipStream_t s, K* keys, uint32_t* values, size_t n, K* keyBuf, uint32_t* valueBuf,
                                   void* workspace, size_t wsBytes, int endBit, int valueMode, const GatherArgs<GT>* g,
-                                  int beginBit = 0)
+                                  int beginBit = 0, bool fromBuf = false)
 {
     if (n == 0) return HIPCSTONE_OK;
     if (n > kValueMask) return invalid("radix sort: more than 2^30-1 keys");
@@ -496,19 +497,19 @@ static hipcstone_status radixSort(hipStream_t s, K* keys, uint32_t* values, size
     if (!workspace || wsBytes < need) return invalid("radix sort: workspace too small");
     if (!keys || !keyBuf) return invalid("radix sort: null key buffer");
     if (valueMode != 0 && (!values || !valueBuf)) return invalid("radix sort: null value buffer");
+    if (fromBuf && passes % 2 == 0) return invalid("radix sort: an even number of passes cannot start in the buffers");
 
     SortWorkspace w = carveWorkspace(workspace, n, passes, pack);
     size_t tiles    = numTiles(n);
     uint32_t* faults         = faultWord();
     const uint32_t spinLimit = sortLookbackLimit();
     if (!faults) return HIPCSTONE_HIP_ERROR;
-    if (auto st = zeroU32(w.hist, size_t(kMaxPasses) * kRadix, s)) return st;
-    if (auto st = zeroU32(w.counter, kMaxPasses + 1, s)) return st;
-    if (auto st = zeroU32(w.status, size_t(passes) * tiles * kRadix, s)) return st;
+    // histograms, counters and status lie one after the other
+    if (auto st = zeroU32(w.hist, size_t(w.status + size_t(passes) * tiles * kRadix - w.hist), s)) return st;
 
     unsigned hb = unsigned(std::min<size_t>(kHistBlocks, (n + kThreads - 1) / kThreads));
     uint32_t* descents = pack ? w.counter + kMaxPasses : nullptr;
-    histogramKernel<K><<<hb, kThreads, 0, s>>>(keys, n, passes, beginBit, endBit, w.hist, descents);
+    histogramKernel<K><<<hb, kThreads, 0, s>>>(fromBuf ? keyBuf : keys, n, passes, beginBit, endBit, w.hist, descents);
     HC_CHECK_LAUNCH("histogramKernel");
     GatherArgs<GT> gp{};
     if (pack)
@@ -525,8 +526,8 @@ static hipcstone_status radixSort(hipStream_t s, K* keys, uint32_t* values, size
     HC_CHECK_LAUNCH("scanHistogramKernel");
 
     // ping-pong so that the last pass writes into keys/values
-    K* src         = keys;
-    uint32_t* vsrc = values;
+    K* src         = fromBuf ? keyBuf : keys;
+    uint32_t* vsrc = fromBuf ? valueBuf : values;
     K* dst;
     uint32_t* vdst;
     GatherArgs<GT> noGather{};
@@ -608,6 +609,12 @@ hipcstone_status sortGatherBits(hipStream_t s, K* keys, uint32_t* perm, size_t n
     if (!xIn || !yIn || !zIn || !xOut || !yOut || !zOut || (hIn && !hOut)) return invalid("sortGather: null array");
     GatherArgs<T> g{xIn, yIn, zIn, hIn, xOut, yOut, zOut, hOut, nullptr, nullptr, 0};
     return radixSort<K, T>(s, keys, perm, n, keyBuf, valueBuf, ws, wsBytes, endBit, 2, &g, beginBit);
+}
+
+hipcstone_status sortPairsFromBuf(hipStream_t s, uint32_t* keyBuf, uint32_t* valueBuf, size_t n, uint32_t* keys,
+                                  uint32_t* values, void* ws, size_t wsBytes, int endBit)
+{
+    return radixSort<uint32_t, float>(s, keys, values, n, keyBuf, valueBuf, ws, wsBytes, endBit, 1, nullptr, 0, true);
 }
 
 template size_t sortGatherWorkspaceBytes<uint64_t>(size_t);

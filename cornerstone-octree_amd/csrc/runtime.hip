@@ -56,7 +56,15 @@ hipcstone_status enqueueFaultRead(hipStream_t s, uint32_t* host)
 {
     uint32_t* w = faultWord();
     if (!w) return HIPCSTONE_HIP_ERROR;
-    HC_CHECK(hipMemcpyAsync(host, w, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    return enqueueWordRead(s, w, host);
+}
+
+__global__ void readWordKernel(const uint32_t* word, uint32_t* host) { *host = *word; }
+
+hipcstone_status enqueueWordRead(hipStream_t s, const uint32_t* word, uint32_t* host)
+{
+    readWordKernel<<<1, 1, 0, s>>>(word, host);
+    HC_CHECK_LAUNCH("readWordKernel");
     return HIPCSTONE_OK;
 }
 

@@ -32,9 +32,12 @@ inline hipStream_t stream(hipcstone_stream s) { return reinterpret_cast<hipStrea
 // The current device's fault word (device address): kernels whose guards fire atomically OR HIPCSTONE_FAULT_* bits
 // into it. Resolved once per device; nullptr if the symbol lookup failed (the error text is then set).
 uint32_t* faultWord();
-// Read back with a stream-ordered copy into host memory (no synchronization); the orchestration objects enqueue it
+// Read back in stream order into pinned host memory (no synchronization); the orchestration objects enqueue it
 // before a synchronization they make anyway and then call checkFaults().
 hipcstone_status enqueueFaultRead(hipStream_t s, uint32_t* host);
+// the same for a word of device memory (host: pinned). A kernel stores it: on the host that takes half of what an
+// asynchronous copy takes.
+hipcstone_status enqueueWordRead(hipStream_t s, const uint32_t* word, uint32_t* host);
 hipcstone_status checkFaults(uint32_t faults);
 // A small pinned host buffer of the calling thread (kPinnedWords words, allocated on first use with hipHostMalloc and
 // kept until the process ends; nullptr if that failed, the error text is then set). Device-to-host copies into it are
@@ -79,12 +82,12 @@ int neighborWaves();
 
 // updateOctree (maxCount unlimited) whose node counts come from oldPos[i] = lower_bound(keys, tree[i]), i in
 // [0, *numNodes] (the bucket offsets of this step's sort through the same leaves): a bounded search per split child
-// instead of one over all keys per node. posWs holds capacity + 1 words.
+// instead of one over all keys per node.
 template<class K>
 hipcstone_status updateOctreeWarm(hipcstone_stream s, const K* keys, size_t numKeys, uint32_t bucketSize,
                                   const K* tree, const uint32_t* counts, int32_t* numNodes, K* newTree,
                                   uint32_t* newCounts, int32_t capacity, void* ws, size_t wsBytes, int* converged,
-                                  const uint32_t* oldPos, uint32_t* posWs);
+                                  const uint32_t* oldPos);
 
 // The neighbor search of hipcstone_find_neighbors_* with a workspace for the compact child blocks the walk reads
 // (neighborGroupsBytes(numNodes) bytes; with less, or none, they are allocated on the stream per call).
