@@ -26,12 +26,13 @@ namespace hipcstone
 // Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a tenth busy): the walk and
 // the chunks' set-up take 2.3 of 6.3 ms, the pair tests 2.5, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
 // search of that size took 7.70 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
-// instructions a wave, now 23.4K); in fp64 at 2M, where nothing was compact either, 1.73 -> 1.05 ms.
+// instructions a wave, now 23.4K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.98 ms.
 
 // Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.66 ms, 6 waves 6.31, 7 waves 7.1 (registers go
-// to memory; 16.8M targets). fp64 would have to spill for more than 4.
+// to memory; 16.8M targets). fp64, 300k uniform targets open / periodic: 4 waves 235 / 379 us, 5 waves 213 / 329, 6 waves
+// 224 / 387; 2M open: 975, 934, 1046 (30k, which do not fill the device: 82, 85, 92).
 template<class T>
-constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> ? 6 : 4;
+constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> ? 6 : 5;
 
 typedef uint32_t Row4 __attribute__((ext_vector_type(4), aligned(4)));
 
