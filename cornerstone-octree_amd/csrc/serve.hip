@@ -38,7 +38,7 @@ namespace serve
 // order-independent digest: the wrapping sum over particles of a hash of (i, key, count, stored neighbors). 16 lanes share
 // a particle's row and read consecutive slots (with a thread per row every load touched 64 rows), and a workgroup adds
 // its sum once: the additions to one word, a chain of about 10 ns each, bound what is left.
-// Mean over clouds of 10k to 150k particles, four on the device at once, ngmax 128: 183 -> 86 us.
+// Mean over clouds of 10k to 1M particles, four on the device at once, ngmax 128: 183 -> 86 us.
 constexpr int kDigestLanes   = 16;
 constexpr int kDigestThreads = 512;
 constexpr int kDigestBlocks  = 512;
