@@ -23,10 +23,10 @@ namespace hipcstone
 // how waves are grouped onto CUs (LDS per workgroup, scheduling granularity), never a result.
 // targetsPerWave: 64, or fewer where that many waves would leave the device idle (kFullWaves).
 //
-// Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a tenth busy): the walk takes
+// Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a sixth busy): the walk takes
 // 2.25 of 6.25 ms, the chunks' set-up 1.05, the pair tests 1.45, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
 // search of that size took 7.65 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
-// instructions a wave, now 23.4K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.98 ms.
+// instructions a wave, now 24.6K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.98 ms.
 
 // Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.66 ms, 6 waves 6.31, 7 waves 7.1 (registers go
 // to memory; 16.8M targets). fp64, 300k uniform targets open / periodic: 4 waves 235 / 379 us, 5 waves 213 / 329, 6 waves
