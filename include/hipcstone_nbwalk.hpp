@@ -263,14 +263,18 @@ struct WaveShared
     uint32_t spilled[kSpills][3][kSpillEntries]; // stack entries that did not fit the registers
     uint32_t marks[kWave];                       // scratch of one chunk
     uint32_t cand[(kChunks + 1) * kWave];        // the kept chunks' candidates (particle indices), and the next one's
-    uint32_t entries[kEntries + 1][kWave];       // column l: target l's kept hits (see HitReader), then a zero
+    uint32_t entries[kEntries + 1][kWave];       // column l: target l's kept hits (see HitReader), then one without any
 };
 
 // LDS by its address
 typedef __attribute__((address_space(3))) uint32_t LdsWord;
 __device__ inline uint32_t ldsAddress(const void* p) { return uint32_t((__UINTPTR_TYPE__)(const LdsWord*)p); }
-__device__ inline uint32_t ldsRead(uint32_t address) { return *(const LdsWord*)(__UINTPTR_TYPE__)address; }
 __device__ inline void ldsWrite(uint32_t address, uint32_t v) { *(LdsWord*)(__UINTPTR_TYPE__)address = v; }
+struct Lds
+{
+    __device__ static inline uint32_t read(uint32_t address) { return *(const LdsWord*)(__UINTPTR_TYPE__)address; }
+    __device__ static inline uint32_t lowest(uint32_t v) { return lowestBit(v); }
+};
 
 template<class T, int kNbWaves>
 struct Shared
@@ -404,37 +408,43 @@ struct Tree
 /*
  * A target's kept hits, in ascending order. They lie in its lane's column of WaveShared::entries, one entry per group of
  * 16 consecutive candidates that has any: bits 0-15 the hits, bits 16-31 the address of the group's first candidate
- * (in words of LDS). next() may be called past the last hit (by lanes that have fewer than others): the zero entry at
- * the end then stays the current one and some word of LDS is returned.
+ * (in words of LDS). After them comes one without hits (noHits), which stays the current one when next() is called past
+ * the last hit (by lanes that have fewer than others): its lowest bit is one of 16 to 31, so those calls read, and
+ * return, one of the candidates.
  */
+template<class Memory>
 struct HitReader
 {
-    uint32_t at, end;    // addresses of the entry read ahead and of the last, zero one
+    uint32_t at, end;    // addresses of the entry read ahead and of the last one, without hits
     uint32_t cur, ahead; // the entry being emptied, the one after it
 
     static constexpr uint32_t kEntryStep = kWave * sizeof(uint32_t);
 
-    __device__ inline HitReader(uint32_t from, uint32_t last)
-        : at(min(from + kEntryStep, last))
+    // candidates: the address (in words, not 0) of at least 32 of them
+    __host__ __device__ static inline uint32_t noHits(uint32_t candidates) { return candidates << 16; }
+
+    __host__ __device__ inline HitReader(uint32_t from, uint32_t last)
+        : at(from + kEntryStep < last ? from + kEntryStep : last)
         , end(last)
-        , cur(ldsRead(from))
-        , ahead(ldsRead(at))
+        , cur(Memory::read(from))
+        , ahead(Memory::read(at))
     {
     }
 
-    __device__ inline uint32_t next()
+    __host__ __device__ inline uint32_t next()
     {
-        const uint32_t j = ldsRead(((cur >> 16) + lowestBit(cur)) * 4u);
+        const uint32_t j = Memory::read(((cur >> 16) + Memory::lowest(cur)) * 4u);
         cur &= cur - 1;
         if (uint16_t(cur) == 0)
         {
             cur   = ahead;
-            at    = min(at + kEntryStep, end);
-            ahead = ldsRead(at);
+            at    = at + kEntryStep < end ? at + kEntryStep : end;
+            ahead = Memory::read(at);
         }
         return j;
     }
 };
+using LdsHits = HitReader<Lds>;
 
 /*
  * Walks the tree from `root` for the wave's targets first + lane (lanes with `valid` false take no part); returns this
@@ -592,13 +602,14 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
     const uint32_t entriesAt = ldsAddress(&sh.entries[0][0]);
     uint32_t entryEnd        = entriesAt + uint32_t(lane) * 4u;
     const uint32_t candAt = ldsAddress(sh.cand) / 4u;
+    static_assert(offsetof(WaveShared, cand) > 0); // (so candAt is not 0, see HitReader)
 
     auto handOver = [&]() __attribute__((always_inline)) {
-        ldsWrite(entryEnd, 0);
+        ldsWrite(entryEnd, LdsHits::noHits(candAt));
         waveSync();
         if (handOn)
         {
-            HitReader hits(entriesAt + uint32_t(lane) * 4u, entryEnd);
+            LdsHits hits(entriesAt + uint32_t(lane) * 4u, entryEnd);
             consume(handed, total - handed, [&]() __attribute__((always_inline)) { return hits.next(); });
         }
         waveSync();
@@ -811,7 +822,7 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
                 // an entry for each group of 16 with hits: every group's is written, only those with hits stay
                 auto append = [&](uint32_t entry) {
                     ldsWrite(entryEnd, entry);
-                    entryEnd += uint16_t(entry) != 0 ? HitReader::kEntryStep : 0u;
+                    entryEnd += uint16_t(entry) != 0 ? LdsHits::kEntryStep : 0u;
                 };
                 append((group << 16) | (lo & 0xFFFFu));
                 append(((group + 16u) << 16) | (lo >> 16));
@@ -821,7 +832,7 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
             }
             // a full set of chunks, or a column without room for another chunk's entries, goes out; at the end the rest
             const bool full = numChunks == kChunks ||
-                              ballot(entryEnd >= entriesAt + (kEntries - 3) * HitReader::kEntryStep) != 0;
+                              ballot(entryEnd >= entriesAt + (kEntries - 3) * LdsHits::kEntryStep) != 0;
             if (more ? full : last && numChunks != 0) handOver();
             if (!more) break;
         }
