@@ -5,6 +5,7 @@
 // sfc/box.hpp:318-335 (centerAndSize). The node order is level-major, SFC order within a level (sorted
 // Warren-Salmon prefixes); every output array is uniquely determined by the leaves.
 #include "common.hpp"
+#include "link.hpp"
 #include "runtime.hpp"
 #include "scan.hpp"
 #include "sort.hpp"
@@ -14,113 +15,29 @@ extern "C" size_t hipcstone_sort_by_key_workspace_size_u32(size_t n);
 namespace hipcstone
 {
 
-// createUnsortedLayout (octree.hpp:77-100): leaf tid is node tid + numInternal of the unsorted layout and, when it
-// and the next leaf share a prefix of whole octal digits, creates internal node (tid + binaryKeyWeight) / 7. Besides
-// the unsorted prefixes, every leaf emits its nodes' levels in creation order: entry 2 tid the internal node's (255
-// when tid creates none), entry 2 tid + 1 its own. Within one level, creation order is key order (keys ascend with
-// tid, and a level holds no node twice), so a stable sort of these entries by level alone gives the level-major,
-// key-ordered node order that sorting the prefixes gives (a level's prefixes are exactly the ones with their
-// placeholder bit at 3 * level).
 template<class K>
 __global__ __launch_bounds__(256) void nodeLevelsKernel(const K* __restrict__ leaves, int32_t numInternal,
                                                         int32_t numLeaves, K* __restrict__ unsortedPrefixes,
-                                                        uint32_t* __restrict__ level, uint32_t* __restrict__ node)
+                                                        uint32_t* __restrict__ level, uint32_t* __restrict__ node,
+                                                        LinkArrays<K> link)
 {
     int32_t tid = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (tid >= numLeaves) return;
-    K key                               = leaves[tid];
-    K next                              = leaves[tid + 1];
-    unsigned leafLevel                  = treeLevel(K(next - key));
-    unsortedPrefixes[tid + numInternal] = encodePlaceholderBit(key, int(3 * leafLevel));
-    level[2 * tid + 1]                  = leafLevel;
-    node[2 * tid + 1]                   = uint32_t(tid + numInternal);
-    unsigned prefixLength               = unsigned(commonPrefix(key, next));
-    if (prefixLength % 3 == 0 && tid < numLeaves - 1)
-    {
-        int32_t octIndex           = (tid + binaryKeyWeight(key, prefixLength / 3)) / 7;
-        unsortedPrefixes[octIndex] = encodePlaceholderBit(key, int(prefixLength));
-        level[2 * tid]             = prefixLength / 3;
-        node[2 * tid]              = uint32_t(octIndex);
-    }
-    else
-    {
-        level[2 * tid] = 255u;
-        node[2 * tid]  = ~0u;
-    }
+    presetLink<K>(tid, link);
+    if (tid < numLeaves) createNodes<K>(tid, leaves, numInternal, numLeaves, unsortedPrefixes, level, node);
 }
 
-// order and level = the first numNodes sorted entries: prefixes[i] = unsorted prefix of node order[i];
-// leafToInternal[order[i]] = i; internalToLeaf[i] = order[i] - numInternal (octree.hpp:176-185); childOffsets[i] = 0 for
-// linkKernel; levelRange (getLevelRangeCpu, octree.hpp:151-160): the first node index of every level from the places
-// where the level changes, levelRange[L + 1] = numNodes
 template<class K>
-__global__ void invertOrderKernel(const uint32_t* __restrict__ order, const uint32_t* __restrict__ level,
-                                  int32_t numNodes, int32_t numInternal, const K* __restrict__ unsortedPrefixes,
-                                  K* __restrict__ prefixes, int32_t* __restrict__ internalToLeaf,
-                                  int32_t* __restrict__ leafToInternal, int32_t* __restrict__ childOffsets,
-                                  int32_t* __restrict__ levelRange)
+__global__ __launch_bounds__(256) void invertOrderKernel(LinkArrays<K> link)
 {
     int32_t i = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= numNodes) return;
-    int32_t o          = int32_t(order[i]);
-    prefixes[i]        = unsortedPrefixes[o];
-    leafToInternal[o]  = i;
-    internalToLeaf[i]  = o - numInternal;
-    childOffsets[i]    = 0;
-    constexpr int L    = int(maxLevel<K>());
-    const int here     = min(int(level[i]), L);
-    const int before   = i > 0 ? int(level[i - 1]) : -1;
-    for (int l = before + 1; l <= here; ++l)
-        levelRange[l] = i;
-    if (i == numNodes - 1)
-    {
-        for (int l = here + 1; l <= L + 1; ++l)
-            levelRange[l] = numNodes;
-    }
+    if (i < link.numNodes) placeNode<K>(i, link);
 }
 
 template<class K>
-__device__ inline int32_t lowerBoundIdx(const K* a, int32_t lo, int32_t hi, K v)
-{
-    int32_t count = hi - lo;
-    while (count > 0)
-    {
-        int32_t step = count / 2;
-        int32_t it   = lo + step;
-        if (a[it] < v)
-        {
-            lo = it + 1;
-            count -= step + 1;
-        }
-        else
-            count = step;
-    }
-    return lo;
-}
-
-// linkTreeCpu (octree.hpp:114-148), childOffsets pre-zeroed (invertOrderKernel)
-template<class K>
-__global__ __launch_bounds__(256) void linkKernel(const K* __restrict__ prefixes, int32_t numInternal,
-                                                  const int32_t* __restrict__ leafToInternal,
-                                                  const int32_t* __restrict__ levelRange,
-                                                  int32_t* __restrict__ childOffsets, int32_t* __restrict__ parents)
+__global__ __launch_bounds__(256) void linkKernel(LinkArrays<K> link)
 {
     int32_t i = int32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= numInternal) return;
-    int32_t idxA          = leafToInternal[i];
-    K prefix              = prefixes[idxA];
-    K nodeKey             = decodePlaceholderBit(prefix);
-    unsigned prefixLength = decodePrefixLength(prefix);
-    unsigned level        = prefixLength / 3;
-    K childPrefix         = encodePlaceholderBit(nodeKey, int(prefixLength) + 3);
-    int32_t lo            = levelRange[level + 1];
-    int32_t hi            = levelRange[level + 2];
-    int32_t childIdx      = lowerBoundIdx(prefixes, lo, hi, childPrefix);
-    if (childIdx != hi && childPrefix == prefixes[childIdx])
-    {
-        childOffsets[idxA]          = childIdx;
-        parents[(childIdx - 1) / 8] = idxA;
-    }
+    if (i < link.numInternal) linkNode<K>(i, link);
 }
 
 // nodeFpCenters + centerAndSize; node keys decoded as Hilbert keys like the reference (sfcKey -> SfcKind)
@@ -189,19 +106,19 @@ static hipcstone_status buildOctree(hipcstone_stream s, const K* leaves, int32_t
     w += a256(E * 4);
     const size_t sortWsBytes = wsBytes - size_t(w - static_cast<char*>(ws));
 
+    const LinkArrays<K> link{order,   level,      unsortedPrefixes, prefixes,       childOffsets,
+                             parents, levelRange, internalToLeaf,   leafToInternal, numNodes,
+                             numInternal};
     nodeLevelsKernel<K><<<ceilDiv(size_t(numLeaves), 256), 256, 0, st>>>(leaves, numInternal, numLeaves,
-                                                                          unsortedPrefixes, keyBuf, valueBuf);
+                                                                          unsortedPrefixes, keyBuf, valueBuf, link);
     HC_CHECK_LAUNCH("nodeLevelsKernel");
     // one 8-bit pass: levels are at most 21, 255 marks the entries without a node (they sort last)
     if (auto e = sortPairsFromBuf(st, keyBuf, valueBuf, E, level, order, w, sortWsBytes, 8)) return e;
-    invertOrderKernel<K><<<ceilDiv(N, 256), 256, 0, st>>>(order, level, numNodes, numInternal, unsortedPrefixes,
-                                                          prefixes, internalToLeaf, leafToInternal, childOffsets,
-                                                          levelRange);
+    invertOrderKernel<K><<<ceilDiv(N, 256), 256, 0, st>>>(link);
     HC_CHECK_LAUNCH("invertOrderKernel");
     if (numInternal > 0)
     {
-        linkKernel<K><<<ceilDiv(size_t(numInternal), 256), 256, 0, st>>>(prefixes, numInternal, leafToInternal,
-                                                                         levelRange, childOffsets, parents);
+        linkKernel<K><<<ceilDiv(size_t(numInternal), 256), 256, 0, st>>>(link);
         HC_CHECK_LAUNCH("linkKernel");
     }
     if (levelRangeHost)

@@ -39,6 +39,36 @@ def test_sort_lookback_give_up_is_reported(hip):
     assert np.array_equal(dv.download(), order.astype(np.uint32))
 
 
+@pytest.mark.parametrize("kd", [np.uint32, np.uint64])
+def test_link_after_a_look_back_give_up_stays_in_the_tree(hip, kd):
+    """The link's one sort pass, given a poll limit of one: whatever the sort leaves behind, every index of the linked
+    tree lies inside it, children come after their parents, and a wrong tree is reported."""
+    levels = 7
+    step = (1 << (63 if kd == np.uint64 else 30)) >> (3 * levels)
+    leaves = (np.arange(8**levels + 1, dtype=np.uint64) * np.uint64(step)).astype(kd)
+    L = leaves.size - 1
+    I = (L - 1) // 7
+    N = L + I
+    print(f"link with look-back poll limit 1, {np.dtype(kd).name}", flush=True)
+    right = hip.build_octree(leaves)
+    hip.set_sort_lookback_limit(1)
+    try:
+        got = hip.build_octree(leaves)
+        faults = hip.device_faults()
+    finally:
+        hip.set_sort_lookback_limit(0)
+    names = ("prefixes", "childOffsets", "parents", "levelRange", "internalToLeaf", "leafToInternal")
+    if not all(np.array_equal(got[k][:I] if k == "parents" else got[k], right[k][:I] if k == "parents" else right[k])
+               for k in names):
+        assert faults & hip.FAULT_SORT_LOOKBACK
+    co, nodes = got["childOffsets"], np.arange(N)
+    assert np.all((co == 0) | ((co > nodes) & (co <= N - 8) & (co % 8 == 1)))
+    assert np.all((got["parents"][:I] >= 0) & (got["parents"][:I] < 8 * np.arange(I) + 1))
+    assert np.all((got["levelRange"] >= 0) & (got["levelRange"] <= N))
+    assert np.all((got["internalToLeaf"] >= -I) & (got["internalToLeaf"] < L))
+    assert np.all((got["leafToInternal"] >= 0) & (got["leafToInternal"] < N))
+
+
 def _flat_tree(T, levels):
     """A 'tree' of 1 + 8 * levels nodes in which all 8 nodes of level k point to the same 8 nodes of level k + 1
     (so the number of root-to-leaf paths is 8^levels), every node box covering the whole unit cube, the last level
