@@ -4,7 +4,8 @@
 // The sort's output is taken as it comes: a look-back that gives up (reported through the fault word, which is read only
 // after these kernels) leaves entries unwritten or written twice. Every step keeps to its arrays for any order and
 // level, and whatever they hold, the results lead no later kernel out of its arrays or round in a circle: indices lie in
-// [0, numNodes), a child block lies in the tree after its parent, and a parent before its children.
+// [0, numNodes), a child block lies in the tree after its parent, a parent before its children, and a node without
+// children has the index of a leaf.
 #pragma once
 
 #include "common.hpp"
@@ -74,7 +75,7 @@ __host__ __device__ inline void createNodes(int32_t t, const Keys& leaves, int32
 }
 
 // Sorted entry i < numNodes: prefixes[i] = unsorted prefix of node order[i]; leafToInternal[order[i]] = i;
-// internalToLeaf[i] = order[i] - numInternal (octree.hpp:176-185); childOffsets[i] = 0 for linkNode; levelRange
+// internalToLeaf[i] = order[i] - numInternal for leaves (octree.hpp:176-185; linkNode does the inner nodes); childOffsets[i] = 0 for linkNode; levelRange
 // (getLevelRangeCpu, octree.hpp:151-160): the first node index of every level from the places where the level changes;
 // the levels after the last one keep numNodes
 template<class K, class Arrays>
@@ -85,7 +86,7 @@ __host__ __device__ inline void placeNode(int32_t i, const Arrays& a)
     const bool known     = o < uint32_t(a.numNodes);
     a.childOffsets[i]    = 0;
     a.prefixes[i]        = known ? a.unsortedPrefixes[o] : K(1); // (the root's)
-    a.internalToLeaf[i]  = known ? int32_t(o) - a.numInternal : 0;
+    a.internalToLeaf[i]  = known && o >= uint32_t(a.numInternal) ? int32_t(o) - a.numInternal : 0;
     if (known) a.leafToInternal[o] = i;
     const uint32_t here = a.level[i] < L ? a.level[i] : L;
     uint32_t from       = 0; // the first level without a place so far
@@ -114,7 +115,8 @@ __host__ __device__ inline int32_t lowerBoundIdx(const Array& a, int32_t lo, int
     return lo;
 }
 
-// Internal node i of the unsorted layout finds its children: linkTreeCpu (octree.hpp:114-148). Blocks of children start
+// Internal node i of the unsorted layout finds its children: linkTreeCpu (octree.hpp:114-148). Only with children does it
+// get its negative internalToLeaf, so a node without any always names a leaf. Blocks of children start
 // at 8 k + 1 (level by level, all nodes but the root come in eights).
 template<class K, class Arrays>
 __host__ __device__ inline void linkNode(int32_t i, const Arrays& a)
@@ -133,6 +135,7 @@ __host__ __device__ inline void linkNode(int32_t i, const Arrays& a)
         childPrefix == a.prefixes[childIdx])
     {
         a.childOffsets[idxA]          = childIdx;
+        a.internalToLeaf[idxA]        = i - a.numInternal;
         a.parents[(childIdx - 1) / 8] = idxA;
     }
 }

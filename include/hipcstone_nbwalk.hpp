@@ -291,8 +291,8 @@ struct Shared
 //   v0, v1, s: the center of child 0, the other center and the size, for x, for the faster of y and z, and for the other
 //   flags:     bit k set if child k is internal; kXFast, kXMiddle: x's pattern (neither: it is the slow axis); kZFaster:
 //              z is faster than y; kGroupValid if every child matched bit for bit (else the walk takes the children's
-//              own centers and sizes); kGroupOutside if an internal child's block lies outside the tree,
-//              kGroupBackward if one does not come after its parent
+//              own centers and sizes); kGroupOutside if an internal child's block lies outside the tree or a leaf
+//              child has no leaf index, kGroupBackward if a block does not come after its parent
 //   link:      a leaf child's leaf index (internalToLeaf), an internal child's own child block (childOffsets)
 template<class T>
 struct alignas(128) ChildGroup
@@ -377,9 +377,10 @@ __global__ void childGroupsKernel(const T* __restrict__ centers, const T* __rest
     {
         const int32_t child = childOffsets[co + k];
         r.link[k]           = child != 0 ? child : internalToLeaf[co + k];
+        if (r.link[k] < 0) flags |= kGroupOutside;
         if (child == 0) continue;
         flags |= 1u << k;
-        if (child < 0 || child > numNodes - 8) flags |= kGroupOutside;
+        if (child > numNodes - 8) flags |= kGroupOutside;
         if (child <= int32_t(co) + k) flags |= kGroupBackward;
     }
     if (same && found) flags |= kGroupValid;

@@ -65,7 +65,7 @@ def test_link_after_a_look_back_give_up_stays_in_the_tree(hip, kd):
     assert np.all((co == 0) | ((co > nodes) & (co <= N - 8) & (co % 8 == 1)))
     assert np.all((got["parents"][:I] >= 0) & (got["parents"][:I] < 8 * np.arange(I) + 1))
     assert np.all((got["levelRange"] >= 0) & (got["levelRange"] <= N))
-    assert np.all((got["internalToLeaf"] >= -I) & (got["internalToLeaf"] < L))
+    assert np.all((got["internalToLeaf"] >= np.where(co == 0, 0, -I)) & (got["internalToLeaf"] < L))
     assert np.all((got["leafToInternal"] >= 0) & (got["leafToInternal"] < N))
 
 
@@ -86,15 +86,7 @@ def _flat_tree(T, levels):
     return N, co, i2l, centers, sizes, layout
 
 
-@pytest.mark.parametrize("case", ["budget", "backward_child"])
-def test_neighbor_walk_guards_are_reported(hip, case):
-    T = np.float32
-    levels = 8
-    N, co, i2l, centers, sizes, layout = _flat_tree(T, levels)
-    expect = hip.FAULT_WALK_BUDGET
-    if case == "backward_child":
-        co[1] = 1  # node 1's children would start at node 1 itself
-        expect = hip.FAULT_MALFORMED_TREE
+def _search_flat_tree(hip, T, N, co, i2l, centers, sizes, layout):
     n = 32
     rng = np.random.default_rng(6)
     x, y, z = (rng.random(n).astype(T) for _ in range(3))
@@ -104,8 +96,31 @@ def test_neighbor_walk_guards_are_reported(hip, case):
     nb = hip.DeviceArray(n * ngmax, np.uint32)
     nc = hip.DeviceArray(n, np.uint32)
     parents = np.zeros(N, np.int32)
-    print(f"neighbor walk on a malformed tree: {case}", flush=True)
     hip.find_neighbors(dev(hip, x), dev(hip, y), dev(hip, z), dev(hip, h), 0, n, box, dev(hip, co), dev(hip, parents),
                        dev(hip, i2l), dev(hip, layout), dev(hip, centers), dev(hip, sizes), N, ngmax, nb, nc)
+
+
+@pytest.mark.parametrize("case", ["budget", "backward_child"])
+def test_neighbor_walk_guards_are_reported(hip, case):
+    T = np.float32
+    levels = 8
+    N, co, i2l, centers, sizes, layout = _flat_tree(T, levels)
+    expect = hip.FAULT_WALK_BUDGET
+    if case == "backward_child":
+        co[1] = 1  # node 1's children would start at node 1 itself
+        expect = hip.FAULT_MALFORMED_TREE
+    print(f"neighbor walk on a malformed tree: {case}", flush=True)
+    _search_flat_tree(hip, T, N, co, i2l, centers, sizes, layout)
     assert hip.device_faults() & expect
     assert hip.device_faults() == 0  # read and cleared
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+def test_node_without_children_or_leaf_is_reported(hip, T):
+    """A node without children whose leaf index is negative (an internal node that lost its children)."""
+    N, co, i2l, centers, sizes, layout = _flat_tree(T, 2)
+    i2l[N - 3] = -5
+    print(f"neighbor walk on a malformed tree: no leaf, {np.dtype(T).name}", flush=True)
+    _search_flat_tree(hip, T, N, co, i2l, centers, sizes, layout)
+    assert hip.device_faults() == hip.FAULT_MALFORMED_TREE
+    assert hip.device_faults() == 0

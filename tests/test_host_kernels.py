@@ -199,7 +199,7 @@ void check(int splits, int numWrong, uint32_t anything, uint32_t seed)
         const int32_t c = a.childOffsets[i];
         need(c == 0 || (c > i && c <= N - 8 && c % 8 == 1), "child block");
         need(a.leafToInternal[i] >= 0 && a.leafToInternal[i] < N, "leafToInternal");
-        need(a.internalToLeaf[i] >= -I && a.internalToLeaf[i] < numLeaves, "internalToLeaf");
+        need(a.internalToLeaf[i] >= (c ? -I : 0) && a.internalToLeaf[i] < numLeaves, "internalToLeaf");
         need(a.prefixes[i] != 0 && decodePrefixLength(a.prefixes[i]) <= 3u * L, "prefix");
         children += c != 0;
         if (numWrong) continue;
