@@ -483,7 +483,7 @@ static hipcstone_status findHalos(hipcstone_stream s, const K* prefixes, const i
     void* owned          = nullptr;
     if (!workspace)
     {
-        HC_CHECK(hipMallocAsync(&owned, lay.bytes, stream(s)));
+        HC_CHECK(deviceMallocAsync(&owned, lay.bytes, stream(s)));
         workspace = owned;
     }
     else if (workspaceBytes < lay.bytes)

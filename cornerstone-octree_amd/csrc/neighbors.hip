@@ -226,7 +226,7 @@ static hipcstone_status findNeighbors(hipcstone_stream s, const T* x, const T* y
         }
         if (allocate)
         {
-            const hipError_t e = hipMallocAsync(&owned, need, stream(s));
+            const hipError_t e = deviceMallocAsync(&owned, need, stream(s));
             if (e != hipSuccess && !optional) return hipFail(e, "findNeighbors: child blocks");
             if (e != hipSuccess)
             {

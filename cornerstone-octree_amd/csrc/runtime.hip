@@ -5,8 +5,6 @@
 
 #include <atomic>
 #include <mutex>
-#include <unordered_map>
-#include <vector>
 
 namespace hipcstone
 {
@@ -95,184 +93,6 @@ hipcstone_status checkFaults(uint32_t faults)
     if (faults & HIPCSTONE_FAULT_CAPACITY) msg += " batched leaf array exceeded its capacity;";
     setError(msg);
     return HIPCSTONE_DEVICE_FAULT;
-}
-
-namespace
-{
-
-struct PoolBlock
-{
-    void* ptr;
-    size_t bytes;
-    int device;
-};
-
-// never destroyed: threads may return memory while the process ends
-struct Pool
-{
-    std::mutex m;
-    std::unordered_map<void*, PoolBlock> taken;
-    std::vector<PoolBlock> kept; // oldest first
-    size_t keptBytes[kMaxDevices] = {};
-    std::vector<hipStream_t> streams[kMaxDevices];
-};
-
-Pool& pool()
-{
-    static Pool* p = new Pool;
-    return *p;
-}
-
-// block sizes are rounded up to steps of at most an eighth, so that blocks of similar sizes serve each other
-size_t poolSize(size_t bytes)
-{
-    size_t step = 4096;
-    while (step * 16 <= bytes)
-        step *= 2;
-    return (bytes + step - 1) / step * step;
-}
-
-thread_local PoolScope* t_scope = nullptr;
-
-} // namespace
-
-hipError_t deviceMalloc(void** ptr, size_t bytes)
-{
-    hipError_t e = hipMalloc(ptr, bytes);
-    if (e == hipSuccess) return e;
-    if (t_scope && !t_scope->freed.empty()) t_scope->flush(false);
-    poolTrim();
-    (void)hipGetLastError();
-    return hipMalloc(ptr, bytes);
-}
-
-hipError_t poolTake(void** ptr, size_t bytes)
-{
-    *ptr       = nullptr;
-    int device = 0;
-    if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
-    if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
-    const size_t size = poolSize(bytes);
-    Pool& p           = pool();
-    {
-        std::lock_guard<std::mutex> lock(p.m);
-        auto best = p.kept.end();
-        for (auto it = p.kept.begin(); it != p.kept.end(); ++it)
-            if (it->device == device && it->bytes >= size && it->bytes <= size + size / 2 &&
-                (best == p.kept.end() || it->bytes < best->bytes))
-                best = it;
-        if (best != p.kept.end())
-        {
-            *ptr           = best->ptr;
-            p.taken[*ptr]  = *best;
-            p.keptBytes[device] -= best->bytes;
-            p.kept.erase(best);
-            return hipSuccess;
-        }
-    }
-    if (hipError_t e = deviceMalloc(ptr, size); e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(p.m);
-    p.taken[*ptr] = PoolBlock{*ptr, size, device};
-    return hipSuccess;
-}
-
-void poolGive(void* ptr, bool idle)
-{
-    if (!ptr) return;
-    Pool& p = pool();
-    std::vector<void*> out;
-    {
-        std::lock_guard<std::mutex> lock(p.m);
-        auto it = p.taken.find(ptr);
-        if (it == p.taken.end()) return;
-        const PoolBlock b = it->second;
-        p.taken.erase(it);
-        if (!idle || b.bytes > kPoolBytes) { out.push_back(b.ptr); }
-        else
-        {
-            p.kept.push_back(b);
-            p.keptBytes[b.device] += b.bytes;
-            for (size_t i = 0; p.keptBytes[b.device] > kPoolBytes; ++i)
-            {
-                if (p.kept[i].device != b.device) continue;
-                p.keptBytes[b.device] -= p.kept[i].bytes;
-                out.push_back(p.kept[i].ptr);
-                p.kept.erase(p.kept.begin() + ptrdiff_t(i--));
-            }
-        }
-    }
-    for (void* o : out)
-        (void)hipFree(o);
-}
-
-void poolTrim()
-{
-    Pool& p = pool();
-    std::vector<PoolBlock> out;
-    {
-        std::lock_guard<std::mutex> lock(p.m);
-        out.swap(p.kept);
-        for (size_t& b : p.keptBytes)
-            b = 0;
-    }
-    for (const PoolBlock& b : out)
-        (void)hipFree(b.ptr);
-}
-
-hipError_t poolTakeStream(hipStream_t* s)
-{
-    int device = 0;
-    if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
-    if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
-    Pool& p = pool();
-    {
-        std::lock_guard<std::mutex> lock(p.m);
-        auto& v = p.streams[device];
-        if (!v.empty())
-        {
-            *s = v.back();
-            v.pop_back();
-            return hipSuccess;
-        }
-    }
-    return hipStreamCreate(s);
-}
-
-void poolGiveStream(hipStream_t s)
-{
-    int device = 0;
-    Pool& p    = pool();
-    if (hipGetDevice(&device) == hipSuccess && device >= 0 && device < kMaxDevices)
-    {
-        std::lock_guard<std::mutex> lock(p.m);
-        if (p.streams[device].size() < kPoolStreams)
-        {
-            p.streams[device].push_back(s);
-            return;
-        }
-    }
-    (void)hipStreamDestroy(s);
-}
-
-PoolScope* poolScope() { return t_scope; }
-
-PoolScope::PoolScope()
-    : outer(t_scope)
-{
-    t_scope = this;
-}
-
-PoolScope::~PoolScope()
-{
-    flush(false);
-    t_scope = outer;
-}
-
-void PoolScope::flush(bool idle)
-{
-    for (void* p : freed)
-        poolGive(p, idle);
-    freed.clear();
 }
 
 static std::atomic<int> g_neighborWaves{4};

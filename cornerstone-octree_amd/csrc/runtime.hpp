@@ -54,8 +54,9 @@ constexpr size_t kPoolBytes = size_t(1) << 30;
 hipError_t poolTake(void** ptr, size_t bytes); // of the current device
 void poolGive(void* ptr, bool idle = true);    // a block of poolTake; not idle: freed
 void poolTrim();
-// hipMalloc, and once more after poolTrim() if it fails
+// hipMalloc and hipMallocAsync, and once more after poolTrim() if there is no memory
 hipError_t deviceMalloc(void** ptr, size_t bytes);
+hipError_t deviceMallocAsync(void** ptr, size_t bytes, hipStream_t s);
 // streams likewise (default priority, idle when returned, at most kPoolStreams kept per device)
 constexpr size_t kPoolStreams = 16;
 hipError_t poolTakeStream(hipStream_t* s);

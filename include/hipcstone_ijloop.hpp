@@ -404,7 +404,7 @@ inline void checkHip(hipError_t e, const char* what)
 
 struct DeviceFree
 {
-    void operator()(void* p) const { (void)hipFree(p); }
+    void operator()(void* p) const { (void)hipcstone_device_free(p); }
 };
 
 } // namespace detail
@@ -423,7 +423,7 @@ public:
     {
         if (ngmax > (1u << 20)) throw std::runtime_error("ijloop: ngmax above 2^20");
         void* p = nullptr;
-        detail::checkHip(hipMalloc(&p, hipcstone::kXcds * sizeof(uint32_t)), "ijloop: group counters");
+        detail::check(hipcstone_device_alloc(&p, hipcstone::kXcds * sizeof(uint32_t)), "ijloop: group counters");
         counters_.reset(static_cast<uint32_t*>(p));
         detail::check(hipcstone_fault_word(&faults_), "ijloop: fault word");
     }
@@ -497,7 +497,7 @@ private:
             records_.reset();
             recordBytes_ = 0;
             void* p      = nullptr;
-            detail::checkHip(hipMalloc(&p, recBytes), "ijloop: record scratch");
+            detail::check(hipcstone_device_alloc(&p, recBytes), "ijloop: record scratch");
             records_.reset(p);
             recordBytes_ = recBytes;
         }
@@ -514,7 +514,8 @@ private:
             if (!childGroups_)
             {
                 void* p = nullptr;
-                detail::checkHip(hipMalloc(&p, numGroups * sizeof(nbwalk::ChildGroup<T>)), "ijloop: child blocks");
+                detail::check(hipcstone_device_alloc(&p, numGroups * sizeof(nbwalk::ChildGroup<T>)),
+                              "ijloop: child blocks");
                 childGroups_.reset(p);
                 childGroupBytes_ = numGroups * sizeof(nbwalk::ChildGroup<T>);
             }
