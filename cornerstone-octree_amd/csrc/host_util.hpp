@@ -35,7 +35,7 @@ struct DeviceBuf
         HC_CHECK(release());
         size_t grown = b + b / 8 + 256;
         pooled       = poolScope() != nullptr;
-        hipError_t e = pooled ? poolTake(&ptr, grown) : deviceMalloc(&ptr, grown);
+        hipError_t e = pooled ? poolTake(&ptr, &grown) : deviceMalloc(&ptr, grown);
         if (e != hipSuccess)
         {
             ptr = nullptr;

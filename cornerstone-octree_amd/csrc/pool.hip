@@ -1,6 +1,7 @@
 // Device memory and streams kept for the next taker (host code only).
 #include "runtime.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -36,7 +37,8 @@ Pool& pool()
     return *p;
 }
 
-// block sizes are rounded up to steps of at most an eighth, so that blocks of similar sizes serve each other
+// Block sizes are rounded up to steps of at most an eighth, so that blocks of similar sizes serve each other. Only blocks
+// of the very size do (blocks up to half larger made neither sorts nor served bursts faster, and hold that much more).
 size_t poolSize(size_t bytes)
 {
     size_t step = 4096;
@@ -76,33 +78,32 @@ hipError_t deviceMallocAsync(void** ptr, size_t bytes, hipStream_t s)
     return allocateOrTrim([&] { return hipMallocAsync(ptr, bytes, s); });
 }
 
-hipError_t poolTake(void** ptr, size_t bytes)
+hipError_t poolTake(void** ptr, size_t* bytes)
 {
     *ptr       = nullptr;
     int device = 0;
     if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
     if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
-    const size_t size = poolSize(bytes);
+    const size_t size = poolSize(*bytes);
     Pool& p           = pool();
     {
         std::lock_guard<std::mutex> lock(p.m);
-        auto best = p.kept.end();
-        for (auto it = p.kept.begin(); it != p.kept.end(); ++it)
-            if (it->device == device && it->bytes >= size && it->bytes <= size + size / 2 &&
-                (best == p.kept.end() || it->bytes < best->bytes))
-                best = it;
-        if (best != p.kept.end())
+        auto it = std::find_if(p.kept.begin(), p.kept.end(),
+                               [&](const PoolBlock& b) { return b.device == device && b.bytes == size; });
+        if (it != p.kept.end())
         {
-            *ptr           = best->ptr;
-            p.taken[*ptr]  = *best;
-            p.keptBytes[device] -= best->bytes;
-            p.kept.erase(best);
+            *ptr          = it->ptr;
+            *bytes        = size;
+            p.taken[*ptr] = *it;
+            p.keptBytes[device] -= size;
+            p.kept.erase(it);
             return hipSuccess;
         }
     }
     if (hipError_t e = deviceMalloc(ptr, size); e != hipSuccess) return e;
     std::lock_guard<std::mutex> lock(p.m);
     p.taken[*ptr] = PoolBlock{*ptr, size, device};
+    *bytes        = size;
     return hipSuccess;
 }
 

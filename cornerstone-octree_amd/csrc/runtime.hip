@@ -219,7 +219,7 @@ hipcstone_status hipcstone_scratch_alloc(void** ptr, size_t bytes)
     if (!ptr) return invalid("ptr");
     *ptr = nullptr;
     if (bytes == 0) return HIPCSTONE_OK;
-    hipError_t e = poolTake(ptr, bytes);
+    hipError_t e = poolTake(ptr, &bytes);
     if (e != hipSuccess)
     {
         *ptr = nullptr;

@@ -51,7 +51,7 @@ uint32_t* pinnedStaging();
 // device are kept (the oldest go first); an allocation of this library that fails gives them all back and tries again,
 // and so does poolTrim(). Safe from several threads.
 constexpr size_t kPoolBytes = size_t(1) << 30;
-hipError_t poolTake(void** ptr, size_t bytes); // of the current device
+hipError_t poolTake(void** ptr, size_t* bytes); // of the current device; at least *bytes, which becomes the block's size
 void poolGive(void* ptr, bool idle = true);    // a block of poolTake; not idle: freed
 void poolTrim();
 // hipMalloc and hipMallocAsync, and once more after poolTrim() if there is no memory

@@ -9,7 +9,9 @@ DEVICE = r"""
 #include <cstdio>
 #include <cstdlib>
 #include <map>
+#include "host_util.hpp"
 #include "pool.hip"
+void hipcstone::setError(const std::string&) {}
 using namespace hipcstone;
 
 static std::map<void*, size_t> g_held;
@@ -53,14 +55,14 @@ static void need(bool ok, const char* what)
 static void* take(size_t n)
 {
     void* p = nullptr;
-    need(poolTake(&p, n) == hipSuccess, "take");
+    need(poolTake(&p, &n) == hipSuccess, "take");
     return p;
 }
 constexpr size_t MB = size_t(1) << 20;
 """
 
 
-@pytest.mark.parametrize("how", ["deviceMalloc(&p, 8 * MB)", "deviceMallocAsync(&p, 8 * MB, nullptr)", "poolTake(&p, 8 * MB)"])
+@pytest.mark.parametrize("how", ["deviceMalloc(&p, 8 * MB)", "deviceMallocAsync(&p, 8 * MB, nullptr)", "poolTake(&p, &size)"])
 def test_allocations_get_the_kept_blocks_back(tmp_path, how):
     """With 10 MB on the device and 6 of them kept, an allocation of 8 MB succeeds, whichever way it is made."""
     run = _run(tmp_path, "trim", DEVICE + r"""
@@ -71,10 +73,80 @@ int main()
     poolGive(a);
     poolGive(b);
     need(g_used >= 6 * MB, "kept");
-    void* p = nullptr;
-    need(%s == hipSuccess && p, "no memory");
+    void* p     = nullptr;
+    size_t size = 8 * MB;
+    need(size && %s == hipSuccess && p, "no memory");
     need(g_held.size() == 1, "the kept blocks are given back");
     return 0;
 }
 """ % how)
+    assert run.returncode == 0, run.stdout + run.stderr
+
+
+def test_buffers_know_what_they_hold(tmp_path):
+    """Buffers that take each other's blocks report what the device holds for them, and that is never much more than was
+    asked for: an eighth of slack of the buffer's own, and the pool's rounding by at most another."""
+    run = _run(tmp_path, "size", DEVICE + r"""
+int main()
+{
+    PoolScope scope;
+    DeviceBuf buf[6];
+    size_t asked[6] = {};
+    unsigned r      = 1;
+    for (int step = 0; step < 4000; ++step)
+    {
+        r              = r * 1664525u + 1013904223u;
+        DeviceBuf& b   = buf[r >> 8 & 3];
+        const size_t n = size_t(1) << (10 + (r >> 12) % 16), more = (r >> 16) % 1000;
+        if (r >> 28 & 1)
+        {
+            DeviceBuf empty;
+            swap(empty, b);
+            asked[&b - buf] = 0;
+        }
+        else if (n + n * more / 1000 > asked[&b - buf])
+        {
+            asked[&b - buf] = n + n * more / 1000;
+            need(b.reserve(asked[&b - buf]) == HIPCSTONE_OK, "reserve");
+        }
+        scope.flush();
+        size_t held = 0;
+        for (DeviceBuf& o : buf)
+        {
+            const size_t n = asked[&o - buf];
+            need(o.bytes >= n && (!o.ptr || g_held[o.ptr] == o.bytes), "a buffer does not know its size");
+            // (what it was asked for last may be less than what it once grew to: then bytes stay)
+            held += o.bytes;
+        }
+        need(held <= g_used, "more than the device holds");
+    }
+    // a block that was kept is not handed out for less than it was made for
+    for (DeviceBuf& o : buf)
+    {
+        DeviceBuf empty;
+        swap(empty, o);
+    }
+    scope.flush();
+    poolTrim();
+    for (int k = 0; k < 64; ++k)
+    {
+        const size_t big = (50 + k) * MB, small = 40 * MB;
+        need(buf[0].reserve(big) == HIPCSTONE_OK, "reserve");
+        {
+            DeviceBuf empty;
+            swap(empty, buf[0]);
+        }
+        scope.flush();
+        need(buf[1].reserve(small) == HIPCSTONE_OK, "reserve");
+        need(g_held[buf[1].ptr] <= small + small / 4 + small / 32, "a block much larger than asked for");
+        {
+            DeviceBuf empty;
+            swap(empty, buf[1]);
+        }
+        scope.flush();
+        poolTrim();
+    }
+    return 0;
+}
+""")
     assert run.returncode == 0, run.stdout + run.stderr
