@@ -56,7 +56,11 @@ private:
     {
         hipError_t e = hipSuccess;
         if (!ptr) return e;
-        if (!pooled) e = hipFree(ptr);
+        if (!pooled)
+        {
+            // (refused, as while a stream is captured: the buffer keeps its memory)
+            if (e = hipFree(ptr); e != hipSuccess) return e;
+        }
         else if (poolScope()) poolScope()->freed.push_back(ptr);
         else poolGive(ptr, false);
         ptr   = nullptr;

@@ -27,6 +27,7 @@ struct Pool
     std::mutex m;
     std::unordered_map<void*, PoolBlock> taken;
     std::vector<PoolBlock> kept; // oldest first
+    std::vector<PoolBlock> late; // to be freed: hipFree was refused (as while a stream is captured)
     size_t keptBytes[kMaxDevices] = {};
     std::vector<hipStream_t> streams[kMaxDevices];
 };
@@ -49,10 +50,23 @@ size_t poolSize(size_t bytes)
 
 thread_local PoolScope* t_scope = nullptr;
 
-} // namespace
-
-namespace
+// frees the blocks, and the late ones with them; those that are refused (again) wait
+void freeBlocks(std::vector<PoolBlock>& blocks)
 {
+    Pool& p = pool();
+    {
+        std::lock_guard<std::mutex> lock(p.m);
+        blocks.insert(blocks.end(), p.late.begin(), p.late.end());
+        p.late.clear();
+    }
+    for (const PoolBlock& b : blocks)
+    {
+        if (hipFree(b.ptr) == hipSuccess) continue;
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> lock(p.m);
+        p.late.push_back(b);
+    }
+}
 
 // once more with all kept blocks given back, where there was no memory
 template<class Allocate>
@@ -111,14 +125,14 @@ void poolGive(void* ptr, bool idle)
 {
     if (!ptr) return;
     Pool& p = pool();
-    std::vector<void*> out;
+    std::vector<PoolBlock> out;
     {
         std::lock_guard<std::mutex> lock(p.m);
         auto it = p.taken.find(ptr);
         if (it == p.taken.end()) return;
         const PoolBlock b = it->second;
         p.taken.erase(it);
-        if (!idle || b.bytes > kPoolBytes) { out.push_back(b.ptr); }
+        if (!idle || b.bytes > kPoolBytes) { out.push_back(b); }
         else
         {
             p.kept.push_back(b);
@@ -127,13 +141,12 @@ void poolGive(void* ptr, bool idle)
             {
                 if (p.kept[i].device != b.device) continue;
                 p.keptBytes[b.device] -= p.kept[i].bytes;
-                out.push_back(p.kept[i].ptr);
+                out.push_back(p.kept[i]);
                 p.kept.erase(p.kept.begin() + ptrdiff_t(i--));
             }
         }
     }
-    for (void* o : out)
-        (void)hipFree(o);
+    if (!out.empty()) freeBlocks(out);
 }
 
 void poolTrim()
@@ -146,8 +159,7 @@ void poolTrim()
         for (size_t& b : p.keptBytes)
             b = 0;
     }
-    for (const PoolBlock& b : out)
-        (void)hipFree(b.ptr);
+    freeBlocks(out);
 }
 
 hipError_t poolTakeStream(hipStream_t* s)

@@ -173,11 +173,17 @@ class DeviceArray:
 
 class _Scratch:
     """Device memory of one call, from the library's kept blocks. free() it only when the device is done with it; an
-    object that is dropped instead (an error on the way) waits for the device first."""
+    object that is dropped instead (an error on the way) waits for the device first, or leaves its block to the next one
+    where waiting is refused (while a stream is captured)."""
+
+    _late = []
 
     def __init__(self, nbytes):
         self.nbytes = int(nbytes)
         self._ptr = C.c_void_p()
+        if _Scratch._late and _lib.hipcstone_device_sync() == 0:
+            while _Scratch._late:
+                _lib.hipcstone_scratch_free(_Scratch._late.pop())
         _check(_lib.hipcstone_scratch_alloc(C.byref(self._ptr), C.c_size_t(max(self.nbytes, 1))), "scratch_alloc")
 
     def free(self):
@@ -187,8 +193,11 @@ class _Scratch:
 
     def __del__(self):
         try:
-            if self._ptr.value and _lib.hipcstone_device_sync() == 0:
-                self.free()
+            if self._ptr.value:
+                if _lib.hipcstone_device_sync() == 0:
+                    self.free()
+                else:
+                    _Scratch._late.append(self._ptr)
         except Exception:
             pass
 

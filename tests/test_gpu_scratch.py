@@ -85,3 +85,27 @@ def test_sorts_through_kept_blocks(hip):
         order = np.argsort(keys, kind="stable")
         assert np.array_equal(p.download(), order) and np.array_equal(k.download(), keys[order])
         assert all(np.array_equal(a.download(), b[order]) for a, b in zip(o, x))
+
+
+def test_a_sort_refused_while_capturing_loses_no_memory(hip):
+    """sort_gather synchronizes, which a capture refuses: it raises, nothing runs, and its blocks serve the next call."""
+    rng = np.random.RandomState(4)
+    n = 5000
+    keys = rng.randint(0, 1 << 28, n).astype(np.uint32)
+    x = [hip.DeviceArray.from_numpy(rng.rand(n).astype(np.float32)) for _ in range(4)]
+    o = [hip.DeviceArray(n, np.float32) for _ in range(4)]
+    k, p = hip.DeviceArray.from_numpy(keys), hip.DeviceArray(n, np.uint32)
+    hip.sort_gather(k, p, *x, *o)
+    order = p.download()
+    k.upload(keys)
+    s, graph = hip.Stream(), C.c_void_p()
+    for _ in range(3):
+        print("sort while capturing", flush=True)
+        assert hip._lib.hipStreamBeginCapture(C.c_void_p(s.handle), 0) == 0
+        with pytest.raises(hip.HipcstoneError):
+            hip.sort_gather(k, p, *x, *o, stream=s)
+        if hip._lib.hipStreamEndCapture(C.c_void_p(s.handle), C.byref(graph)) == 0 and graph.value:
+            assert hip._lib.hipGraphDestroy(graph) == 0
+        hip._lib.hipGetLastError()
+    hip.sort_gather(k, p, *x, *o)
+    assert np.array_equal(p.download(), order) and not hip._Scratch._late

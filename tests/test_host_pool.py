@@ -150,3 +150,31 @@ int main()
 }
 """)
     assert run.returncode == 0, run.stdout + run.stderr
+
+
+def test_memory_outlives_a_refused_free(tmp_path):
+    """Where hipFree is refused (while a stream is captured) nothing is lost: blocks are freed at the next chance, a
+    buffer keeps its memory, and an allocation that is refused too does not give the kept blocks away."""
+    run = _run(tmp_path, "refused", DEVICE + r"""
+int main()
+{
+    void *a = take(MB), *b = take(2 * MB), *c = take(4 * MB), *p = nullptr;
+    DeviceBuf buf;
+    need(buf.reserve(MB) == HIPCSTONE_OK, "reserve");
+    void* before = buf.ptr;
+    const size_t bytes = buf.bytes;
+    poolGive(a);
+    poolGive(b);
+    g_refused = true;
+    need(deviceMalloc(&p, MB) == hipErrorStreamCaptureUnsupported, "refused allocation");
+    poolGive(c, false);
+    need(buf.reserve(8 * MB) != HIPCSTONE_OK && buf.ptr == before && buf.bytes == bytes, "buffer without its memory");
+    g_refused = false;
+    need(g_held.size() == 4, "held");
+    need(take(MB) == a, "the kept blocks are still kept");
+    poolTrim();
+    need(g_held.size() == 2 && g_held.count(a) && g_held.count(before), "everything else is freed");
+    return 0;
+}
+""")
+    assert run.returncode == 0, run.stdout + run.stderr
