@@ -202,6 +202,12 @@ class _Scratch:
             pass
 
 
+def scratch_trim():
+    """Gives the device memory that the library keeps for later calls (sorts, served bursts) back to the driver, for
+    other users of the device; the library's own allocations do so themselves where there is no memory."""
+    _check(_lib.hipcstone_scratch_trim(), "scratch_trim")
+
+
 def download_ptr(ptr, count, dtype, stream=None):
     dt = np.dtype(dtype)
     out = np.empty(int(count), dtype=dt)

@@ -4,6 +4,7 @@ kept blocks give the same as the first."""
 
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -85,6 +86,27 @@ def test_sorts_through_kept_blocks(hip):
         order = np.argsort(keys, kind="stable")
         assert np.array_equal(p.download(), order) and np.array_equal(k.download(), keys[order])
         assert all(np.array_equal(a.download(), b[order]) for a, b in zip(o, x))
+
+
+def test_a_program_gets_the_kept_memory_back(hip):
+    """What a sort leaves in the library's keeping is free for others after scratch_trim()."""
+    n = 4_000_000
+    k, p = hip.DeviceArray(n, np.uint32), hip.DeviceArray(n, np.uint32)
+    k.upload(np.random.RandomState(7).randint(0, 1 << 30, n).astype(np.uint32))
+    x, o = ([hip.DeviceArray(n, np.float32) for _ in range(4)] for _ in range(2))
+    for d in x:
+        d.upload(np.zeros(n, np.float32))
+    hip.sort_gather(k, p, *x, *o)  # (the runtime's own memory for kernels of this size stays)
+    hip.scratch_trim()
+    before = _free_bytes(hip)
+    hip.sort_gather(k, p, *x, *o)
+    assert before - _free_bytes(hip) > 100 * MB
+    hip.scratch_trim()
+    for _ in range(100):  # (the driver counts memory that was just in use as free a little later)
+        if before - _free_bytes(hip) <= 64 * MB:
+            break
+        time.sleep(0.02)
+    assert before - _free_bytes(hip) <= 64 * MB
 
 
 def test_a_sort_refused_while_capturing_loses_no_memory(hip):
