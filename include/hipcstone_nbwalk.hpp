@@ -35,10 +35,13 @@
  * with u = 2^-24, a = |x_i|, r = 2 h_i and S = 2 a + r, a pair with D near 0 has |x_j| <= a + r, so the roundings of
  * the relative coordinates (2 u r S), of |x_j|^2 and |x_i|^2 (7 u S^2), of the four accumulations (each of at most
  * (a + |x_j|)^2 + r^2 <= S^2 + r^2, counted with a whole ulp) and of the reference's distance (5 u r^2) stay below
- * 16 u (S^2 + r^2); pairs farther away have D > |x_j|^2 / 4, far above their error. E is that bound at the wave's
- * largest target. A chunk with a |D| < E (about one wave in five has one at 100 neighbors) tests the 16-candidate
- * groups it occurs in again, in the reference's own operations; if E is not a normal number (coordinates or h out of
- * fp32's range) every chunk is. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
+ * 16 u (S^2 + r^2). E is 1e-6 (S^2 + r^2), more by 0.7 u S^2. A pair with |x_j| = a + r + d, d > 0, has D >= d^2 and an
+ * error that is larger by at most 44 u S d + 22 u d^2: less than both together, so it never comes out at -E or below. E is
+ * taken at the wave's largest target. A chunk with a |D| < E (about one wave in five has one at 100 neighbors) tests the
+ * 16-candidate groups it occurs in again, in the reference's own operations. fp64 lengths are first multiplied by one
+ * power of two for the whole wave, so the products do not depend on the unit of length; only waves whose largest length
+ * is beyond 2^-48 to 2^60 (fp32, where the reference's own squares near the ends of the range) or 2^-100 to 2^101 (fp64)
+ * have every chunk tested again. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
  * A wave with a target whose 2h box leaves a periodic domain folds its candidates to their images nearest to c. While
  * S < L / 2 these are the reference's images for every pair that can be a hit, and the folded differences are off by at
  * most 2 u L per dimension, the reference's included, so E grows by 8 u r L; with a larger S every chunk is tested in
@@ -138,6 +141,15 @@ constexpr int kSpills       = 3;
 // lane, with more waves the latencies hide better: 16 chunks at 2 waves per SIMD took 13.0 ms, 10 at 3 9.9, 8 at 4 8.4.
 constexpr int kChunks  = 5;
 constexpr int kEntries = 13;
+
+// Exponents of a wave's largest relative coordinate or radius for which the products decide: while the reference's own
+// squares stay well inside fp32's range, and while an fp64 length as a float does. Squares of lengths below all of
+// these are below kFarSq.
+template<class T>
+constexpr int kMinExponent = std::is_same_v<T, float> ? -48 : -100;
+template<class T>
+constexpr int kMaxExponent = std::is_same_v<T, float> ? 59 : 100;
+constexpr float kFarSq     = 1.0e38f;
 
 typedef float Float4 __attribute__((ext_vector_type(4)));
 
@@ -263,6 +275,7 @@ struct WaveShared
     uint32_t spilled[kSpills][3][kSpillEntries]; // stack entries that did not fit the registers
     uint32_t marks[kWave];                       // scratch of one chunk
     uint32_t cand[(kChunks + 1) * kWave];        // the kept chunks' candidates (particle indices), and the next one's
+    float unit;                                  // fp64: the wave's unit of length in the products
     uint32_t entries[kEntries + 1][kWave];       // column l: target l's kept hits (see HitReader), then one without any
 };
 
@@ -546,39 +559,61 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
     float errBound;
     bool allExact;
     [[maybe_unused]] bool images = false; // some target's neighbors are looked for across a periodic face
+    [[maybe_unused]] const uint32_t unitAt = ldsAddress(&sh.unit);
+    // fp64: what lengths are multiplied by for the products, a power of two that brings the largest to [1, 2)
+    [[maybe_unused]] float unit = 1.0f;
+    auto inUnits                = [&](float length) {
+        if constexpr (std::is_same_v<T, float>) { return length; }
+        else { return length * unit; }
+    };
     {
-        const float xr  = inRoot ? float(xi - cx) : 0.0f;
-        const float yr  = inRoot ? float(yi - cy) : 0.0f;
-        const float zr  = inRoot ? float(zi - cz) : 0.0f;
+        float xr        = inRoot ? float(xi - cx) : 0.0f;
+        float yr        = inRoot ? float(yi - cy) : 0.0f;
+        float zr        = inRoot ? float(zi - cz) : 0.0f;
+        const float big = fmaxf(fmaxf(fabsf(xr), fabsf(yr)), fmaxf(fabsf(zr), inRoot ? fabsf(float(T(2) * hi)) : 0.0f));
+        // (non-negative floats order as their bit patterns)
+        const int exponent = int(readLane(waveScanMax(__float_as_uint(big)), kWave - 1) >> 23) - 127;
+        allExact           = exponent < kMinExponent<T> || exponent > kMaxExponent<T>;
+        if constexpr (!std::is_same_v<T, float>)
+        {
+            // (read back for each chunk: a register that holds it all along costs fp64 2 to 4 %)
+            unit    = __uint_as_float(uint32_t(127 - exponent) << 23);
+            ldsWrite(unitAt, __float_as_uint(unit));
+        }
+        xr                 = inUnits(xr);
+        yr                 = inUnits(yr);
+        zr                 = inUnits(zr);
         const float a2  = xr * xr + yr * yr + zr * zr;
-        const float r2  = inRoot ? float(radiusSq0) : 0.0f;
+        float r2        = 0.0f;
+        if constexpr (std::is_same_v<T, float>) { r2 = inRoot ? radiusSq0 : 0.0f; }
+        else { r2 = inRoot ? float(radiusSq0 * T(unit) * T(unit)) : 0.0f; }
         const float s   = 2.0f * __builtin_amdgcn_sqrtf(a2) + __builtin_amdgcn_sqrtf(r2);
         const float s2r = inRoot ? s * s + r2 : 0.0f;
-        // (non-negative floats order as their bit patterns; a NaN's is above infinity's)
-        const float most = __uint_as_float(readLane(waveScanMax(__float_as_uint(s2r) & 0x7FFFFFFFu), kWave - 1));
+        const float most = __uint_as_float(readLane(waveScanMax(__float_as_uint(s2r)), kWave - 1));
         errBound         = readLane(1.0e-6f * most, 0); // 16 u (S^2 + r^2), rounded up
-        allExact         = !(errBound >= 1.0e-30f && errBound <= 1.0e20f);
+        allExact         = allExact || !(most < kFarSq); // (a coordinate that is not a number)
         if constexpr (AnyPbc)
         {
             images = ballot(px | py | pz) != 0;
             if (images)
             {
-                const float mostR2 = __uint_as_float(readLane(waveScanMax(__float_as_uint(r2) & 0x7FFFFFFFu), kWave - 1));
+                const float mostR2 = __uint_as_float(readLane(waveScanMax(__float_as_uint(r2)), kWave - 1));
                 float longest      = 0.0f;
                 for (int d = 0; d < 3; ++d)
                 {
                     if (box.bnd[d] != HIPCSTONE_PERIODIC) continue;
-                    longest  = fmaxf(longest, float(box.len[d]));
-                    allExact = allExact || !(sqrtf(most) < 0.4999f * float(box.len[d]));
+                    const float len = inUnits(float(box.len[d]));
+                    longest         = fmaxf(longest, len);
+                    allExact        = allExact || !(sqrtf(most) < 0.4999f * len);
                 }
                 // (u of the coordinates' own type: fp64 ones are folded in fp64)
                 constexpr float kFold = std::is_same_v<T, float> ? 5.0e-7f : 1.0e-15f;
                 errBound = readLane(errBound + kFold * sqrtf(mostR2) * longest, 0);
-                allExact = allExact || !(errBound <= 1.0e20f);
+                allExact = allExact || !(errBound <= 1.0e-6f * kFarSq);
             }
         }
         float c0[4];
-        c0[0] = c0[1] = c0[2] = c0[3] = inRoot ? a2 - r2 : 1.0e30f;
+        c0[0] = c0[1] = c0[2] = c0[3] = inRoot ? a2 - r2 : kFarSq;
         transposeRows(c0);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
@@ -756,11 +791,12 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
                                   (bz && !(zj >= box.lim[4] && zj <= box.lim[5]));
                     }
                 }
-                cnd[0]          = float(dx);
-                cnd[1]          = float(dy);
-                cnd[2]          = float(dz);
+                if constexpr (!std::is_same_v<T, float>) { unit = __uint_as_float(Lds::read(unitAt)); }
+                cnd[0]          = inUnits(float(dx));
+                cnd[1]          = inUnits(float(dy));
+                cnd[2]          = inUnits(float(dz));
                 cnd[3]          = __builtin_fmaf(cnd[2], cnd[2], __builtin_fmaf(cnd[1], cnd[1], cnd[0] * cnd[0]));
-                const bool far  = !(cnd[3] < 1.0e30f); // or not a number
+                const bool far  = !(cnd[3] < kFarSq); // or not a number
                 transposeRows(cnd);
                 float least = std::numeric_limits<float>::max();
                 auto tile   = [&](uint32_t bits, int t) __attribute__((always_inline)) -> uint32_t {

@@ -112,7 +112,10 @@ def test_deep_tree_with_everything_in_reach(hip, oracle, T):
 
 
 @pytest.mark.parametrize("T,scale", [(np.float32, 1e-17), (np.float32, 1e-12), (np.float32, 1e12), (np.float32, 3e18),
-                                     (np.float64, 1e-40), (np.float64, 1e-12), (np.float64, 1e12), (np.float64, 1e40)])
+                                     (np.float64, 1e-40), (np.float64, 1e-12), (np.float64, 1e12), (np.float64, 1e40),
+                                     # both sides of where the products' power of two ends
+                                     (np.float32, 2e-14), (np.float32, 1e-13), (np.float32, 2e18), (np.float32, 8e18),
+                                     (np.float64, 3e-30), (np.float64, 3e-29), (np.float64, 3e30), (np.float64, 3e31)])
 def test_magnitudes(hip, oracle, T, scale):
     """Coordinates and radii whose squares leave fp32's range, or come near its ends, and a box far from the origin."""
     rng = np.random.default_rng(9)
@@ -166,3 +169,38 @@ def test_periodic_radii(hip, oracle, T, radius, boundary):
     p["x"][out[:10]] -= T(0.02)
     p["y"][out[10:]] += T(1.03)
     _check(hip, oracle, p, 0.0, 1.0, 150, boundary=boundary, ext=1.1)
+
+
+@pytest.mark.parametrize("T,scales", [(np.float32, (1e-12, 1e15)), (np.float64, (1e-20, 1e21))])
+def test_unit_of_length_leaves_rows_and_times(hip, T, scales):
+    """The same particles in other units of length (powers of two): the same rows, in at most half more time."""
+    rng = np.random.default_rng(21)
+    n, ngmax = 300_000, 128
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    h = np.full(n, 0.5 * (80 / (4.19 * n)) ** (1 / 3), T)
+
+    def search(unit):
+        d = [hip.DeviceArray.from_numpy((a * T(unit)).astype(T)) for a in (x, y, z, h)]
+        box = hip.make_box(0.0, float(unit), T)
+        pipe = hip.Pipeline(curve=HILBERT, key_bits=64, real_bits=8 * np.dtype(T).itemsize, bucket_size=64, ngmax=0)
+        pipe.sync(*d, n, box, full_build=True)
+        v = pipe.view()
+        nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
+        nb.upload(np.zeros(n * ngmax, np.uint32))
+        times = []
+        for _ in range(6):
+            a, b = hip.Event(), hip.Event()
+            a.record()
+            hip.find_neighbors(v.x, v.y, v.z, v.h, 0, n, box, v.child_offsets, v.parents, v.internal_to_leaf, v.layout,
+                               v.centers, v.sizes, v.num_nodes, ngmax, nb, nc)
+            b.record()
+            hip.device_sync()
+            times.append(a.elapsed_ms(b))
+        return nb.download(), nc.download(), min(times)
+
+    nb, nc, ms = search(1.0)
+    for s in scales:
+        print(f"unit of length {s:g}", flush=True)
+        nb2, nc2, ms2 = search(2.0 ** round(np.log2(s)))
+        assert np.array_equal(nc, nc2) and np.array_equal(nb, nb2)
+        assert ms2 < 1.5 * ms, (ms, ms2)
