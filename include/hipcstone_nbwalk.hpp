@@ -41,12 +41,12 @@
  * 16-candidate groups it occurs in again, in the reference's own operations. fp64 lengths are first multiplied by one
  * power of two for the whole wave, so the products do not depend on the unit of length; only waves whose largest length
  * is beyond 2^-48 to 2^60 (fp32, where the reference's own squares near the ends of the range) or 2^-100 to 2^101 (fp64)
- * have every chunk tested again. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
+ * do without the products and test each target against a chunk's 64 candidates at once. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
  * A wave with a target whose 2h box leaves a periodic domain folds its candidates to their images nearest to c. While
  * S < L / 2 these are the reference's images for every pair that can be a hit, and the folded differences are off by at
- * most 2 u L per dimension, the reference's included, so E grows by 8 u r L; with a larger S every chunk is tested in
- * the reference's operations, and so is a chunk with a particle outside the domain (the reference folds only for
- * targets near its faces).
+ * most 2 u L per dimension, the reference's included, so E grows by 8 u r L; with a larger S the wave does without the
+ * products, and a chunk with a particle outside the domain is tested again (the reference folds only for targets near
+ * its faces).
  *
  * What bounds it is instruction issue: a wave of 64 targets with 100 neighbors takes 12.1K vector, 7.1K scalar and
  * 2.6K branch instructions, and 322 matrix products, which replace some 90K multiply-adds and compares by lane. Pair
@@ -625,8 +625,9 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
         transposeRows(tgt);
     }
     // the candidate (of a chunk of 64) whose position this lane loads: with rows 4 g + r of the q-th product being
-    // candidates 16 g + 4 q + r, the 16 results a lane gets for one target are 16 consecutive candidates
-    const int loadPos = 16 * ((lane & 15) >> 2) + 4 * (lane >> 4) + (lane & 3);
+    // candidates 16 g + 4 q + r, the 16 results a lane gets for one target are 16 consecutive candidates; in their order
+    // where the products are not used
+    const int loadPos = allExact ? lane : 16 * ((lane & 15) >> 2) + 4 * (lane >> 4) + (lane & 3);
     // byte selector that joins the even rows' low or the odd rows' high halves of two words
     const uint32_t halfSel = (lane & 16) ? 0x07060302u : 0x05040100u;
 
@@ -772,85 +773,113 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
                 }
                 const uint64_t active = ballot((seenLo | seenHi) != 0);
 
-                // D of 4 x 16 candidates and 4 x 16 targets: per 16 targets four products, whose signs are shifted
-                // into one word (bit s of its half: candidate 16 (lane / 16) + s)
-                float cnd[4];
-                T dx = xj - cx, dy = yj - cy, dz = zj - cz;
-                bool outside = false;
-                if constexpr (AnyPbc)
+                uint32_t lo = 0, hw = 0;
+                // (where the compiler places this costs: as unlikely 0.5 % less at 16.8M in open boxes, 1.2 % more in the
+                // segmented walk and 15 % more in periodic fp64 steps)
+                if (__builtin_expect(allExact, AnyPbc || Segmented ? allExact : 0))
                 {
-                    if (images)
+                    // target by target against the chunk's 64 candidates (in their order, see loadPos), in the
+                    // reference's operations
+                    const T hAgain       = valid ? h[i] : T(0);
+                    const T radiusSq     = T(4.0) * hAgain * hAgain;
+                    const uint64_t folds = AnyPbc ? ballot(px | py | pz) : 0;
+                    for (uint64_t rest = active; rest != 0; rest &= rest - 1)
                     {
-                        const bool bx = box.bnd[0] == HIPCSTONE_PERIODIC, by = box.bnd[1] == HIPCSTONE_PERIODIC,
-                                   bz = box.bnd[2] == HIPCSTONE_PERIODIC;
-                        dx      = fold(dx, bx, 0);
-                        dy      = fold(dy, by, 1);
-                        dz      = fold(dz, bz, 2);
-                        outside = (bx && !(xj >= box.lim[0] && xj <= box.lim[1])) ||
-                                  (by && !(yj >= box.lim[2] && yj <= box.lim[3])) ||
-                                  (bz && !(zj >= box.lim[4] && zj <= box.lim[5]));
+                        const int t = __builtin_ctzll(rest);
+                        T ax = xj - readLane(xi, t), ay = yj - readLane(yi, t), az = zj - readLane(zi, t);
+                        if (AnyPbc && (folds >> t & 1))
+                        {
+                            ax = fold(ax, box.bnd[0] == HIPCSTONE_PERIODIC, 0);
+                            ay = fold(ay, box.bnd[1] == HIPCSTONE_PERIODIC, 1);
+                            az = fold(az, box.bnd[2] == HIPCSTONE_PERIODIC, 2);
+                        }
+                        const uint64_t hits = ballot(ax * ax + ay * ay + az * az < readLane(radiusSq, t));
+                        lo                  = writeLane(lo, t, uint32_t(hits));
+                        hw                  = writeLane(hw, t, uint32_t(hits >> 32));
                     }
                 }
-                if constexpr (!std::is_same_v<T, float>) { unit = __uint_as_float(Lds::read(unitAt)); }
-                cnd[0]          = inUnits(float(dx));
-                cnd[1]          = inUnits(float(dy));
-                cnd[2]          = inUnits(float(dz));
-                cnd[3]          = __builtin_fmaf(cnd[2], cnd[2], __builtin_fmaf(cnd[1], cnd[1], cnd[0] * cnd[0]));
-                const bool far  = !(cnd[3] < kFarSq); // or not a number
-                transposeRows(cnd);
-                float least = std::numeric_limits<float>::max();
-                auto tile   = [&](uint32_t bits, int t) __attribute__((always_inline)) -> uint32_t {
-                    if ((uint32_t(active >> (16 * t)) & 0xFFFFu) == 0) return bits << 16;
-                    Float4 d[4];
-#pragma unroll
-                    for (int q = 3; q >= 0; --q)
-                        d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(cnd[q], tgt[t], tgtConst[t], 0, 0, 0);
-#pragma unroll
-                    for (int q = 3; q >= 0; --q)
-                    {
-#pragma unroll
-                        for (int r = 3; r >= 0; --r)
-                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[q][r]), 31);
-                        least = fminf(fminf(least, fabsf(d[q][0])), fabsf(d[q][1]));
-                        least = fminf(fminf(least, fabsf(d[q][2])), fabsf(d[q][3]));
-                    }
-                    return bits;
-                };
-                uint32_t b01 = 0, b23 = 0;
-                b01 = tile(b01, 1);
-                b01 = tile(b01, 0);
-                b23 = tile(b23, 3);
-                b23 = tile(b23, 2);
-                // row k of a lane's targets gets its 16 bits from all four rows: candidates [0, 32) and [32, 64)
-                swapHalves(b01, b23);
-                uint32_t o01 = b01, o23 = b23;
-                swapRows(b01, o01);
-                swapRows(b23, o23);
-                uint32_t lo = __builtin_amdgcn_perm(o01, b01, halfSel);
-                uint32_t hw = __builtin_amdgcn_perm(o23, b23, halfSel);
-
-                uint64_t unsure = ballot(least < errBound);
-                if (allExact || ballot(far || outside) != 0) unsure = ~uint64_t(0);
-                if (unsure != 0)
+                else
                 {
-                    // the 16-candidate groups with a pair too close to call, in the reference's operations
-                    const T hAgain   = valid ? h[i] : T(0);
-                    const T radiusSq = T(4.0) * hAgain * hAgain;
-#pragma unroll 1
-                    for (int g = 0; g < 4; ++g)
+                    // D of 4 x 16 candidates and 4 x 16 targets: per 16 targets four products, whose signs are shifted
+                    // into one word (bit s of its half: candidate 16 (lane / 16) + s)
+                    float cnd[4];
+                    T dx = xj - cx, dy = yj - cy, dz = zj - cz;
+                    bool outside = false;
+                    if constexpr (AnyPbc)
                     {
-                        if ((uint32_t(unsure >> (16 * g)) & 0xFFFFu) == 0) continue;
-                        uint32_t bits = 0;
-#pragma unroll 1
-                        for (int s = 0; s < 16; ++s)
+                        if (images)
                         {
-                            const int from = 16 * (s >> 2) + 4 * g + (s & 3);
-                            bits |= uint32_t(close(readLane(xj, from), readLane(yj, from), readLane(zj, from), radiusSq))
-                                    << s;
+                            const bool bx = box.bnd[0] == HIPCSTONE_PERIODIC, by = box.bnd[1] == HIPCSTONE_PERIODIC,
+                                       bz = box.bnd[2] == HIPCSTONE_PERIODIC;
+                            dx      = fold(dx, bx, 0);
+                            dy      = fold(dy, by, 1);
+                            dz      = fold(dz, bz, 2);
+                            outside = (bx && !(xj >= box.lim[0] && xj <= box.lim[1])) ||
+                                      (by && !(yj >= box.lim[2] && yj <= box.lim[3])) ||
+                                      (bz && !(zj >= box.lim[4] && zj <= box.lim[5]));
                         }
-                        const uint32_t shift = 16u * (g & 1);
-                        uint32_t& word       = g < 2 ? lo : hw;
-                        word                 = (word & ~(0xFFFFu << shift)) | (bits << shift);
+                    }
+                    if constexpr (!std::is_same_v<T, float>) { unit = __uint_as_float(Lds::read(unitAt)); }
+                    cnd[0]          = inUnits(float(dx));
+                    cnd[1]          = inUnits(float(dy));
+                    cnd[2]          = inUnits(float(dz));
+                    cnd[3]          = __builtin_fmaf(cnd[2], cnd[2], __builtin_fmaf(cnd[1], cnd[1], cnd[0] * cnd[0]));
+                    const bool far  = !(cnd[3] < kFarSq); // or not a number
+                    transposeRows(cnd);
+                    float least = std::numeric_limits<float>::max();
+                    auto tile   = [&](uint32_t bits, int t) __attribute__((always_inline)) -> uint32_t {
+                        if ((uint32_t(active >> (16 * t)) & 0xFFFFu) == 0) return bits << 16;
+                        Float4 d[4];
+#pragma unroll
+                        for (int q = 3; q >= 0; --q)
+                            d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(cnd[q], tgt[t], tgtConst[t], 0, 0, 0);
+#pragma unroll
+                        for (int q = 3; q >= 0; --q)
+                        {
+#pragma unroll
+                            for (int r = 3; r >= 0; --r)
+                                bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[q][r]), 31);
+                            least = fminf(fminf(least, fabsf(d[q][0])), fabsf(d[q][1]));
+                            least = fminf(fminf(least, fabsf(d[q][2])), fabsf(d[q][3]));
+                        }
+                        return bits;
+                    };
+                    uint32_t b01 = 0, b23 = 0;
+                    b01 = tile(b01, 1);
+                    b01 = tile(b01, 0);
+                    b23 = tile(b23, 3);
+                    b23 = tile(b23, 2);
+                    // row k of a lane's targets gets its 16 bits from all four rows: candidates [0, 32) and [32, 64)
+                    swapHalves(b01, b23);
+                    uint32_t o01 = b01, o23 = b23;
+                    swapRows(b01, o01);
+                    swapRows(b23, o23);
+                    lo = __builtin_amdgcn_perm(o01, b01, halfSel);
+                    hw = __builtin_amdgcn_perm(o23, b23, halfSel);
+
+                    uint64_t unsure = ballot(least < errBound);
+                    if (ballot(far || outside) != 0) unsure = ~uint64_t(0);
+                    if (unsure != 0)
+                    {
+                        // the 16-candidate groups with a pair too close to call, in the reference's operations
+                        const T hAgain   = valid ? h[i] : T(0);
+                        const T radiusSq = T(4.0) * hAgain * hAgain;
+#pragma unroll 1
+                        for (int g = 0; g < 4; ++g)
+                        {
+                            if ((uint32_t(unsure >> (16 * g)) & 0xFFFFu) == 0) continue;
+                            uint32_t bits = 0;
+#pragma unroll 1
+                            for (int s = 0; s < 16; ++s)
+                            {
+                                const int from = 16 * (s >> 2) + 4 * g + (s & 3);
+                                bits |= uint32_t(close(readLane(xj, from), readLane(yj, from), readLane(zj, from), radiusSq))
+                                        << s;
+                            }
+                            const uint32_t shift = 16u * (g & 1);
+                            uint32_t& word       = g < 2 ? lo : hw;
+                            word                 = (word & ~(0xFFFFu << shift)) | (bits << shift);
+                        }
                     }
                 }
                 lo &= seenLo;

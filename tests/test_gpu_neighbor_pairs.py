@@ -171,6 +171,42 @@ def test_periodic_radii(hip, oracle, T, radius, boundary):
     _check(hip, oracle, p, 0.0, 1.0, 150, boundary=boundary, ext=1.1)
 
 
+def _timed_search(hip, T, particles, lo, hi, ngmax, boundary=(0, 0, 0), repeats=6):
+    """Rows, counts and the least time of a search over the particles (in the order of their keys)."""
+    d = [hip.DeviceArray.from_numpy(a) for a in particles]
+    n = d[0].count
+    box = hip.make_box(lo, hi, T, boundary)
+    pipe = hip.Pipeline(curve=HILBERT, key_bits=64, real_bits=8 * np.dtype(T).itemsize, bucket_size=64, ngmax=0)
+    pipe.sync(*d, n, box, full_build=True)
+    v = pipe.view()
+    nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
+    nb.upload(np.zeros(n * ngmax, np.uint32))
+    times = []
+    for _ in range(repeats):
+        a, b = hip.Event(), hip.Event()
+        a.record()
+        hip.find_neighbors(v.x, v.y, v.z, v.h, 0, n, box, v.child_offsets, v.parents, v.internal_to_leaf, v.layout,
+                           v.centers, v.sizes, v.num_nodes, ngmax, nb, nc)
+        b.record()
+        hip.device_sync()
+        times.append(a.elapsed_ms(b))
+    return nb.download(), nc.download(), min(times)
+
+
+@pytest.mark.parametrize("T", TS)
+def test_small_periodic_box_is_not_slow(hip, T):
+    """1000 particles whose search radius is 0.29 of the box: periodic images are looked for across a range as large as
+    the box. That takes at most twice the time of the open box."""
+    rng = np.random.default_rng(23)
+    n = 1000
+    p = [rng.random(n).astype(T) for _ in range(3)] + [np.full(n, 0.144, T)]
+    _, _, ms = _timed_search(hip, T, p, 0.0, 1.0, 150, repeats=20)
+    print("periodic", flush=True)
+    _, counts, ms2 = _timed_search(hip, T, p, 0.0, 1.0, 150, boundary=(1, 1, 1), repeats=20)
+    assert counts.min() > 60
+    assert ms2 < 2 * ms, (ms, ms2)
+
+
 @pytest.mark.parametrize("T,scales", [(np.float32, (1e-12, 1e15)), (np.float64, (1e-20, 1e21))])
 def test_unit_of_length_leaves_rows_and_times(hip, T, scales):
     """The same particles in other units of length (powers of two): the same rows, in at most half more time."""
@@ -180,23 +216,7 @@ def test_unit_of_length_leaves_rows_and_times(hip, T, scales):
     h = np.full(n, 0.5 * (80 / (4.19 * n)) ** (1 / 3), T)
 
     def search(unit):
-        d = [hip.DeviceArray.from_numpy((a * T(unit)).astype(T)) for a in (x, y, z, h)]
-        box = hip.make_box(0.0, float(unit), T)
-        pipe = hip.Pipeline(curve=HILBERT, key_bits=64, real_bits=8 * np.dtype(T).itemsize, bucket_size=64, ngmax=0)
-        pipe.sync(*d, n, box, full_build=True)
-        v = pipe.view()
-        nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
-        nb.upload(np.zeros(n * ngmax, np.uint32))
-        times = []
-        for _ in range(6):
-            a, b = hip.Event(), hip.Event()
-            a.record()
-            hip.find_neighbors(v.x, v.y, v.z, v.h, 0, n, box, v.child_offsets, v.parents, v.internal_to_leaf, v.layout,
-                               v.centers, v.sizes, v.num_nodes, ngmax, nb, nc)
-            b.record()
-            hip.device_sync()
-            times.append(a.elapsed_ms(b))
-        return nb.download(), nc.download(), min(times)
+        return _timed_search(hip, T, [(a * T(unit)).astype(T) for a in (x, y, z, h)], 0.0, float(unit), ngmax)
 
     nb, nc, ms = search(1.0)
     for s in scales:
