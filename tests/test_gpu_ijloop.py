@@ -56,11 +56,26 @@ def test_ijloop_example_gpu(hip, oracle, T, bnd, ngmax, first, last, ext):
     assert want[1][first:last].min() >= 1 and want[1][first:last].max() >= min(ngmax + 1, 9)
 
 
-def test_ijloop_example_gpu_chunked(hip, oracle):
-    """ngmax = 65536: a wave's scratch slice is 16 MiB, so the 2 GiB scratch cap leaves 128 waves, and each wave
-    walks and folds several of the 469 groups of 64 bodies."""
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("bnd", [(0, 0, 0), (1, 1, 1)])
+def test_ijloop_example_gpu_many_groups(hip, oracle, T, bnd):
+    """25000 groups of 64 bodies, three for each of the 8192 waves that the device holds at most: every wave walks and
+    folds several, one after the other, in the same memory."""
+    n, ngmax = 1_600_000, 24
+    print(f"ijloop many groups {np.dtype(T).name} bnd {bnd}", flush=True)
+    p, obox, m = _case(oracle, T, n, bnd, seed=15)
+    tree = {k: p[k] for k in ("childOffsets", "parents", "internalToLeaf")}
+    want = oracle.ijloop_example(p["x"], p["y"], p["z"], p["h"], m, 0, n, obox, tree, p["layout"], p["centers"],
+                                 p["sizes"], ngmax)
+    got = _gpu(hip, p, T, bnd, m, 0, n, ngmax)
+    for name, g, w in zip(("rho", "count", "dmin", "dmax", "fx"), got, want):
+        assert np.array_equal(g, w), name
+
+
+def test_ijloop_example_gpu_large_ngmax(hip, oracle):
+    """ngmax = 65536, far above every count: no memory is set aside for it, and nothing is cut."""
     T = np.float32
-    print("ijloop chunked", flush=True)
+    print("ijloop large ngmax", flush=True)
     p, obox, m = _case(oracle, T, 30000, (0, 0, 0), seed=13)
     tree = {k: p[k] for k in ("childOffsets", "parents", "internalToLeaf")}
     want = oracle.ijloop_example(p["x"], p["y"], p["z"], p["h"], m, 0, 30000, obox, tree, p["layout"], p["centers"],
