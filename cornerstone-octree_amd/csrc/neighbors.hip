@@ -218,12 +218,7 @@ static hipcstone_status findNeighbors(hipcstone_stream s, const T* x, const T* y
         const bool optional      = kOptional || anyPbc;
         void* dst                = groupsWs && groupsWsBytes >= need ? groupsWs : nullptr;
         bool allocate            = !dst;
-        if (allocate && optional)
-        {
-            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-            HC_CHECK(hipStreamIsCapturing(stream(s), &capturing));
-            allocate = capturing == hipStreamCaptureStatusNone;
-        }
+        if (allocate && optional) allocate = mayAllocate(stream(s));
         if (allocate)
         {
             const hipError_t e = deviceMallocAsync(&owned, need, stream(s));

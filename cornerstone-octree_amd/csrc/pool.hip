@@ -92,6 +92,14 @@ hipError_t deviceMallocAsync(void** ptr, size_t bytes, hipStream_t s)
     return allocateOrTrim([&] { return hipMallocAsync(ptr, bytes, s); });
 }
 
+bool mayAllocate(hipStream_t s)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) == hipSuccess) return status == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 hipError_t poolTake(void** ptr, size_t* bytes)
 {
     *ptr       = nullptr;

@@ -57,6 +57,8 @@ void poolTrim();
 // hipMalloc and hipMallocAsync, and once more after poolTrim() if there is no memory
 hipError_t deviceMalloc(void** ptr, size_t bytes);
 hipError_t deviceMallocAsync(void** ptr, size_t bytes, hipStream_t s);
+// not while the stream is captured, nor where that is not told (the null stream, while any blocking stream is)
+bool mayAllocate(hipStream_t s);
 // streams likewise (default priority, idle when returned, at most kPoolStreams kept per device)
 constexpr size_t kPoolStreams = 16;
 hipError_t poolTakeStream(hipStream_t* s);

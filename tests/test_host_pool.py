@@ -41,6 +41,13 @@ extern "C" hipError_t hipFree(void* p)
     ++g_frees;
     return hipSuccess;
 }
+static hipError_t g_query = hipSuccess;
+static hipStreamCaptureStatus g_status = hipStreamCaptureStatusNone;
+extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
+{
+    *s = g_status;
+    return g_query;
+}
 extern "C" hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 extern "C" hipError_t hipGetLastError() { return hipSuccess; }
 extern "C" hipError_t hipStreamCreate(hipStream_t*) { return hipErrorUnknown; }
@@ -174,6 +181,24 @@ int main()
     need(take(MB) == a, "the kept blocks are still kept");
     poolTrim();
     need(g_held.size() == 2 && g_held.count(a) && g_held.count(before), "everything else is freed");
+    return 0;
+}
+""")
+    assert run.returncode == 0, run.stdout + run.stderr
+
+
+def test_no_allocation_where_a_capture_may_run(tmp_path):
+    """Searches that can do without memory of their own take none while their stream is captured, nor where the runtime
+    does not tell (it refuses the question for the null stream while another stream is captured); that is no error."""
+    run = _run(tmp_path, "capture", DEVICE + r"""
+int main()
+{
+    need(mayAllocate(nullptr), "no capture");
+    g_status = hipStreamCaptureStatusActive;
+    need(!mayAllocate(nullptr), "captured");
+    g_status = hipStreamCaptureStatusNone;
+    g_query  = hipErrorStreamCaptureImplicit;
+    need(!mayAllocate(nullptr), "not told");
     return 0;
 }
 """)
