@@ -24,13 +24,14 @@ namespace hipcstone
 // targetsPerWave: 64, or fewer where that many waves would leave the device idle (kFullWaves).
 //
 // Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a sixth busy): the walk takes
-// 2.25 of 6.25 ms, the chunks' set-up 1.05, the pair tests 1.45, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
+// 2.25 of 6.2 ms, the chunks' set-up 1.0, the pair tests 1.45, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
 // search of that size took 7.65 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
-// instructions a wave, now 24.6K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.98 ms.
+// instructions a wave, now 24.9K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.95 ms.
 
-// Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.66 ms, 6 waves 6.31, 7 waves 7.1 (registers go
-// to memory; 16.8M targets). fp64, 300k uniform targets open / periodic: 4 waves 235 / 379 us, 5 waves 213 / 329, 6 waves
-// 224 / 387; 2M open: 975, 934, 1046 (30k, which do not fill the device: 82, 85, 92).
+// Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.53 ms, 6 waves 6.20, where 5 vector registers go
+// to memory, none of them in the inner loops (16.8M targets); the LDS holds no seventh wave. fp64, 300k uniform targets
+// open / periodic: 4 waves 232 / 283 us, 5 waves 211 / 254, 6 waves 222 / 272; 2M open: 977, 949, 1040 (30k, which do not
+// fill the device: 80, 83, 88). At 5 fp64 spills 4 or 5 vector registers, and in periodic boxes 49 to 58 scalar ones.
 template<class T>
 constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> ? 6 : 5;
 

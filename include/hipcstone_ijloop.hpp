@@ -306,8 +306,9 @@ __global__ void zeroCountersKernel(uint32_t* counters)
  * each lane takes its own body's (the first ngmax, ascending j) and folds them in order; the postamble result is stored
  * after the walk. Bodies outside the subgroups take no part.
  * The walk bounds it. Lists kept in registers and LDS instead of a per-wave scratch save the rows' way to memory and
- * back and, per neighborhood, the allocation of that scratch (64 * ngmax slots for every resident wave, 197 MB):
- * build and loop over 1M uniform bodies, 40 neighbors, fp32: 12.3 -> 0.95 ms, most of it the allocation.
+ * back and, per neighborhood, the allocation of that scratch (64 * ngmax slots for every resident wave, 262 MB at ngmax
+ * 200). 1M uniform bodies, 100 neighbors, ngmax 200, fp32: the kernel 1.12 -> 0.87 ms, with the neighborhood's
+ * allocations 12.4 -> 0.94. 16.8M bodies, ngmax 150: the kernel 14.0 -> 10.5 ms.
  */
 template<bool AnyPbc, class T, class InTuple, class OutTuple, class Interaction, class Postamble>
 __global__ __launch_bounds__(kFusedWaves * 64) void fusedIjLoopKernel(
