@@ -20,7 +20,7 @@
  * The neighbor search and the fold run in one kernel, instantiated here, in the caller's translation unit, for the
  * caller's interaction and postamble (device-callable functors or lambdas), as the reference's GPU loop folds each
  * warp's lists right after that warp's traversal (gpu_alwaystraverse.cuh:32-91): a persistent grid of waves takes
- * groups of 64 consecutive bodies; each wave walks the tree for its group with the library's own walk
+ * groups of up to 64 consecutive bodies; each wave walks the tree for its group with the library's own walk
  * (hipcstone_nbwalk.hpp), which hands every lane its own body's next neighbors, in list order, and the lane folds them
  * right away: no list is written to memory. x, y, z, h of all totalBodies bodies are also staged as one
  * record per body at each ijLoop, so a neighbor's position and h come in one wide load (the values are copies, the
@@ -299,8 +299,8 @@ __global__ void zeroCountersKernel(uint32_t* counters)
 }
 
 /*
- * The fused always-traverse loop. Bodies [first, last) form groups of 64; the groups are split into 8 contiguous
- * ranges, one per XCD (workgroups are dealt to the XCDs round-robin, so workgroup b runs on XCD b % 8 and neighbouring
+ * The fused always-traverse loop. Bodies [first, last) form groups of groupSize (up to 64); the groups are split into 8
+ * contiguous ranges, one per XCD (workgroups are dealt to the XCDs round-robin, so workgroup b runs on XCD b % 8 and neighbouring
  * groups share tree nodes and particles in that XCD's L2). Each wave takes the next group of its XCD's range from
  * counters[xcd] and, when that range is exhausted, helps with the next XCD's. Per group: as the walk finds neighbors,
  * each lane takes its own body's (the first ngmax, ascending j) and folds them in order; the postamble result is stored
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fusedIjLoopKernel(
     int32_t numNodes, float ext, const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z,
     const T* __restrict__ h, const Record<T>* __restrict__ rec, InTuple input, OutTuple output,
     Interaction interaction, Postamble postamble, unsigned ngmax, LocalIndex first, LocalIndex last,
-    GroupView groups, uint32_t* __restrict__ counters,
+    uint32_t groupSize, GroupView groups, uint32_t* __restrict__ counters,
     uint32_t* __restrict__ faults, const nbwalk::ChildGroup<T>* __restrict__ childGroups)
 {
     using namespace hipcstone;
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fusedIjLoopKernel(
     __shared__ nbwalk::Shared<T, kFusedWaves> sh;
     const int w             = uniform(int(threadIdx.x) / kWave);
     const int lane          = laneId();
-    const uint32_t numGrp   = uint32_t((uint64_t(last) - first + kWave - 1) / kWave);
+    const uint32_t numGrp   = uint32_t((uint64_t(last) - first + groupSize - 1) / groupSize);
     const uint32_t xcd      = blockIdx.x % kXcds;
 
     for (uint32_t r = 0; r < kXcds; ++r)
@@ -342,9 +342,9 @@ __global__ __launch_bounds__(kFusedWaves * 64) void fusedIjLoopKernel(
             if (lane == 0) g = atomicAdd(&counters[part], 1u);
             g = uniform(g);
             if (g >= ge - gb) break;
-            const uint64_t gFirst = uint64_t(first) + uint64_t(gb + g) * kWave;
+            const uint64_t gFirst = uint64_t(first) + uint64_t(gb + g) * groupSize;
             const LocalIndex i    = LocalIndex(gFirst) + LocalIndex(lane);
-            const bool valid      = i < last && inGroups(groups, i);
+            const bool valid      = i < last && uint32_t(lane) < groupSize && inGroups(groups, i);
             if (ballot(valid) == 0) continue;
 
             // the self term first, then the neighbors in list order as the walk hands them on: kFoldBatch at a time,
@@ -482,15 +482,19 @@ private:
         constexpr int kThreads = detail::kFusedWaves * 64;
         auto kernel = &detail::fusedIjLoopKernel<AnyPbc, T, InTuple, OutTuple, Interaction, Postamble>;
         // a persistent grid: as many workgroups as fit on the device at once (whole rounds over the 8 XCDs), and no more
-        // than the groups of 64 bodies need
+        // than the groups of bodies need
         int device = 0, cus = 0, perCu = 0;
         detail::checkHip(hipGetDevice(&device), "ijloop: device");
         detail::checkHip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device), "ijloop: CUs");
         detail::checkHip(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, kernel, kThreads, 0),
                          "ijloop: occupancy");
-        const std::size_t groups64  = (std::size_t(last - first) + 63) / 64;
+        // Few bodies in a periodic box: their search radii come near half of it, and there the walk takes one body of a
+        // wave after the other. Groups of 16 / 64 (us, neighborhood included, 60 to 100 neighbors, fp32; fp64 alike): 1000
+        // bodies 132 / 214, 2000 112 / 202, 4000 231 / 286, 8000 214 / 281, 20000 213 / 220, 60000 448 / 372.
+        const uint32_t groupSize    = AnyPbc && last - first < 16384 ? 16 : 64;
+        const std::size_t numGrp    = (std::size_t(last - first) + groupSize - 1) / groupSize;
         std::size_t blocks          = std::size_t(std::max(perCu, 1)) * std::size_t(std::max(cus, 1));
-        blocks = std::min(blocks, (groups64 + detail::kFusedWaves - 1) / detail::kFusedWaves);
+        blocks = std::min(blocks, (numGrp + detail::kFusedWaves - 1) / detail::kFusedWaves);
         if (blocks > hipcstone::kXcds) blocks = blocks / hipcstone::kXcds * hipcstone::kXcds;
         const std::size_t recBytes = std::max<std::size_t>(total_, 1) * sizeof(detail::Record<T>);
         if (recBytes > recordBytes_)
@@ -530,7 +534,7 @@ private:
         kernel<<<unsigned(blocks), kThreads, 0, stream_>>>(
             box_, tree_.childOffsets, tree_.internalToLeaf, tree_.layout, reinterpret_cast<const T*>(tree_.centers),
             reinterpret_cast<const T*>(tree_.sizes), tree_.numNodes, tree_.searchExtFactor, x_, y_, z_, h_,
-            rec, input, output, interaction, postamble, ngmax_, first, last, groups,
+            rec, input, output, interaction, postamble, ngmax_, first, last, groupSize, groups,
             counters_.get(), faults_, childGroups);
         detail::checkHip(hipGetLastError(), "ijloop: fused search and interaction kernel");
     }

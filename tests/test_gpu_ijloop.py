@@ -72,6 +72,48 @@ def test_ijloop_example_gpu_many_groups(hip, oracle, T, bnd):
         assert np.array_equal(g, w), name
 
 
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("first,last", [(0, 1), (5, 21), (3, 20), (0, 300), (100, 16483), (100, 16484), (100, 16485)])
+def test_ijloop_example_gpu_periodic_groups(hip, oracle, T, first, last):
+    """Periodic loops around the sizes of a group and of the range that takes smaller groups."""
+    n, bnd, ngmax = max(last + 7, 320), (1, 1, 1), 40
+    print(f"ijloop periodic groups {np.dtype(T).name} [{first},{last})", flush=True)
+    p, obox, m = _case(oracle, T, n, bnd, seed=16)
+    tree = {k: p[k] for k in ("childOffsets", "parents", "internalToLeaf")}
+    want = oracle.ijloop_example(p["x"], p["y"], p["z"], p["h"], m, first, last, obox, tree, p["layout"],
+                                 p["centers"], p["sizes"], ngmax)
+    got = _gpu(hip, p, T, bnd, m, first, last, ngmax)
+    for name, g, w in zip(("rho", "count", "dmin", "dmax", "fx"), got, want):
+        assert np.array_equal(g, w), name
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+def test_small_periodic_ijloop_is_not_slow(hip, oracle, T):
+    """2000 bodies with 60 neighbors: a periodic box takes at most 1.8 times the time of an open one."""
+    import time
+
+    rng = np.random.default_rng(17)
+    n = 2000
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    h = np.full(n, 0.5 * (60 / (4.19 * n)) ** (1 / 3), T)
+    ms = {}
+    for bnd in ((0, 0, 0), (1, 1, 1)):
+        print(f"ijloop time {np.dtype(T).name} {bnd}", flush=True)
+        p = cpu_pipeline(oracle, x, y, z, h, orc_box(0.0, 1.0, T, bnd), np.uint64, 64, HILBERT)
+        d = {k: dev(hip, p[k]) for k in ("x", "y", "z", "h", "childOffsets", "parents", "internalToLeaf", "layout")}
+        dc, ds, m = dev(hip, p["centers"].reshape(-1)), dev(hip, p["sizes"].reshape(-1)), dev(hip, p["x"])
+        outs = [hip.DeviceArray(n, t) for t in (T, np.uint32, T, T, T)]
+        times = []
+        for _ in range(30):
+            t = time.perf_counter()
+            hip.ijloop_example(d["x"], d["y"], d["z"], d["h"], m, 0, n, hip.make_box(0.0, 1.0, T, bnd), d["childOffsets"],
+                               d["parents"], d["internalToLeaf"], d["layout"], dc, ds, p["prefixes"].size, 100, *outs)
+            hip.device_sync()
+            times.append(time.perf_counter() - t)
+        ms[bnd] = min(times)
+    assert ms[(1, 1, 1)] < 1.8 * ms[(0, 0, 0)], ms
+
+
 def test_ijloop_example_gpu_large_ngmax(hip, oracle):
     """ngmax = 65536, far above every count: no memory is set aside for it, and nothing is cut."""
     T = np.float32
