@@ -11,7 +11,7 @@
 namespace hipcstone
 {
 
-// SlotMajor: the wave's 64 rows are stored slot-major (neighbor k of the wave's lane l at k * 64 + l) instead of
+// SlotMajor: the rows of 64 targets are stored slot-major (neighbor k of the l-th of them at k * 64 + l) instead of
 // row-major (l * ngmax + k), so that a consumer with one thread per target reads each slot with one coalesced load.
 // Segmented: many independent trees in one set of arrays (the batched clouds). Wave `group` then takes its targets
 // [first, last) (at most 64, inside one cloud) and the index of its cloud's root node from the wave table
@@ -74,9 +74,10 @@ void findNeighborsKernel(
     }
     const uint32_t i = uint32_t(first) + uint32_t(lane);
     const bool valid = i < lastId && uint32_t(lane) < targetsPerWave;
-    // the wave's rows: row-major, or slot-major (then a wave has 64 targets)
-    const size_t rowBase   = Segmented ? size_t(first) : size_t(first) - firstId;
-    uint32_t* rows         = neighbors + (ngmax ? rowBase * ngmax : 0);
+    // the wave's rows: row-major, or slot-major in their group of 64 (which holds whole waves)
+    const size_t row = Segmented ? size_t(first) : size_t(first) - firstId;
+    uint32_t* rows   = neighbors;
+    if (ngmax) rows += SlotMajor ? row / kWave * kWave * ngmax + row % kWave : row * ngmax;
     const nbwalk::Tree<T> tree{childOffsets, internalToLeaf, layout, centers, sizes, numNodes, ext, groups};
     const uint32_t count = nbwalk::walk<T, AnyPbc, Segmented, kNbWaves>(
         x, y, z, h, box, tree, root, first, valid, ngmax != 0, sh, w, faults,
@@ -202,7 +203,7 @@ static hipcstone_status findNeighbors(hipcstone_stream s, const T* x, const T* y
     if (ngmax > 0 && !neighbors) return invalid("findNeighbors: neighbors is null with ngmax > 0");
     if (ngmax > (1u << 20)) return invalid("findNeighbors: ngmax above 2^20");
     if (numNodes <= 0) return invalid("findNeighbors: numNodes must be positive");
-    const uint32_t perWave  = slotMajor ? uint32_t(kWave) : targetsPerWave(lastId - firstId);
+    const uint32_t perWave  = targetsPerWave(lastId - firstId);
     const size_t waveGroups = (size_t(lastId - firstId) + perWave - 1) / perWave;
     uint32_t* faults = faultWord();
     if (!faults) return HIPCSTONE_HIP_ERROR;

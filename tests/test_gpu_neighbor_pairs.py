@@ -171,7 +171,7 @@ def test_periodic_radii(hip, oracle, T, radius, boundary):
     _check(hip, oracle, p, 0.0, 1.0, 150, boundary=boundary, ext=1.1)
 
 
-def _timed_search(hip, T, particles, lo, hi, ngmax, boundary=(0, 0, 0), repeats=6):
+def _timed_search(hip, T, particles, lo, hi, ngmax, boundary=(0, 0, 0), repeats=6, slot_major=False):
     """Rows, counts and the least time of a search over the particles (in the order of their keys)."""
     d = [hip.DeviceArray.from_numpy(a) for a in particles]
     n = d[0].count
@@ -179,14 +179,15 @@ def _timed_search(hip, T, particles, lo, hi, ngmax, boundary=(0, 0, 0), repeats=
     pipe = hip.Pipeline(curve=HILBERT, key_bits=64, real_bits=8 * np.dtype(T).itemsize, bucket_size=64, ngmax=0)
     pipe.sync(*d, n, box, full_build=True)
     v = pipe.view()
-    nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
-    nb.upload(np.zeros(n * ngmax, np.uint32))
+    size = (n + 63) // 64 * 64 * ngmax
+    nb, nc = hip.DeviceArray(size, np.uint32), hip.DeviceArray(n, np.uint32)
+    nb.upload(np.zeros(size, np.uint32))
     times = []
     for _ in range(repeats):
         a, b = hip.Event(), hip.Event()
         a.record()
         hip.find_neighbors(v.x, v.y, v.z, v.h, 0, n, box, v.child_offsets, v.parents, v.internal_to_leaf, v.layout,
-                           v.centers, v.sizes, v.num_nodes, ngmax, nb, nc)
+                           v.centers, v.sizes, v.num_nodes, ngmax, nb, nc, slot_major=slot_major)
         b.record()
         hip.device_sync()
         times.append(a.elapsed_ms(b))
@@ -224,3 +225,45 @@ def test_unit_of_length_leaves_rows_and_times(hip, T, scales):
         nb2, nc2, ms2 = search(2.0 ** round(np.log2(s)))
         assert np.array_equal(nc, nc2) and np.array_equal(nb, nb2)
         assert ms2 < 1.5 * ms, (ms, ms2)
+
+
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("boundary", [(0, 0, 0), (1, 1, 1)])
+@pytest.mark.parametrize("n,first,last", [(1, 0, 1), (65, 0, 65), (70, 3, 66), (1000, 1, 999), (16500, 0, 16383),
+                                          (16500, 7, 16391), (33000, 0, 32769), (70000, 5, 65599), (131200, 0, 131071),
+                                          (131200, 3, 131075)])
+def test_slot_major_rows(hip, oracle, T, boundary, n, first, last):
+    """Slot-major rows in waves of 4 to 64 targets, against the row-major ones; no other word is written."""
+    print(f"slot-major {np.dtype(T).name} [{first},{last}) {boundary}", flush=True)
+    rng = np.random.default_rng(n)
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    h = np.full(n, 0.5 * (25 / (4.19 * max(n, 100))) ** (1 / 3), T)
+    p = _tree(oracle, x, y, z, h, 0.0, 1.0, 32, boundary=boundary)
+    gbox = hip.make_box(0.0, 1.0, T, boundary)
+    ngmax, m = 22, last - first
+    rows, counts = _search(hip, p, gbox, first, last, ngmax)
+    d = {k: hip.DeviceArray.from_numpy(np.ascontiguousarray(p[k]).reshape(-1))
+         for k in ("x", "y", "z", "h", "childOffsets", "parents", "internalToLeaf", "layout", "centers", "sizes")}
+    groups = (m + 63) // 64
+    nb, nc = hip.DeviceArray(groups * 64 * ngmax, np.uint32), hip.DeviceArray(m, np.uint32)
+    nb.fill(0xFF)
+    hip.find_neighbors(d["x"], d["y"], d["z"], d["h"], first, last, gbox, d["childOffsets"], d["parents"],
+                       d["internalToLeaf"], d["layout"], d["centers"], d["sizes"], p["prefixes"].size, ngmax, nb, nc,
+                       slot_major=True)
+    assert np.array_equal(nc.download(), counts)
+    got = nb.download().reshape(groups, ngmax, 64).transpose(0, 2, 1).reshape(groups * 64, ngmax)
+    held = np.arange(ngmax)[None, :] < np.minimum(counts, ngmax)[:, None]
+    assert np.array_equal(got[:m], np.where(held, rows, np.uint32(0xFFFFFFFF)))
+    assert np.all(got[m:] == np.uint32(0xFFFFFFFF))
+
+
+@pytest.mark.parametrize("T", TS)
+def test_small_slot_major_search_is_not_slow(hip, T):
+    """Slot-major rows of a small periodic search take at most half more time than row-major ones."""
+    rng = np.random.default_rng(29)
+    n = 2000
+    p = [rng.random(n).astype(T) for _ in range(3)] + [np.full(n, 0.0965, T)]
+    _, _, ms = _timed_search(hip, T, p, 0.0, 1.0, 100, boundary=(1, 1, 1), repeats=20)
+    print("slot-major", flush=True)
+    _, _, ms2 = _timed_search(hip, T, p, 0.0, 1.0, 100, boundary=(1, 1, 1), repeats=20, slot_major=True)
+    assert ms2 < 1.5 * ms, (ms, ms2)
