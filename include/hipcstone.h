@@ -447,10 +447,9 @@ HIPCSTONE_DECL_NEIGHBORS(f64, double)
 
 /* ---- the same search with the neighbor rows stored slot-major per group of 64 bodies: for body i, r = i - first_id,
  * neighbor k is at neighbors[((r / 64) * ngmax + k) * 64 + r % 64]; neighbors must hold ceil((last_id - first_id) /
- * 64) * 64 * ngmax elements. No reference counterpart: it is the scratch layout of the ijloop consumer
- * (hipcstone_ijloop.hpp), whose one-thread-per-body fold reads one slot of 64 bodies per coalesced load, like the
- * per-warp column layout of the reference's GpuAlwaysTraverseNeighborhood (gpu_alwaystraverse.cuh:47-75). Counts
- * are exact up to 2^26 neighbors per body. ---- */
+ * 64) * 64 * ngmax elements. No reference counterpart: it is for consumers with one thread per body, which read one slot
+ * of 64 bodies per coalesced load, like the per-warp column layout of the reference's GpuAlwaysTraverseNeighborhood
+ * (gpu_alwaystraverse.cuh:47-75). Counts are exact up to 2^26 neighbors per body. ---- */
 #define HIPCSTONE_DECL_NEIGHBORS_SLOT_MAJOR(RS, T)                                                                     \
     hipcstone_status hipcstone_find_neighbors_slot_major_##RS(                                                         \
         hipcstone_stream s, const T* x, const T* y, const T* z, const T* h, uint32_t first_id, uint32_t last_id,      \

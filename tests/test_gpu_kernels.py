@@ -275,15 +275,16 @@ def test_find_neighbors(hip, oracle, T, kd):
         assert neighbor_rows_equal(nb, nc, ref_nb, ref_nc, ngmax)
 
 
-def test_find_neighbors_mixed_child_geometry(hip, oracle):
-    """fp32 open-box searches read each block of 8 children in a compact form (two center values and one size per
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("boundary", [(0, 0, 0), (1, 1, 0)])
+def test_find_neighbors_mixed_child_geometry(hip, oracle, T, boundary):
+    """Searches read each block of 8 children in a compact form (two center values and one size per
     dimension) and fall back to the children's own centers and sizes for blocks where that form does not hold. Here
     some blocks are made irregular by one-ulp changes of a child's center or size, so both forms run in one walk;
     rows must still equal the oracle's on the same (changed) geometry, with and without a search extension."""
-    T = np.float32
     n = 50000
     x, y, z, h = plummer_input(n, T, a=0.2, target=80)
-    gbox, obox = boxes(hip, T, -1.0, 1.0)
+    gbox, obox = boxes(hip, T, -1.0, 1.0, boundary)
     p = cpu_pipeline(oracle, x, y, z, h, obox, np.uint64, 32, HILBERT)
     N = p["prefixes"].size
     centers = p["centers"].reshape(-1, 3).copy()
@@ -306,6 +307,53 @@ def test_find_neighbors_mixed_child_geometry(hip, oracle):
                                                q["centers"], q["sizes"], 96, ext)
         nb, nc = _gpu_neighbors(hip, q, gbox, 0, n, 96, ext)
         assert neighbor_rows_equal(nb, nc, ref_nb, ref_nc, 96), ext
+
+
+@pytest.mark.parametrize("T,boundary", [(np.float64, (0, 0, 0)), (np.float64, (1, 1, 1)), (np.float32, (1, 0, 1))])
+def test_find_neighbors_in_a_graph(hip, T, boundary):
+    """fp64 and periodic searches allocate nothing while their stream is captured (they walk child by child there): every
+    replay gives the eager call's rows, also after the particles have moved in place."""
+    import ctypes as C
+
+    n, ngmax = 9000, 64
+    rng = np.random.default_rng(31)
+    p = [rng.random(n).astype(T) for _ in range(3)] + [np.full(n, 0.04, T)]
+    gbox = hip.make_box(0.0, 1.0, T, boundary)
+    pipe = hip.Pipeline(curve=HILBERT, key_bits=64, real_bits=8 * np.dtype(T).itemsize, bucket_size=32, ngmax=0)
+    pipe.sync(*[dev(hip, a) for a in p], n, gbox, full_build=True)
+    v, a = pipe.view(), pipe.arrays()
+    x, y, z, h = (dev(hip, a[k]) for k in "xyzh")
+
+    def search(nb, nc, stream=None):
+        hip.find_neighbors(x, y, z, h, 0, n, gbox, v.child_offsets, v.parents, v.internal_to_leaf, v.layout, v.centers,
+                           v.sizes, v.num_nodes, ngmax, nb, nc, 1.0, stream)
+
+    def arrays():
+        nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
+        nb.fill(0)
+        return nb, nc
+
+    lib, s = hip._lib, hip.Stream()
+    handle, graph, run = C.c_void_p(s.handle), C.c_void_p(), C.c_void_p()
+    eager, out = arrays(), arrays()
+    search(*out)  # (what the first call sets up is there before the capture)
+    hip.device_sync()
+    print(f"search in a graph {np.dtype(T).name} {boundary}", flush=True)
+    assert lib.hipStreamBeginCapture(handle, 1) == 0  # thread-local
+    search(*out, stream=s)
+    assert lib.hipStreamEndCapture(handle, C.byref(graph)) == 0 and graph.value
+    assert lib.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for step in range(4):
+        x.upload((a["x"] + T(1e-3) * T(step) * (rng.random(n).astype(T) - T(0.5))).astype(T))
+        for d in (*eager, *out):
+            d.fill(0)
+        search(*eager)
+        hip.device_sync()
+        assert lib.hipGraphLaunch(run, handle) == 0
+        s.sync()
+        assert np.array_equal(out[1].download(), eager[1].download()), step
+        assert np.array_equal(out[0].download(), eager[0].download()), step
+    assert lib.hipGraphExecDestroy(run) == 0 and lib.hipGraphDestroy(graph) == 0
 
 
 @pytest.mark.parametrize("boundary", [(1, 1, 1), (1, 0, 0)])
