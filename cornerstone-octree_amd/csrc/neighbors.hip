@@ -26,12 +26,13 @@ namespace hipcstone
 // Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a sixth busy): the walk takes
 // 2.25 of 6.2 ms, the chunks' set-up 1.0, the pair tests 1.45, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
 // search of that size took 7.65 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
-// instructions a wave, now 24.9K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.95 ms.
+// instructions a wave, now 24.9K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.90 ms.
 
 // Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.53 ms, 6 waves 6.20, where 5 vector registers go
 // to memory, none of them in the inner loops (16.8M targets); the LDS holds no seventh wave. fp64, 300k uniform targets
-// open / periodic: 4 waves 232 / 283 us, 5 waves 211 / 254, 6 waves 222 / 272; 2M open: 977, 949, 1040 (30k, which do not
-// fill the device: 80, 83, 88). At 5 fp64 spills 4 or 5 vector registers, and in periodic boxes 49 to 58 scalar ones.
+// open / periodic: 4 and 5 waves (one allocation in open boxes) 201 / 282 and 200 / 254 us, 6 waves 217 / 274; 2M open:
+// 904, 906, 999; 30k, which do not fill the device: 79, 79, 87. At 5 open fp64 walks spill nothing, periodic ones 5 vector
+// and 49 to 58 scalar registers.
 template<class T>
 constexpr int kNbMinWavesPerEu = std::is_same_v<T, float> ? 6 : 5;
 
