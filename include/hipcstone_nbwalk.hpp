@@ -300,10 +300,11 @@ struct Shared
 // node boxes are decoded from) the children's octants follow one pattern up to the order of the axes: one axis changes
 // with every second child (kFast), one with every fourth (kMiddle), one half way (kSlow). With the first child's
 // center as each axis' first value, child k therefore lies at the second one where bit k of the axis' pattern is set.
+// Along the Morton curve (a caller's own geometry) x is the slow axis, the others have patterns of their own.
 // Record g describes the children [8 g + 1, 8 g + 9), the child block of some internal node.
 //   v0, v1, s: the center of child 0, the other center and the size, for x, for the faster of y and z, and for the other
 //   flags:     bit k set if child k is internal; kXFast, kXMiddle: x's pattern (neither: it is the slow axis); kZFaster:
-//              z is faster than y; kGroupValid if every child matched bit for bit (else the walk takes the children's
+//              z is faster than y; kMorton: the Morton curve's patterns; kGroupValid if every child matched bit for bit (else the walk takes the children's
 //              own centers and sizes); kGroupOutside if an internal child's block lies outside the tree or a leaf
 //              child has no leaf index, kGroupBackward if a block does not come after its parent
 //   link:      a leaf child's leaf index (internalToLeaf), an internal child's own child block (childOffsets)
@@ -318,8 +319,8 @@ typedef uint32_t Words16 __attribute__((ext_vector_type(16)));
 typedef uint32_t Words8 __attribute__((ext_vector_type(8)));
 typedef int32_t Links8 __attribute__((ext_vector_type(8)));
 constexpr uint32_t kGroupValid = 0x80000000u, kGroupOutside = 0x40000000u, kGroupBackward = 0x20000000u;
-constexpr uint32_t kXFast = 0x100u, kXMiddle = 0x200u, kZFaster = 0x400u;
-constexpr uint32_t kFast = 0x66u, kMiddle = 0x3Cu, kSlow = 0xF0u;
+constexpr uint32_t kXFast = 0x100u, kXMiddle = 0x200u, kZFaster = 0x400u, kMorton = 0x800u;
+constexpr uint32_t kFast = 0x66u, kMiddle = 0x3Cu, kSlow = 0xF0u, kMortonFast = 0xAAu, kMortonMiddle = 0xCCu;
 
 // the ChildGroup records of a tree with numNodes nodes: (numNodes - 1) / 8 of them (none for a root-only tree)
 inline size_t childGroupCount(int32_t numNodes) { return numNodes > 8 ? size_t((numNodes - 1) / 8) : 0; }
@@ -361,12 +362,14 @@ __global__ void childGroupsKernel(const T* __restrict__ centers, const T* __rest
         size[d] = s;
     }
     // the axes' order; an axis whose two centers round to one value goes with any pattern
-    constexpr uint32_t kOrders[6][4] = {{kFast, kMiddle, kSlow, kXFast},   {kFast, kSlow, kMiddle, kXFast | kZFaster},
+    constexpr uint32_t kOrders[8][4] = {{kFast, kMiddle, kSlow, kXFast},   {kFast, kSlow, kMiddle, kXFast | kZFaster},
                                         {kMiddle, kFast, kSlow, kXMiddle}, {kMiddle, kSlow, kFast, kXMiddle | kZFaster},
-                                        {kSlow, kFast, kMiddle, 0u},       {kSlow, kMiddle, kFast, kZFaster}};
+                                        {kSlow, kFast, kMiddle, 0u},       {kSlow, kMiddle, kFast, kZFaster},
+                                        {kSlow, kMortonFast, kMortonMiddle, kMorton},
+                                        {kSlow, kMortonMiddle, kMortonFast, kMorton | kZFaster}};
     bool found     = false;
     uint32_t flags = 0;
-    for (int o = 0; o < 6; ++o)
+    for (int o = 0; o < 8; ++o)
     {
         bool ok = true;
         for (int d = 0; d < 3; ++d)
@@ -979,6 +982,7 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
             };
             if (flags & kXFast) compare(kFast, kMiddle, kSlow);
             else if (flags & kXMiddle) compare(kMiddle, kFast, kSlow);
+            else if (flags & kMorton) compare(kSlow, kMortonFast, kMortonMiddle);
             else compare(kSlow, kFast, kMiddle);
         }
         if (!(flags & kGroupValid))

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from helpers import cpu_pipeline, neighbor_rows_equal
-from oracle_py import HILBERT
+from oracle_py import HILBERT, MORTON
 from oracle_py import make_box as orc_box
 
 pytestmark = pytest.mark.gpu
@@ -267,3 +267,68 @@ def test_small_slot_major_search_is_not_slow(hip, T):
     print("slot-major", flush=True)
     _, _, ms2 = _timed_search(hip, T, p, 0.0, 1.0, 100, boundary=(1, 1, 1), repeats=20, slot_major=True)
     assert ms2 < 1.5 * ms, (ms, ms2)
+
+
+def _morton_geometry(prefixes, T):
+    """Centers and half sizes of the nodes' regions along the Morton curve, in the unit box."""
+    p = [int(v) for v in prefixes]
+    level = np.array([(v.bit_length() - 1) // 3 for v in p])
+    width = 2.0 ** -level.astype(np.float64)
+    c = np.zeros((len(p), 3))
+    for d in range(3):
+        at = np.zeros(len(p), np.int64)
+        for b in range(int(level.max())):
+            bit = np.array([(v >> (3 * b + 2 - d)) & 1 for v in p]) * (b < level)
+            at |= bit << b
+        c[:, d] = (at + 0.5) * width
+    return c.astype(T), np.repeat((0.5 * width)[:, None], 3, 1).astype(T)
+
+
+@pytest.mark.parametrize("T", TS)
+@pytest.mark.parametrize("boundary", [(0, 0, 0), (1, 0, 1)])
+def test_morton_geometry(hip, oracle, T, boundary):
+    """A caller's own node geometry, that of the Morton curve, along which child blocks have patterns of their own."""
+    rng = np.random.default_rng(37)
+    n = 12000
+    x, y, z = (rng.random(n).astype(T) for _ in range(3))
+    x[:4000], y[:4000], z[:4000] = (T(0.4) + T(0.05) * rng.random((3, 4000)).astype(T))
+    h = np.full(n, 0.03, T)
+    h[:4000] = T(0.008)
+    obox = orc_box(0.0, 1.0, T, boundary)
+    p = cpu_pipeline(oracle, x, y, z, h, obox, np.uint64, 16, MORTON)
+    centers, sizes = _morton_geometry(p["prefixes"], T)
+    p = dict(p, centers=centers.reshape(-1), sizes=sizes.reshape(-1))
+    counts = _check(hip, oracle, p, 0.0, 1.0, 96, boundary=boundary)
+    assert counts.mean() > 20
+    _check(hip, oracle, p, 0.0, 1.0, 96, boundary=boundary, ext=1.3)
+
+
+def test_morton_geometry_is_not_slow(hip):
+    """A search over a Morton tree with its own geometry takes at most 1.45 times that over a Hilbert tree."""
+    T, n, ngmax = np.float32, 300_000, 150
+    rng = np.random.default_rng(41)
+    part = [rng.random(n).astype(T) for _ in range(3)] + [np.full(n, 0.5 * (100 / (4.19 * n)) ** (1 / 3), T)]
+    box = hip.make_box(0.0, 1.0, T)
+    nb, nc = hip.DeviceArray(n * ngmax, np.uint32), hip.DeviceArray(n, np.uint32)
+    ms = {}
+    for curve in (hip.HILBERT, hip.MORTON):
+        pipe = hip.Pipeline(curve=curve, key_bits=64, real_bits=32, bucket_size=64, ngmax=0)
+        pipe.sync(*[hip.DeviceArray.from_numpy(a) for a in part], n, box, full_build=True)
+        v, a = pipe.view(), pipe.arrays()
+        centers, sizes = a["centers"], a["sizes"]
+        if curve == hip.MORTON:
+            centers, sizes = _morton_geometry(a["prefixes"], T)
+        c, s = (hip.DeviceArray.from_numpy(np.ascontiguousarray(g).reshape(-1)) for g in (centers, sizes))
+        times = []
+        print(f"search over curve {curve}", flush=True)
+        for _ in range(10):
+            t = [hip.Event(), hip.Event()]
+            t[0].record()
+            hip.find_neighbors(v.x, v.y, v.z, v.h, 0, n, box, v.child_offsets, v.parents, v.internal_to_leaf, v.layout, c,
+                               s, v.num_nodes, ngmax, nb, nc)
+            t[1].record()
+            hip.device_sync()
+            times.append(t[0].elapsed_ms(t[1]))
+        ms[curve] = min(times)
+        assert nc.download().mean() > 80
+    assert ms[hip.MORTON] < 1.45 * ms[hip.HILBERT], ms
