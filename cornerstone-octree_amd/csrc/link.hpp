@@ -75,9 +75,9 @@ __host__ __device__ inline void createNodes(int32_t t, const Keys& leaves, int32
 }
 
 // Sorted entry i < numNodes: prefixes[i] = unsorted prefix of node order[i]; leafToInternal[order[i]] = i;
-// internalToLeaf[i] = order[i] - numInternal for leaves (octree.hpp:176-185; linkNode does the inner nodes); childOffsets[i] = 0 for linkNode; levelRange
-// (getLevelRangeCpu, octree.hpp:151-160): the first node index of every level from the places where the level changes;
-// the levels after the last one keep numNodes
+// internalToLeaf[i] = order[i] - numInternal for leaves (octree.hpp:176-185; linkNode does the inner nodes);
+// childOffsets[i] = 0 for linkNode; levelRange (getLevelRangeCpu, octree.hpp:151-160): the first node index of every level
+// from the places where the level changes; the levels after the last one keep numNodes
 template<class K, class Arrays>
 __host__ __device__ inline void placeNode(int32_t i, const Arrays& a)
 {

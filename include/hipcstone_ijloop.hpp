@@ -300,8 +300,8 @@ __global__ void zeroCountersKernel(uint32_t* counters)
 
 /*
  * The fused always-traverse loop. Bodies [first, last) form groups of groupSize (up to 64); the groups are split into 8
- * contiguous ranges, one per XCD (workgroups are dealt to the XCDs round-robin, so workgroup b runs on XCD b % 8 and neighbouring
- * groups share tree nodes and particles in that XCD's L2). Each wave takes the next group of its XCD's range from
+ * contiguous ranges, one per XCD (workgroups are dealt to the XCDs round-robin, so workgroup b runs on XCD b % 8 and
+ * neighbouring groups share tree nodes and particles in that XCD's L2). Each wave takes the next group of its XCD's range from
  * counters[xcd] and, when that range is exhausted, helps with the next XCD's. Per group: as the walk finds neighbors,
  * each lane takes its own body's (the first ngmax, ascending j) and folds them in order; the postamble result is stored
  * after the walk. Bodies outside the subgroups take no part.

@@ -41,7 +41,8 @@
  * 16-candidate groups it occurs in again, in the reference's own operations. fp64 lengths are first multiplied by one
  * power of two for the whole wave, so the products do not depend on the unit of length; only waves whose largest length
  * is beyond 2^-48 to 2^60 (fp32, where the reference's own squares near the ends of the range) or 2^-100 to 2^101 (fp64)
- * do without the products and test each target against a chunk's 64 candidates at once. So every decision is the reference's, bit for bit, for fp32 and fp64 alike.
+ * do without the products and test each target against a chunk's 64 candidates at once. So every decision is the
+ * reference's, bit for bit, for fp32 and fp64 alike.
  * A wave with a target whose 2h box leaves a periodic domain folds its candidates to their images nearest to c. While
  * S < L / 2 these are the reference's images for every pair that can be a hit, and the folded differences are off by at
  * most 2 u L per dimension, the reference's included, so E grows by 8 u r L; with a larger S the wave does without the
@@ -304,9 +305,10 @@ struct Shared
 // Record g describes the children [8 g + 1, 8 g + 9), the child block of some internal node.
 //   v0, v1, s: the center of child 0, the other center and the size, for x, for the faster of y and z, and for the other
 //   flags:     bit k set if child k is internal; kXFast, kXMiddle: x's pattern (neither: it is the slow axis); kZFaster:
-//              z is faster than y; kMorton: the Morton curve's patterns; kGroupValid if every child matched bit for bit (else the walk takes the children's
-//              own centers and sizes); kGroupOutside if an internal child's block lies outside the tree or a leaf
-//              child has no leaf index, kGroupBackward if a block does not come after its parent
+//              z is faster than y; kMorton: the Morton curve's patterns; kGroupValid if every child matched bit for bit
+//              (else the walk takes the children's own centers and sizes); kGroupOutside if an internal child's block
+//              lies outside the tree or a leaf child has no leaf index, kGroupBackward if a block does not come after
+//              its parent
 //   link:      a leaf child's leaf index (internalToLeaf), an internal child's own child block (childOffsets)
 template<class T>
 struct alignas(128) ChildGroup
@@ -982,7 +984,8 @@ walk(const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z, 
             };
             if (flags & kXFast) compare(kFast, kMiddle, kSlow);
             else if (flags & kXMiddle) compare(kMiddle, kFast, kSlow);
-            else if (flags & kMorton) compare(kSlow, kMortonFast, kMortonMiddle);
+            // (the hint keeps this out of the way of the reference's own geometry, 0.4 % of a search of 16.8M)
+            else if (__builtin_expect((flags & kMorton) != 0, 0)) compare(kSlow, kMortonFast, kMortonMiddle);
             else compare(kSlow, kFast, kMiddle);
         }
         if (!(flags & kGroupValid))

@@ -115,7 +115,7 @@ def test_deep_tree_with_everything_in_reach(hip, oracle, T):
                                      (np.float64, 1e-40), (np.float64, 1e-12), (np.float64, 1e12), (np.float64, 1e40),
                                      # both sides of where the products' power of two ends
                                      (np.float32, 2e-14), (np.float32, 1e-13), (np.float32, 2e18), (np.float32, 8e18),
-                                     (np.float64, 3e-30), (np.float64, 3e-29), (np.float64, 3e30), (np.float64, 3e31)])
+                                     (np.float32, 1e-14), (np.float32, 3e19), (np.float64, 3e-30), (np.float64, 3e-29), (np.float64, 3e30), (np.float64, 3e31)])
 def test_magnitudes(hip, oracle, T, scale):
     """Coordinates and radii whose squares leave fp32's range, or come near its ends, and a box far from the origin."""
     rng = np.random.default_rng(9)

@@ -69,7 +69,8 @@ constexpr size_t MB = size_t(1) << 20;
 """
 
 
-@pytest.mark.parametrize("how", ["deviceMalloc(&p, 8 * MB)", "deviceMallocAsync(&p, 8 * MB, nullptr)", "poolTake(&p, &size)"])
+@pytest.mark.parametrize("how", ["deviceMalloc(&p, 8 * MB)", "deviceMallocAsync(&p, 8 * MB, nullptr)",
+                                 "poolTake(&p, &size)"])
 def test_allocations_get_the_kept_blocks_back(tmp_path, how):
     """With 10 MB on the device and 6 of them kept, an allocation of 8 MB succeeds, whichever way it is made."""
     run = _run(tmp_path, "trim", DEVICE + r"""
