@@ -26,7 +26,7 @@ namespace hipcstone
 // Vector and scalar issue bound it (no unit of memory is near its limit, the matrix cores are a sixth busy): the walk takes
 // 2.25 of 6.2 ms, the chunks' set-up 1.0, the pair tests 1.45, the rows 1.5 (16.8M targets, 100 neighbors, fp32). The
 // search of that size took 7.65 ms with the pair tests in vector code, one candidate of one leaf at a time (38.7K
-// instructions a wave, now 24.9K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.90 ms.
+// instructions a wave, now 25.0K); in fp64 at 2M, where nothing was compact either, 1.57 -> 0.90 ms.
 
 // Minimum waves per SIMD the registers are allocated for. fp32: 5 waves 6.53 ms, 6 waves 6.20, where 5 vector registers go
 // to memory, none of them in the inner loops (16.8M targets); the LDS holds no seventh wave. fp64, 300k uniform targets

@@ -308,7 +308,7 @@ __global__ void zeroCountersKernel(uint32_t* counters)
  * The walk bounds it. Lists kept in registers and LDS instead of a per-wave scratch save the rows' way to memory and
  * back and, per neighborhood, the allocation of that scratch (64 * ngmax slots for every resident wave, 262 MB at ngmax
  * 200). 1M uniform bodies, 100 neighbors, ngmax 200, fp32: the kernel 1.12 -> 0.87 ms, with the neighborhood's
- * allocations 12.4 -> 0.94. 16.8M bodies, ngmax 150: the kernel 14.0 -> 10.5 ms.
+ * allocations 12.4 -> 0.94. 16.8M bodies, ngmax 150: the kernel 14.0 -> 10.2 ms.
  */
 template<bool AnyPbc, class T, class InTuple, class OutTuple, class Interaction, class Postamble>
 __global__ __launch_bounds__(kFusedWaves * 64) void fusedIjLoopKernel(

@@ -49,7 +49,7 @@
  * products, and a chunk with a particle outside the domain is tested again (the reference folds only for targets near
  * its faces).
  *
- * What bounds it is instruction issue: a wave of 64 targets with 100 neighbors takes 12.3K vector, 7.1K scalar and
+ * What bounds it is instruction issue: a wave of 64 targets with 100 neighbors takes 12.2K vector, 7.1K scalar and
  * 2.6K branch instructions, and 323 matrix products, which replace some 90K multiply-adds and compares by lane. Pair
  * tests one candidate at a time took 16.2K vector and 12.8K scalar instructions (16.8M targets: 7.65 ms, now 6.2).
  *
